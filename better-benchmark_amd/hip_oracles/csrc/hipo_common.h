@@ -54,6 +54,11 @@ typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+// The same 16 bytes at any element's address (2- or 4-byte aligned): one
+// global_load / store_dwordx4 still, the target runs with unaligned access
+// enabled.  Rows and planes that are not a whole number of vectors use them.
+typedef u32x4_t u32x4_a2_t __attribute__((aligned(2)));
+typedef f32x4_t f32x4_a4_t __attribute__((aligned(4)));
 
 inline bool aligned16(const void* p) {
   return reinterpret_cast<uintptr_t>(p) % 16 == 0;

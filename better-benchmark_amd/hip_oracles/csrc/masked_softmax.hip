@@ -29,6 +29,15 @@
 //     through LDS, row reductions within the wave;
 //   otherwise (or a per-batch mask the grouping cannot share): the
 //     row_layout.h plan, W waves per row, 2 KiB per wave.
+// Rows that are not whole 16-byte groups, or not 16-byte aligned, take the
+// first and the last of these with element-aligned groups (row_layout.h,
+// RaggedGroup) instead of a one-value-per-lane kernel that read each row
+// three times: graph replays, [1536, 197, 197] 209 -> 56 us (4.2 TB/s),
+// [96, 577, 577] 75 -> 34, [512, 50, 77] causal 11.2 -> 4.7, [8, 1500, 1501]
+// with a bias 55 -> 20.  What bounds them is the arithmetic of the lanes a
+// row leaves idle (25 groups on 32 lanes at K = 197) more than the
+// misalignment: K = 193 takes 53 us and K = 192, aligned, 50.5, while 256,
+// no lane idle, moves the same bytes in 43.
 // HBM-bound: algorithmic bytes per element = 2 (read) + 2 (write), plus the
 // mask once.
 #include "row_layout.h"
@@ -44,35 +53,52 @@ __device__ __forceinline__ float exp_shifted(float s, float m) {
   return exp_f32_nonpos(__builtin_elementwise_maximum(s - m, -104.0f));
 }
 
-template <int U, int WT>
+// RAGGED: rows of any length >= 8 and any alignment (row_layout.h).
+template <int U, int WT, bool RAGGED>
 __global__ __launch_bounds__(kRowMaxThreads) void masked_softmax_rows(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ mask,
     uint16_t* __restrict__ out, int64_t rows, int64_t Q, int64_t K,
-    int64_t mask_stride, int64_t mask_batch_stride, int64_t heads, float scale,
-    int w_arg, int rpb_arg) {
+    int64_t mask_stride, int64_t mask_batch_stride, int64_t heads, DivMagic q_div,
+    DivMagic heads_div, float scale, int w_arg, int rpb_arg) {
   const int waves_per_row = WT > 0 ? WT : w_arg;
   const int rows_per_block = WT > 0 ? kRowMaxWaves / WT : rpb_arg;
   __shared__ float pmax[kRowMaxWaves], psum[kRowMaxWaves];
   const RowPlace p = row_place(waves_per_row, rows_per_block, rows);
-  const int64_t b = p.row / Q;
+  int64_t b, hb;  // batch entry and mask batch group
+  if (rows < (int64_t{1} << 31)) {
+    b = div_by(static_cast<uint32_t>(p.row), q_div);
+    hb = div_by(static_cast<uint32_t>(b), heads_div);
+  } else {
+    b = p.row / Q;
+    hb = b / heads;
+  }
   const int64_t q = p.row - b * Q;
   const uint16_t* xr = x + p.row * K;
-  const uint16_t* mr = mask + (b / heads) * mask_batch_stride + q * mask_stride;
+  const uint16_t* mr = mask + hb * mask_batch_stride + q * mask_stride;
   uint16_t* orow = out + p.row * K;
 
   u32x4_t xv[U], mv[U];
+  RaggedGroup rg[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t col = row_group_col(u, waves_per_row, p);
-    xv[u] = row_load_stream(xr, col, K);
-    mv[u] = row_load_cached(mr, col, K);
+    if constexpr (RAGGED) {
+      rg[u] = ragged_group(col, K);
+      xv[u] = ragged_load_stream(xr + rg[u].col);
+      mv[u] = ragged_load_cached(mr + rg[u].col);
+    } else {
+      xv[u] = row_load_stream(xr, col, K);
+      mv[u] = row_load_cached(mr, col, K);
+    }
   }
 
   float s[U][8];
   float m = -__builtin_inff();
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const bool in = row_group_col(u, waves_per_row, p) < K;
+    // A ragged group past the row holds the row's last values: no change to
+    // the maximum.
+    const bool in = RAGGED || row_group_col(u, waves_per_row, p) < K;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       s[u][2 * d] = in ? __builtin_fmaf(bf16lo(xv[u][d]), scale, bf16lo(mv[u][d]))
@@ -98,7 +124,11 @@ __global__ __launch_bounds__(kRowMaxThreads) void masked_softmax_rows(
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       s[u][e] = exp_shifted(s[u][e], m);
-      sum += s[u][e];
+      if constexpr (RAGGED) {
+        sum = __builtin_fmaf(s[u][e], e >= rg[u].skip ? 1.0f : 0.0f, sum);
+      } else {
+        sum += s[u][e];
+      }
     }
   }
   sum = wave_sum(sum);
@@ -118,7 +148,11 @@ __global__ __launch_bounds__(kRowMaxThreads) void masked_softmax_rows(
 #pragma unroll
     for (int d = 0; d < 4; ++d)
       o[d] = pack_bf16x2(div_rn(s[u][2 * d], sum, inv), div_rn(s[u][2 * d + 1], sum, inv));
-    if (p.valid && col < K) row_store_stream(orow, col, o);
+    if constexpr (RAGGED) {
+      if (p.valid && rg[u].skip < kRowGroup) ragged_store(orow + rg[u].col, o);
+    } else {
+      if (p.valid && col < K) row_store_stream(orow, col, o);
+    }
   }
 }
 
@@ -141,7 +175,7 @@ __global__ __launch_bounds__(kRowMaxThreads) void masked_softmax_rows(
 constexpr int kShortV = 2;
 constexpr int kShortThreads = 256;
 
-template <int L>
+template <int L, bool RAGGED>
 __global__ __launch_bounds__(kShortThreads) void masked_softmax_short_rows(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ mask,
     uint16_t* __restrict__ out, uint32_t rows, uint32_t Q, DivMagic q_div, int K,
@@ -151,7 +185,13 @@ __global__ __launch_bounds__(kShortThreads) void masked_softmax_short_rows(
   const uint32_t wave = blockIdx.x * (kShortThreads / kWave) + (threadIdx.x >> 6);
   const int col = (lane % L) * kRowGroup;
   const bool col_in = col < K;
-  const int c = col_in ? col : K - kRowGroup;
+  // Lanes past the row, and a ragged row's last group, hold the row's last
+  // 8 values; a ragged group's first `skip` values belong to its neighbour.
+  const int c = RAGGED ? (col < K - kRowGroup ? col : K - kRowGroup)
+                       : (col_in ? col : K - kRowGroup);
+  float own[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) own[e] = e >= col - c ? 1.0f : 0.0f;
 
   uint32_t row[kShortV];
   u32x4_t xv[kShortV], mv[kShortV];
@@ -163,9 +203,14 @@ __global__ __launch_bounds__(kShortThreads) void masked_softmax_short_rows(
     const uint32_t q = r - b * Q;
     const uint16_t* mr = mask + static_cast<int64_t>(div_by(b, heads_div)) * mask_batch_stride +
                          static_cast<int64_t>(q) * mask_stride;
-    xv[v] = __builtin_nontemporal_load(
-        reinterpret_cast<const u32x4_t*>(x + static_cast<int64_t>(r) * K + c));
-    mv[v] = *reinterpret_cast<const u32x4_t*>(mr + c);
+    const uint16_t* xr = x + static_cast<int64_t>(r) * K;
+    if constexpr (RAGGED) {
+      xv[v] = ragged_load_stream(xr + c);
+      mv[v] = ragged_load_cached(mr + c);
+    } else {
+      xv[v] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(xr + c));
+      mv[v] = *reinterpret_cast<const u32x4_t*>(mr + c);
+    }
   }
 
 #pragma unroll
@@ -174,10 +219,11 @@ __global__ __launch_bounds__(kShortThreads) void masked_softmax_short_rows(
     float m = -__builtin_inff();
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      s[2 * d] = col_in ? __builtin_fmaf(bf16lo(xv[v][d]), scale, bf16lo(mv[v][d]))
+      const bool in = RAGGED || col_in;
+      s[2 * d] = in ? __builtin_fmaf(bf16lo(xv[v][d]), scale, bf16lo(mv[v][d]))
+                    : -__builtin_inff();
+      s[2 * d + 1] = in ? __builtin_fmaf(bf16hi(xv[v][d]), scale, bf16hi(mv[v][d]))
                         : -__builtin_inff();
-      s[2 * d + 1] = col_in ? __builtin_fmaf(bf16hi(xv[v][d]), scale, bf16hi(mv[v][d]))
-                            : -__builtin_inff();
       m = fmaxf(m, fmaxf(s[2 * d], s[2 * d + 1]));
     }
     m = seg_max<L>(m);
@@ -185,7 +231,12 @@ __global__ __launch_bounds__(kShortThreads) void masked_softmax_short_rows(
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       s[e] = exp_shifted(s[e], m);
-      sum += s[e];
+      // own[e] is 0 or 1; s[e] is finite or the row is NaN anyway
+      if constexpr (RAGGED) {
+        sum = __builtin_fmaf(s[e], own[e], sum);
+      } else {
+        sum += s[e];
+      }
     }
     const float tot = seg_sum<L>(sum);
     const float inv = 1.0f / tot;
@@ -193,20 +244,25 @@ __global__ __launch_bounds__(kShortThreads) void masked_softmax_short_rows(
 #pragma unroll
     for (int d = 0; d < 4; ++d)
       o[d] = pack_bf16x2(div_rn(s[2 * d], tot, inv), div_rn(s[2 * d + 1], tot, inv));
-    if (row[v] < rows && col_in)
-      __builtin_nontemporal_store(
-          o, reinterpret_cast<u32x4_t*>(out + static_cast<int64_t>(row[v]) * K + col));
+    if (row[v] < rows && col_in) {
+      uint16_t* orow = out + static_cast<int64_t>(row[v]) * K;
+      if constexpr (RAGGED) {
+        ragged_store(orow + c, o);
+      } else {
+        __builtin_nontemporal_store(o, reinterpret_cast<u32x4_t*>(orow + col));
+      }
+    }
   }
 }
 
-template <int L>
+template <int L, bool RAGGED>
 void launch_short(dim3 grid, hipStream_t stream, const uint16_t* x, const uint16_t* mask,
                   uint16_t* out, int64_t rows, int64_t Q, int64_t K, int64_t ms, int64_t mbs,
                   int64_t heads, float scale) {
   const auto r = static_cast<uint32_t>(rows);
   const auto q = static_cast<uint32_t>(Q);
   const DivMagic qd = div_magic(q), hd = div_magic(static_cast<uint32_t>(heads));
-  masked_softmax_short_rows<L><<<grid, dim3(kShortThreads), 0, stream>>>(
+  masked_softmax_short_rows<L, RAGGED><<<grid, dim3(kShortThreads), 0, stream>>>(
       x, mask, out, r, q, qd, static_cast<int>(K), ms, mbs, hd, scale);
 }
 
@@ -414,12 +470,17 @@ __global__ __launch_bounds__(256) void masked_softmax_rows_scalar(
   }
 }
 
-template <int U, int WT>
+template <int U, int WT, bool RAGGED>
 void launch_vec(dim3 grid, const RowPlan& plan, hipStream_t stream, const uint16_t* x,
                 const uint16_t* mask, uint16_t* out, int64_t rows, int64_t Q, int64_t K,
                 int64_t ms, int64_t mbs, int64_t heads, float scale) {
-  masked_softmax_rows<U, WT><<<grid, dim3(plan.threads()), 0, stream>>>(
-      x, mask, out, rows, Q, K, ms, mbs, heads, scale, plan.waves_per_row, plan.rows_per_block);
+  // Used for rows < 2^31 only, where q and heads are below 2^31 too.
+  const bool small = rows < (int64_t{1} << 31);
+  const DivMagic qd = small ? div_magic(static_cast<uint32_t>(Q)) : DivMagic{};
+  const DivMagic hd = small ? div_magic(static_cast<uint32_t>(heads)) : DivMagic{};
+  masked_softmax_rows<U, WT, RAGGED><<<grid, dim3(plan.threads()), 0, stream>>>(
+      x, mask, out, rows, Q, K, ms, mbs, heads, qd, hd, scale, plan.waves_per_row,
+      plan.rows_per_block);
 }
 
 }  // namespace
@@ -440,16 +501,23 @@ int softmax_impl(const uint16_t* x, const uint16_t* mask, uint16_t* out, int64_t
   HIPO_REQUIRE(mask_batch_stride >= 0, "%s: negative mask_batch_stride", what);
   const int64_t rows = batch * q;
   RowPlan plan;
-  const bool vec = (k % 8 == 0) && (mask_row_stride % 8 == 0) &&
-                   (mask_batch_stride % 8 == 0) && row_plan(k, plan) && aligned16(x) &&
-                   aligned16(mask) && aligned16(out);
+  // Rows of 8 to 32768 values are held in registers; whole 16-byte groups at
+  // 16-byte alignment take the aligned kernels, any other length or
+  // alignment the same kernels with element-aligned groups.
+  const bool held = k >= kRowGroup && row_plan(k, plan);
+  const bool vec = held && k % 8 == 0 && mask_row_stride % 8 == 0 &&
+                   mask_batch_stride % 8 == 0 && aligned16(x) && aligned16(mask) &&
+                   aligned16(out);
   const int lanes = short_row_lanes(k);
-  if (vec && lanes > 0 && rows < (int64_t{1} << 31)) {
+  if (held && lanes > 0 && rows < (int64_t{1} << 31)) {
     const int64_t rows_per_block = int64_t{kShortV} * (kWave / lanes) * (kShortThreads / kWave);
     const dim3 grid(static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block));
-#define HIPO_SHORT(L_)                                                                  \
-  launch_short<L_>(grid, stream, x, mask, out, rows, q, k, mask_row_stride, mask_batch_stride, \
-                   heads, scale)
+#define HIPO_SHORT(L_)                                                                       \
+  do {                                                                                       \
+    auto launch = vec ? launch_short<L_, false> : launch_short<L_, true>;                    \
+    launch(grid, stream, x, mask, out, rows, q, k, mask_row_stride, mask_batch_stride, heads, \
+           scale);                                                                           \
+  } while (0)
     switch (lanes) {
       case 1: HIPO_SHORT(1); break;
       case 2: HIPO_SHORT(2); break;
@@ -471,13 +539,16 @@ int softmax_impl(const uint16_t* x, const uint16_t* mask, uint16_t* out, int64_t
       launch_shared_mask<2048>(sp, stream, x, mask, out, batch, q, mask_row_stride,
                                mask_batch_stride, scale);
     }
-  } else if (vec) {
+  } else if (held) {
     const int64_t blocks = (rows + plan.rows_per_block - 1) / plan.rows_per_block;
     HIPO_REQUIRE(blocks <= 0x7fffffff, "%s: too many rows", what);
     const dim3 grid(static_cast<unsigned>(blocks));
-#define HIPO_SOFTMAX(U_, W_)                                                            \
-  launch_vec<U_, W_>(grid, plan, stream, x, mask, out, rows, q, k, mask_row_stride,   \
-                     mask_batch_stride, heads, scale)
+#define HIPO_SOFTMAX(U_, W_)                                                                  \
+  do {                                                                                        \
+    auto launch = vec ? launch_vec<U_, W_, false> : launch_vec<U_, W_, true>;                 \
+    launch(grid, plan, stream, x, mask, out, rows, q, k, mask_row_stride, mask_batch_stride,  \
+           heads, scale);                                                                     \
+  } while (0)
     HIPO_ROW_DISPATCH(plan, HIPO_SOFTMAX);
 #undef HIPO_SOFTMAX
   } else {

@@ -100,6 +100,39 @@ __device__ __forceinline__ void row_store_stream(uint16_t* row, int64_t col,
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(row + col));
 }
 
+// Rows of any length >= 8 and any alignment ("ragged"): group `col` of a row
+// keeps its place except the one that would cross the row's end, which moves
+// back to end there (col = cols - 8); its first `skip` values are the
+// previous group's, which owns them.  skip >= 8: past the row, owns nothing.
+// Loads and stores stay whole 16-byte ones, at element alignment; the values
+// two groups share are computed from the same bits by both and stored twice
+// with the same bytes, and only the owner adds them to a sum.  Stores are
+// ordinary ones: neighbouring rows share cache lines, which meet in the L2
+// (non-temporal stores measured the same within 2 % either way).
+struct RaggedGroup {
+  int64_t col;
+  int skip;
+};
+
+__device__ __forceinline__ RaggedGroup ragged_group(int64_t col, int64_t cols) {
+  const int64_t last = cols - kRowGroup;
+  const int64_t c = col < last ? col : last;
+  const int64_t skip = col - c;
+  return RaggedGroup{c, static_cast<int>(skip < kRowGroup ? skip : kRowGroup)};
+}
+
+__device__ __forceinline__ u32x4_t ragged_load_stream(const uint16_t* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2_t*>(p));
+}
+
+__device__ __forceinline__ u32x4_t ragged_load_cached(const uint16_t* p) {
+  return *reinterpret_cast<const u32x4_a2_t*>(p);
+}
+
+__device__ __forceinline__ void ragged_store(uint16_t* p, u32x4_t v) {
+  *reinterpret_cast<u32x4_a2_t*>(p) = v;
+}
+
 // Short rows (cols <= 512): a row owns L = 2^j consecutive lanes (L groups
 // of 8 bf16), so one 16-byte access instruction of a wave covers 64 / L
 // rows.  seg_sum / seg_max reduce within each aligned segment of L lanes

@@ -1,0 +1,104 @@
+"""Rows, planes and channel counts that are not whole 16-byte vectors, and
+operands that are not 16-byte aligned, against the C oracle.
+
+Every call goes through the C entry points with operands inside larger
+buffers, so that a store outside the output changes a guard value; offsets of
+one element make every pointer misaligned."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+GUARD = 64  # elements around every output
+
+
+class Guarded:
+    """A tensor of `shape` at element offset GUARD + shift of a buffer whose
+    other elements hold a guard value."""
+
+    def __init__(self, shape, dtype, dev, shift=0):
+        n = 1
+        for d in shape:
+            n *= d
+        self.buf = torch.full((n + 2 * GUARD + shift,), 3.0, dtype=dtype, device=dev)
+        self.lo, self.hi = GUARD + shift, GUARD + shift + n
+        self.t = self.buf[self.lo:self.hi].view(shape)
+
+    def check(self, what):
+        assert bool((self.buf[:self.lo] == 3).all()), f"{what}: written before the output"
+        assert bool((self.buf[self.hi:] == 3).all()), f"{what}: written past the output"
+
+
+def place(t, dev, shift):
+    """t on the device, `shift` elements off its allocation's alignment."""
+    g = Guarded(t.shape, t.dtype, dev, shift)
+    g.t.copy_(t)
+    return g.t
+
+
+def lib():
+    import hip_oracles
+    return hip_oracles.load_library()
+
+
+def ok(rc):
+    assert rc == 0, lib().hipo_last_error()
+
+
+def close(got, want, rtol, atol, what):
+    g, w = got.float().cpu(), want.float()
+    assert torch.allclose(g, w, rtol=rtol, atol=atol, equal_nan=True), (
+        f"{what}: max |diff| {(g - w).abs().max().item():.3e}")
+
+
+# One 16-byte group, one value more and one less; the ends of the short-row
+# kernel (512) and of its lane counts; ViT and CLIP rows; several waves per
+# row; the longest row held in registers is 32768 (past it, the general one).
+SOFTMAX_K = [7, 8, 9, 15, 17, 50, 77, 127, 129, 197, 257, 511, 513, 577, 1023, 1025, 1500, 2047,
+             4099, 8195]
+
+
+@pytest.mark.parametrize("k", SOFTMAX_K)
+def test_softmax_any_row_length(k, rocm_device):
+    """bf16 results: relative 2^-8 is one bf16 ulp, twice that where kernel
+    and oracle round to different sides of a boundary."""
+    import oracle as ref
+    torch.manual_seed(k)
+    b, heads, q = 4, 2, 5
+    x = torch.randn(b, q, k).to(torch.bfloat16)
+    mask = torch.zeros(q, k, dtype=torch.bfloat16)
+    mask[torch.arange(k)[None, :] > torch.arange(q)[:, None] + k - q] = float("-inf")
+    mask[2, k // 2:] = float("-inf")
+    bias = torch.randn(b // heads, q, k).to(torch.bfloat16)
+    for shift in (0, 1):
+        xd, md, bd = (place(t, rocm_device, shift) for t in (x, mask, bias))
+        out = Guarded((b, q, k), torch.bfloat16, rocm_device, shift)
+        ok(lib().hipo_scaled_masked_softmax_bf16(xd.data_ptr(), md.data_ptr(), out.t.data_ptr(),
+                                                 b, q, k, k, 0.125, None))
+        torch.cuda.synchronize()
+        out.check(f"masked K={k}")
+        close(out.t, ref.scaled_masked_softmax(x, mask, 0.125), 2 ** -7, 1e-6, f"masked K={k}")
+        out = Guarded((b, q, k), torch.bfloat16, rocm_device, shift)
+        ok(lib().hipo_scaled_bias_softmax_bf16(xd.data_ptr(), bd.data_ptr(), out.t.data_ptr(), b,
+                                               q, k, k, q * k, heads, 0.5, None))
+        torch.cuda.synchronize()
+        out.check(f"bias K={k}")
+        close(out.t, ref.scaled_bias_softmax(x, bias, 0.5, heads), 2 ** -7, 1e-6, f"bias K={k}")
+
+
+@pytest.mark.parametrize("k", [9, 197, 577, 1025])
+def test_softmax_odd_rows_special_values(k, rocm_device):
+    """A row that is -inf throughout is NaN; NaN and +inf scores make their
+    row NaN and no other."""
+    import hip_oracles
+    torch.manual_seed(k)
+    x = torch.randn(6, k).to(torch.bfloat16)
+    x[1] = float("-inf")
+    x[2, k - 1] = float("nan")
+    x[3, k - 2] = float("inf")
+    x[4, : k - 1] = float("-inf")
+    got = hip_oracles.softmax_lastdim(x.to(rocm_device)).float().cpu()
+    assert bool(got[1:4].isnan().all())
+    want = torch.softmax(x.double(), -1).to(torch.bfloat16).float()
+    for r in (0, 4, 5):
+        close(got[r], want[r], 2 ** -7, 1e-6, f"row {r}")
