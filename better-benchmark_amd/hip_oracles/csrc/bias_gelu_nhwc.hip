@@ -9,141 +9,65 @@
 // (gelu_bf16.h: an fp32 evaluation for t > -4 that rounds correctly for
 // every such bf16 t, the exact table in global memory below that).
 //
-// Layout: one wave64 per tile of 64 channels x 64 spatial positions of one
-// image.  Lane l owns an 8x8 (channel x position) block: cb = l / 8 picks 8
-// channels, hb = l % 8 picks 8 positions.  It issues 8 16-byte loads, one
-// per channel row (the 8 lanes of equal cb read one contiguous 128-byte
-// segment of that row), and 8 16-byte stores, one per position (the 8 lanes
-// of equal hb write one contiguous 128-byte segment of that NHWC row); the
-// 8x8 transpose happens in registers, with no LDS and no barrier.  Tiles are
-// numbered channel group fastest, then position tile, then image; a 256-
-// thread workgroup takes four consecutive tiles (with C = 256: all channel
-// groups of one position tile, i.e. 64 whole NHWC rows).  The grid is one-
-// shot (no persistent loop): on MI355X many short workgroups dispatched in
-// order keep the chip's in-flight address window compact (a persistent
-// one-workgroup-per-CU version of this kernel ran 71 us at config 2).  The
-// kernel uses no LDS and has no barrier: a 7 KiB table staged into LDS by
-// every workgroup cost 3-5 us at config 2 (25,088 waves, each waiting at the
-// barrier for the table before its first lookup).
-// Loads and stores are non-temporal.  Launches of at most 2^19 elements
-// (and shapes off the 16-byte vector path) take a one-element-per-thread
-// kernel instead.
+// Layout: 8 x 8 (channel x position) register blocks, 64 of them to a wave
+// (block_tiles.h): 8 16-byte loads along the channel rows, 8 16-byte stores
+// along the NHWC rows, the transpose in registers, with no LDS and no
+// barrier (a 7 KiB table staged into LDS by every workgroup cost 3-5 us at
+// [128, 256, 56, 56]).  Channel tiles are numbered fastest, so a workgroup's
+// four waves write neighbouring parts of the same NHWC rows.  The grid is
+// one-shot (a persistent one-workgroup-per-CU version ran 71 us there).
+// Planes and channel counts of any size >= 8 take it; before, those that are
+// not multiples of 8 took the one-element-per-thread kernel.  Graph replays,
+// before -> now: [128, 384, 14, 14] 49.2 -> 9.4 us, [128, 1024, 14, 14] 111
+// -> 18, [128, 512, 7, 7] 15.3 -> 5.4, [13, 230, 77, 74] 82 -> 14.6; and,
+// multiples of 8, [128, 512, 28, 28] 49.8 -> 38.7, [128, 256, 28, 28] 27.6 ->
+// 17.8, [128, 16, 112, 112] 48 -> 20 ([128, 256, 56, 56] 70 either way).  What is left at 14 x 14
+// (floor 5.8 us) is arithmetic: about 23 issue slots per value.
+// Launches of at most 2^19 elements take the one-element-per-thread kernel.
 // HBM-bound: algorithmic bytes per element = 2 (read) + 2 (write).
+#include "block_tiles.h"
 #include "gelu_bf16.h"
-#include "hipo_common.h"
 
 namespace hipo {
 namespace {
 
-constexpr int kTileHw = 64;  // positions per wave tile
-constexpr int kTileC = 64;   // channels per wave tile
-constexpr int kWavesC = 4;  // waves of a workgroup along channels (consecutive channel tiles)
-constexpr int kWavesP = 1;  // and along positions (consecutive position tiles)
-constexpr int kWavesPerBlock = kWavesC * kWavesP;
-constexpr int kBlockThreads = kWavesPerBlock * kWave;
-constexpr int kTilesPerWave = 1;  // consecutive position tiles per wave (3-D grid)
 constexpr int64_t kTileMinElems = int64_t{1} << 19;  // smaller launches: scalar kernel
 
-struct TileGeom {
-  int64_t C, HW;
-  int c_tiles, hw_tiles, ntiles;  // ntiles < 2^31 (checked on the host)
-};
-
-// GRID3: the grid carries the tile coordinates (x = group of kWavesC channel
-// tiles, y = group of kWavesP x TPW position tiles, z = image), so a workgroup starts its
-// loads without integer divisions (66.1 against 66.6 us at config 2); the
-// dispatch order is the 1-D numbering's.  Otherwise (grids past the y / z
-// limits) the block index is split by division.
-template <bool GRID3, int TPW>
-__global__ __launch_bounds__(kBlockThreads) void bias_gelu_nchw_to_nhwc_tiles(
+template <TileAccess ACCESS>
+__global__ __launch_bounds__(kTileThreads) void bias_gelu_nchw_to_nhwc_blocks(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ bias,
-    uint16_t* __restrict__ out, TileGeom g) {
-  const int lane = threadIdx.x & (kWave - 1);
-  int ct, ht0;
-  int64_t img;
-  bool tile_ok;  // wave-uniform
-  if constexpr (GRID3) {
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    ct = static_cast<int>(blockIdx.x) * kWavesC + wave % kWavesC;
-    ht0 = (static_cast<int>(blockIdx.y) * kWavesP + wave / kWavesC) * TPW;
-    tile_ok = ct < g.c_tiles && ht0 < g.hw_tiles;
-    if (!tile_ok) ct = 0, ht0 = 0;
-    img = blockIdx.z;
-  } else {
-    static_assert(GRID3 || TPW == 1, "the 1-D numbering takes one tile per wave");
-    int t = __builtin_amdgcn_readfirstlane(
-        static_cast<int>(blockIdx.x) * kWavesPerBlock + static_cast<int>(threadIdx.x >> 6));
-    tile_ok = t < g.ntiles;
-    if (!tile_ok) t = 0;
-    ct = t % g.c_tiles;
-    const int rest = t / g.c_tiles;
-    ht0 = rest % g.hw_tiles;
-    img = rest / g.hw_tiles;
-  }
-  const int64_t c0 = static_cast<int64_t>(ct) * kTileC + (lane >> 3) * 8;
-  // Lanes outside a partial tile load from the tile's first block (always in
-  // bounds, no branch around the loads) and store nothing.
-  const bool c_ok = tile_ok && c0 < g.C;
-  const int64_t cl = c_ok ? c0 : static_cast<int64_t>(ct) * kTileC;
-
-  auto load_tile = [&](int ht, u32x4_t (&v)[8]) {
-    const int64_t p0 = static_cast<int64_t>(ht) * kTileHw + (lane & 7) * 8;
-    const int64_t pl = p0 < g.HW ? p0 : static_cast<int64_t>(ht) * kTileHw;
-    const int64_t in_off = (img * g.C + cl) * g.HW + pl;
+    uint16_t* __restrict__ out, BlockTiles t) {
+  const BlockPlace p = block_place(t, 8);  // t.R channels, t.C positions
+  const int64_t img = static_cast<int64_t>(p.mat) * t.R * t.C;
+  const uint16_t* xb = x + img + p.r * t.C + p.c;
+  u32x4_t v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      v[j] = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x4_t*>(x + in_off + j * g.HW));
-  };
-
-  u32x4_t va[8], vb[8];
-  load_tile(ht0, va);
-  const u32x4_t bw = *reinterpret_cast<const u32x4_t*>(bias + cl);
+  for (int j = 0; j < 8; ++j) v[j] = tile_load<ACCESS>(xb + j * t.C);
+  const u32x4_t bw = *reinterpret_cast<const u32x4_a2_t*>(bias + p.r);
   float b[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) b[j] = (j & 1) ? bf16hi(bw[j >> 1]) : bf16lo(bw[j >> 1]);
-
-  auto gelu_store = [&](int ht, const u32x4_t (&v)[8]) {
-    const int64_t p0 = static_cast<int64_t>(ht) * kTileHw + (lane & 7) * 8;
-    if (!c_ok || p0 >= g.HW) return;
-    const int64_t out_off = (img * g.HW + p0) * g.C + c0;
+  if (!p.own) return;  // no barrier follows
+  uint16_t* ob = out + img + p.c * t.R + p.r;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      // Position p0 + i, channels c0 .. c0 + 7: round t for two channels
-      // into one word (v_cvt_pk_bf16_f32), map both halves, pack them.
-      u32x4_t o, tt;
-      bool rare = false;
+  for (int i = 0; i < 8; ++i) {
+    // Position p.c + i, channels p.r .. p.r + 7: round t for two channels
+    // into one word (v_cvt_pk_bf16_f32), map both halves, pack them.
+    u32x4_t o, tt;
+    bool rare = false;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t w0 = v[2 * k][i >> 1];
-        const uint32_t w1 = v[2 * k + 1][i >> 1];
-        const float x0 = (i & 1) ? bf16hi(w0) : bf16lo(w0);
-        const float x1 = (i & 1) ? bf16hi(w1) : bf16lo(w1);
-        tt[k] = pack_bf16x2(x0 + b[2 * k], x1 + b[2 * k + 1]);
-        o[k] = gelu_pair_fast(tt[k], rare);
-      }
-      if (rare) {  // one branch per 8 values, rarely taken for ordinary data
-        gelu_exact_x8(tt, o);
-      }
-      __builtin_nontemporal_store(
-          o, reinterpret_cast<u32x4_t*>(out + out_off + static_cast<int64_t>(i) * g.C));
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t w0 = v[2 * k][i >> 1];
+      const uint32_t w1 = v[2 * k + 1][i >> 1];
+      const float x0 = (i & 1) ? bf16hi(w0) : bf16lo(w0);
+      const float x1 = (i & 1) ? bf16hi(w1) : bf16lo(w1);
+      tt[k] = pack_bf16x2(x0 + b[2 * k], x1 + b[2 * k + 1]);
+      o[k] = gelu_pair_fast(tt[k], rare);
     }
-  };
-
-  // TPW consecutive position tiles per wave: the next tile's loads are
-  // issued before the current one is mapped and stored.
-#pragma unroll
-  for (int r = 0; r < TPW; ++r) {
-    const int ht = ht0 + r;
-    if (ht >= g.hw_tiles) break;  // wave-uniform; no barrier follows
-    const bool next = r + 1 < TPW && ht + 1 < g.hw_tiles;
-    if (r % 2 == 0) {
-      if (next) load_tile(ht + 1, vb);
-      gelu_store(ht, va);
-    } else {
-      if (next) load_tile(ht + 1, va);
-      gelu_store(ht, vb);
+    if (rare) {  // one branch per 8 values, rarely taken for ordinary data
+      gelu_exact_x8(tt, o);
     }
+    tile_store<ACCESS>(o, ob + i * t.R);
   }
 }
 
@@ -185,34 +109,15 @@ extern "C" int hipo_bias_gelu_nchw_to_nhwc_bf16(const uint16_t* x,
   // memory (steady-state: 5.4 against 2.5 us at [3, 320, 8, 10], 5.9
   // against 3.2 us at [4, 128, 28, 28]; 6.7 against 10.8 us at
   // [2, 256, 56, 56], where the tiles win).
-  const bool vec = n * c * hw > kTileMinElems && (c % 8 == 0) && (hw % 8 == 0) &&
-                   aligned16(x) && aligned16(bias) && aligned16(out);
-  if (vec) {
-    const int64_t c_tiles = (c + kTileC - 1) / kTileC;
-    const int64_t hw_tiles = (hw + kTileHw - 1) / kTileHw;
-    const int64_t ntiles = n * c_tiles * hw_tiles;
-    HIPO_REQUIRE(ntiles < (int64_t{1} << 31) - kWavesPerBlock,
-                 "bias_gelu: %lld tiles exceed the 32-bit tile index",
-                 (long long)ntiles);
-    TileGeom g;
-    g.C = c;
-    g.HW = hw;
-    g.c_tiles = static_cast<int>(c_tiles);
-    g.hw_tiles = static_cast<int>(hw_tiles);
-    g.ntiles = static_cast<int>(ntiles);
-    const int64_t c_groups = (c_tiles + kWavesC - 1) / kWavesC;
-    const int64_t hw_groups =
-        (hw_tiles + kWavesP * kTilesPerWave - 1) / (kWavesP * kTilesPerWave);
-    if (hw_groups <= 65535 && n <= 65535) {
-      const dim3 grid(static_cast<unsigned>(c_groups), static_cast<unsigned>(hw_groups),
-                      static_cast<unsigned>(n));
-      bias_gelu_nchw_to_nhwc_tiles<true, kTilesPerWave>
-          <<<grid, dim3(kBlockThreads), 0, stream>>>(x, bias, out, g);
-    } else {
-      const int64_t blocks = (ntiles + kWavesPerBlock - 1) / kWavesPerBlock;
-      bias_gelu_nchw_to_nhwc_tiles<false, 1><<<dim3(static_cast<unsigned>(blocks)),
-                                               dim3(kBlockThreads), 0, stream>>>(x, bias, out, g);
-    }
+  BlockTiles t;
+  TileAccess access;
+  if (n * c * hw > kTileMinElems && block_tiles(x, out, n, c, hw, 2, t, access)) {
+    auto kernel = access == TileAccess::kCached
+                      ? bias_gelu_nchw_to_nhwc_blocks<TileAccess::kCached>
+                  : access == TileAccess::kStreamOut
+                      ? bias_gelu_nchw_to_nhwc_blocks<TileAccess::kStreamOut>
+                      : bias_gelu_nchw_to_nhwc_blocks<TileAccess::kStream>;
+    kernel<<<dim3(t.workgroups()), dim3(kTileThreads), 0, stream>>>(x, bias, out, t);
   } else {
     const int64_t total = n * c * hw;
     int64_t blocks = (total + 255) / 256;

@@ -56,7 +56,8 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // The same 16 bytes at any element's address (2- or 4-byte aligned): one
 // global_load / store_dwordx4 still, the target runs with unaligned access
-// enabled.  Rows and planes that are not a whole number of vectors use them.
+// enabled.  Rows and planes that are not a whole number of vectors use them
+// (as plain pointee types: a template argument drops the alignment).
 typedef u32x4_t u32x4_a2_t __attribute__((aligned(2)));
 typedef f32x4_t f32x4_a4_t __attribute__((aligned(4)));
 
@@ -110,6 +111,16 @@ inline DivMagic div_magic(uint32_t d) {
 
 __device__ __forceinline__ uint32_t div_by(uint32_t n, DivMagic m) {
   return static_cast<uint32_t>((static_cast<uint64_t>(n) * m.magic) >> m.shift);
+}
+
+// XCD-aware order: workgroup ids go round-robin over the 8 XCDs, each with
+// its own L2.  Block `bid` of `n` takes place (bid % 8) * (n / 8) + bid / 8,
+// so each XCD works through one contiguous eighth, and the cache lines that
+// neighbouring blocks share are fetched into (and merged in) one L2.  The
+// last n % 8 blocks keep their place.
+__device__ __forceinline__ uint32_t xcd_order(uint32_t bid, uint32_t n) {
+  const uint32_t per = n >> 3;
+  return bid < per * 8 ? (bid & 7) * per + (bid >> 3) : bid;
 }
 
 // DPP controls (GFX9 encoding).

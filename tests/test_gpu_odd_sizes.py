@@ -102,3 +102,50 @@ def test_softmax_odd_rows_special_values(k, rocm_device):
     want = torch.softmax(x.double(), -1).to(torch.bfloat16).float()
     for r in (0, 4, 5):
         close(got[r], want[r], 2 ** -7, 1e-6, f"row {r}")
+
+
+# (channels, positions): one block each way, one value more, odd planes, more
+# block columns than a tile's 8 and fewer rows, thin output rows, fewer values
+# than a block (the one-element kernel).  n fills the tile kernel's minimum.
+BIAS_GELU_CP = [(8, 8), (9, 8), (8, 9), (65, 49), (64, 196), (100, 25), (16, 1001), (230, 77),
+                (513, 17), (7, 500), (300, 7)]
+
+
+@pytest.mark.parametrize("c,hw", BIAS_GELU_CP)
+def test_bias_gelu_any_plane(c, hw, rocm_device):
+    """Both sides hold the correctly rounded bf16: equal bit for bit."""
+    import oracle as ref
+    torch.manual_seed(c * 1000 + hw)
+    for n in (1, (1 << 19) // (c * hw) + 2):
+        x = torch.randn(n, c, 1, hw).to(torch.bfloat16) * 3
+        bias = torch.randn(c).to(torch.bfloat16)
+        want = ref.bias_gelu_nchw_to_nhwc(x, bias).permute(0, 2, 3, 1)
+        for shift in (0, 1):
+            xd, bd = place(x, rocm_device, shift), place(bias, rocm_device, shift)
+            out = Guarded((n, 1, hw, c), torch.bfloat16, rocm_device, shift)
+            ok(lib().hipo_bias_gelu_nchw_to_nhwc_bf16(xd.data_ptr(), bd.data_ptr(),
+                                                      out.t.data_ptr(), n, c, hw, None))
+            torch.cuda.synchronize()
+            out.check(f"[{n}, {c}, {hw}]")
+            assert torch.equal(out.t.cpu(), want), f"[{n}, {c}, {hw}] shift {shift}"
+
+
+# Matrices past the whole-matrix kernel's 32 KiB: sides of exactly one block,
+# one element more, odd on either side or both, thin ones (general kernel).
+TRANSPOSE_RC = [(8, 4096), (4096, 8), (9, 2500), (2500, 9), (197, 768), (768, 197), (333, 129),
+                (129, 333), (1001, 65), (3, 20000), (20000, 3), (200, 200)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["b16", "b32"])
+@pytest.mark.parametrize("r,c", TRANSPOSE_RC)
+def test_transpose_any_matrix(r, c, dtype, rocm_device):
+    torch.manual_seed(r * 7 + c)
+    x = torch.randn(3, r, c).to(dtype)
+    for shift in (0, 1):
+        xd = place(x, rocm_device, shift)
+        out = Guarded((3, c, r), dtype, rocm_device, shift)
+        ok(lib().hipo_transpose_last2(xd.data_ptr(), out.t.data_ptr(), 3, r, c,
+                                      x.element_size(), None))
+        torch.cuda.synchronize()
+        out.check(f"[{r}, {c}]")
+        assert torch.equal(out.t.cpu(), x.transpose(1, 2).contiguous()), f"[{r}, {c}]"
