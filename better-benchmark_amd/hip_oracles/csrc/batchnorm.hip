@@ -1,23 +1,24 @@
 // BatchNorm training forward, fp32 NCHW: per-channel statistics over
 // (N, H, W), normalisation + affine (+ ReLU), running-stat update.
 //
-// Entry point.  Channels of at most 16384 values take one launch with a
-// workgroup per channel that holds its channel in registers
-// (bn_channel_small).  Larger channels take the single-pass persistent
-// kernel (batchnorm_fused.hip) wherever it applies, and the split-K path
-// below otherwise (HW not a multiple of 4, unaligned pointers, very large
-// tensors, more than 64 workgroups per channel or 64 rounds).
+// Entry point.  Channels of at most 16384 values, and larger ones where that
+// measured faster (kLargeChannel), take one launch with a workgroup per
+// channel that holds its channel in registers (bn_channel_small).  Other
+// channels take the single-pass persistent kernel (batchnorm_fused.hip)
+// wherever it applies, and the split-K path below otherwise (HW not a
+// multiple of 4, unaligned pointers, very large tensors, more than 64
+// workgroups per channel or 64 rounds).
 //
 // Split-K structure (two launches on the caller's stream):
-//   1. bn_partial_stats: grid (S, C).  Workgroup (s, c) reduces the planes
+//   1. bn_partial_stats: S x C workgroups.  Workgroup (s, c) reduces the planes
 //      n in [s*N/S, (s+1)*N/S) of channel c to a Welford triple
 //      (count, mean, M2) and writes it to the workspace.  Inside the
 //      workgroup each thread reduces its slice of every plane exactly
 //      (two-pass over registers) and merges it into a running triple with
 //      Chan's formula; threads then merge across the wave with DPP and
 //      across waves through LDS.
-//   2. bn_normalize: grid (S, C).  Every workgroup of channel c merges the S
-//      triples of that channel (Chan, fp64, fixed order), derives
+//   2. bn_normalize: S x C workgroups.  The first wave of each merges the S
+//      triples of its channel (fp64, fixed order), derives
 //      mean / invstd, and writes y = relu?(x * alpha + beta') for its planes
 //      with alpha = invstd * gamma, beta' = beta - mean * alpha.  Workgroup
 //      (0, c) also writes save_mean / save_invstd and updates the running
@@ -32,7 +33,6 @@ namespace hipo {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWavesPerBlock = kThreads / kWave;
 
 // max(v, 0) that keeps NaN (torch.relu propagates NaN; fmaxf would not).
 __device__ __forceinline__ float relu_f32(float v) { return v < 0.f ? 0.f : v; }
@@ -57,6 +57,32 @@ __device__ __forceinline__ void absorb(Welford& acc, const float4 (&v)[U],
     if (ok[u]) {
       const float a = v[u].x - m, b = v[u].y - m, c = v[u].z - m, d = v[u].w - m;
       q += (a * a + b * b) + (c * c + d * d);
+    }
+  }
+  acc = welford_merge(acc, Welford{cnt, m, q});
+}
+
+// The same for up to U vectors whose first skip[u] values (4: all) belong to
+// another vector.
+template <int U>
+__device__ __forceinline__ void absorb(Welford& acc, const f32x4_t (&v)[U],
+                                       const int (&skip)[U]) {
+  float cnt = 0.f, s = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    cnt += static_cast<float>(4 - skip[u]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s += e >= skip[u] ? v[u][e] : 0.f;
+  }
+  if (cnt == 0.f) return;
+  const float m = s / cnt;
+  float q = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float d = e >= skip[u] ? v[u][e] - m : 0.f;
+      q = __builtin_fmaf(d, d, q);
     }
   }
   acc = welford_merge(acc, Welford{cnt, m, q});
@@ -90,41 +116,88 @@ __device__ __forceinline__ void split_range(int64_t N, int64_t S, int64_t s,
   n1 = (N * (s + 1)) / S;
 }
 
-// Merge the threads' triples: DPP across the wave, LDS across the waves.
-// Every thread returns the workgroup's total.
+// Merge the threads' triples: DPP across the wave, then the waves' triples,
+// through LDS, by the same butterflies in every wave (4 or 16 waves: two or
+// four steps), of which lane 0's order counts.  Every thread returns the
+// workgroup's total.
+template <int T = kThreads>
 __device__ __forceinline__ Welford block_welford(Welford acc) {
+  constexpr int kWaves = T / kWave;
+  static_assert(kWaves == 4 || kWaves == 16, "the waves' triples fill quads or rows");
   acc = wave_welford(acc);
-  __shared__ Welford part[kWavesPerBlock];
+  __shared__ Welford part[kWaves];
   const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & (kWave - 1)) == 0) part[wave] = acc;
   __syncthreads();
-  return welford_merge(welford_merge(part[0], part[1]), welford_merge(part[2], part[3]));
+  Welford w = part[threadIdx.x & (kWaves - 1)];
+  w = welford_merge(w, welford_dpp<kDppQuadXor1>(w));
+  w = welford_merge(w, welford_dpp<kDppQuadXor2>(w));
+  if constexpr (kWaves == 16) {
+    w = welford_merge(w, welford_dpp<kDppRowRor4>(w));
+    w = welford_merge(w, welford_dpp<kDppRowRor8>(w));
+  }
+  return welford_lane(w, 0);
 }
 
+// Planes of HW >= 4 values, any alignment, as F = ceil(HW / 4) vectors each:
+// vector j of a plane starts at value min(4 j, HW - 4), so the last one of a
+// plane that is not a whole number of vectors ends with it, and its first
+// 4 j - start values (`skip`) are its neighbour's.  16-byte accesses at value
+// alignment; a value that two vectors share is normalised by both to the
+// same bits.
+struct PlaneGeom {
+  int64_t HW;
+  int F;  // 1 for planes of 2^30 values and more, which go value by value
+  DivMagic by_F;
+};
+
+inline PlaneGeom plane_geom(int64_t hw) {
+  PlaneGeom g;
+  g.HW = hw;
+  g.F = hw < (int64_t{1} << 30) ? static_cast<int>((hw + 3) / 4) : 1;
+  g.by_F = div_magic(static_cast<uint32_t>(g.F));
+  return g;
+}
+
+struct PlaneVec {
+  int64_t off;  // value offset, planes `stride` values apart
+  int skip;
+};
+
+__device__ __forceinline__ PlaneVec plane_vec(const PlaneGeom& g, int64_t stride, uint32_t i) {
+  const uint32_t n = div_by(i, g.by_F);
+  const int first = static_cast<int>(i - n * static_cast<uint32_t>(g.F)) * 4;
+  const int last = static_cast<int>(g.HW) - 4;
+  const int start = first < last ? first : last;
+  return PlaneVec{static_cast<int64_t>(n) * stride + start, first - start};
+}
+
+constexpr int kSplitLoads = 8;  // vectors in flight per thread
+
 // Welford triple of planes [n0, n1) of channel c over the workgroup: each
-// thread reduces its slice of every plane exactly (two-pass over registers)
-// and merges it into a running triple with Chan's formula; the wave merges
-// with DPP and the waves through LDS.  Thread 0 returns the total.
+// thread reduces its values exactly (two-pass over registers), kSplitLoads
+// vectors of consecutive planes at a time, and merges them into a running
+// triple with Chan's formula; the wave merges with DPP and the waves through
+// LDS.  Thread 0 returns the total.
 template <bool VEC>
 __device__ Welford planes_welford(const float* __restrict__ x, int64_t n0, int64_t n1,
-                                  int64_t C, int64_t HW, int64_t c) {
+                                  int64_t C, const PlaneGeom& g, int64_t c) {
   Welford acc{0.f, 0.f, 0.f};
+  const int64_t HW = g.HW;
   if constexpr (VEC) {
-    constexpr int U = 4;
-    const int64_t hw4 = HW / 4;
-    for (int64_t n = n0; n < n1; ++n) {
-      const float4* plane = reinterpret_cast<const float4*>(x + (n * C + c) * HW);
-      for (int64_t base = 0; base < hw4; base += kThreads * U) {
-        float4 v[U];
-        bool ok[U];
+    const float* base = x + (n0 * C + c) * HW;
+    const uint32_t total = static_cast<uint32_t>(n1 - n0) * static_cast<uint32_t>(g.F);
+    for (uint32_t i0 = threadIdx.x; i0 < total; i0 += kThreads * kSplitLoads) {
+      f32x4_t v[kSplitLoads];
+      int skip[kSplitLoads];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int64_t i = base + u * kThreads + threadIdx.x;
-          ok[u] = i < hw4;
-          v[u] = ok[u] ? plane[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        absorb<U>(acc, v, ok);
+      for (int u = 0; u < kSplitLoads; ++u) {
+        const uint32_t i = i0 + static_cast<uint32_t>(u) * kThreads;
+        const PlaneVec p = plane_vec(g, C * HW, i < total ? i : i0);
+        v[u] = *reinterpret_cast<const f32x4_a4_t*>(base + p.off);
+        skip[u] = i < total ? p.skip : 4;
       }
+      absorb<kSplitLoads>(acc, v, skip);
     }
   } else {
     for (int64_t n = n0; n < n1; ++n) {
@@ -140,12 +213,13 @@ __device__ Welford planes_welford(const float* __restrict__ x, int64_t n0, int64
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void bn_partial_stats(
     const float* __restrict__ x, float* __restrict__ ws, int64_t N, int64_t C,
-    int64_t HW, int64_t S) {
-  const int64_t s = blockIdx.x;
-  const int64_t c = blockIdx.y;
+    PlaneGeom g, int64_t S, DivMagic by_S) {
+  const uint32_t bid = xcd_order(blockIdx.x, gridDim.x);
+  const int64_t c = div_by(bid, by_S);
+  const int64_t s = bid - c * S;
   int64_t n0, n1;
   split_range(N, S, s, n0, n1);
-  const Welford t = planes_welford<VEC>(x, n0, n1, C, HW, c);
+  const Welford t = planes_welford<VEC>(x, n0, n1, C, g, c);
   if (threadIdx.x == 0) {
     float* dst = ws + (c * S + s) * 3;
     dst[0] = t.n;
@@ -154,23 +228,30 @@ __global__ __launch_bounds__(kThreads) void bn_partial_stats(
   }
 }
 
-// Merge the S partial triples of channel c in fp64, fixed order.
+// Merge the S partial triples of channel c in fp64 about the first one's
+// mean K: with d_s = mean_s - K, S1 = sum n_s d_s and S2 = sum M2_s + n_s
+// d_s^2, mean = K + S1 / N and M2 = S2 - S1^2 / N.  One wave: lane l adds
+// splits l, l + 64, ... in order, then wave_sum (a fixed order).  All 64
+// lanes active; every lane returns the result.
 __device__ void channel_stats(const float* __restrict__ ws, int64_t c,
                               int64_t S, double& mean, double& m2,
                               double& count) {
-  double n = 0.0, mu = 0.0, q = 0.0;
-  for (int64_t s = 0; s < S; ++s) {
-    const float* p = ws + (c * S + s) * 3;
-    const double nb = p[0], mb = p[1], qb = p[2];
-    const double nn = n + nb;
-    if (nn == 0.0) continue;
-    const double d = mb - mu;
-    mu += d * (nb / nn);
-    q += qb + d * d * n * (nb / nn);
-    n = nn;
+  const float* p = ws + c * S * 3;
+  const double K = p[1];
+  double n = 0.0, s1 = 0.0, s2 = 0.0;
+  for (int64_t s = threadIdx.x & (kWave - 1); s < S; s += kWave) {
+    const double nb = p[3 * s], d = static_cast<double>(p[3 * s + 1]) - K;
+    n += nb;
+    s1 = __builtin_fma(nb, d, s1);
+    s2 += __builtin_fma(nb * d, d, static_cast<double>(p[3 * s + 2]));
   }
-  mean = mu;
-  m2 = q;
+  n = wave_sum(n);
+  s1 = wave_sum(s1);
+  s2 = wave_sum(s2);
+  const double dm = s1 / n;
+  mean = K + dm;
+  // max (NaN from the data kept): rounding can leave a tiny negative.
+  m2 = __builtin_elementwise_maximum(s2 - s1 * dm, 0.0);
   count = n;
 }
 
@@ -214,28 +295,35 @@ __device__ void channel_coefs(double mean, double m2, double count, int64_t c,
 // y = relu?(x * alpha + shift) over planes [n0, n1) of channel c.
 template <bool VEC>
 __device__ void normalize_planes(const float* __restrict__ x, float* __restrict__ y,
-                                 int64_t n0, int64_t n1, int64_t C, int64_t HW, int64_t c,
-                                 float alpha, float shift, int relu) {
-  for (int64_t n = n0; n < n1; ++n) {
-    const int64_t off = (n * C + c) * HW;
-    if (VEC) {
-      const float4* src = reinterpret_cast<const float4*>(x + off);
-      float4* dst = reinterpret_cast<float4*>(y + off);
-      for (int64_t i = threadIdx.x; i < HW / 4; i += kThreads) {
-        float4 v = src[i];
-        v.x = __builtin_fmaf(v.x, alpha, shift);
-        v.y = __builtin_fmaf(v.y, alpha, shift);
-        v.z = __builtin_fmaf(v.z, alpha, shift);
-        v.w = __builtin_fmaf(v.w, alpha, shift);
-        if (relu) {
-          v.x = relu_f32(v.x);
-          v.y = relu_f32(v.y);
-          v.z = relu_f32(v.z);
-          v.w = relu_f32(v.w);
-        }
-        dst[i] = v;
+                                 int64_t n0, int64_t n1, int64_t C, const PlaneGeom& g,
+                                 int64_t c, float alpha, float shift, int relu) {
+  const int64_t HW = g.HW;
+  if constexpr (VEC) {
+    const int64_t base = (n0 * C + c) * HW;
+    const uint32_t total = static_cast<uint32_t>(n1 - n0) * static_cast<uint32_t>(g.F);
+    for (uint32_t i0 = threadIdx.x; i0 < total; i0 += kThreads * kSplitLoads) {
+      f32x4_t v[kSplitLoads];
+      int64_t off[kSplitLoads];
+#pragma unroll
+      for (int u = 0; u < kSplitLoads; ++u) {
+        const uint32_t i = i0 + static_cast<uint32_t>(u) * kThreads;
+        off[u] = plane_vec(g, C * HW, i < total ? i : i0).off;
+        v[u] = *reinterpret_cast<const f32x4_a4_t*>(x + base + off[u]);
       }
-    } else {
+#pragma unroll
+      for (int u = 0; u < kSplitLoads; ++u) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[u][e] = __builtin_fmaf(v[u][e], alpha, shift);
+          if (relu) v[u][e] = relu_f32(v[u][e]);
+        }
+        if (i0 + static_cast<uint32_t>(u) * kThreads < total)
+          *reinterpret_cast<f32x4_a4_t*>(y + base + off[u]) = v[u];
+      }
+    }
+  } else {
+    for (int64_t n = n0; n < n1; ++n) {
+      const int64_t off = (n * C + c) * HW;
       for (int64_t i = threadIdx.x; i < HW; i += kThreads) {
         float v = __builtin_fmaf(x[off + i], alpha, shift);
         if (relu) v = relu_f32(v);
@@ -251,21 +339,23 @@ __global__ __launch_bounds__(kThreads) void bn_normalize(
     const float* __restrict__ beta, float* __restrict__ running_mean,
     float* __restrict__ running_var, float* __restrict__ y,
     float* __restrict__ save_mean, float* __restrict__ save_invstd,
-    const float* __restrict__ ws, int64_t N, int64_t C, int64_t HW, int64_t S,
+    const float* __restrict__ ws, int64_t N, int64_t C, PlaneGeom g, int64_t S, DivMagic by_S,
     float momentum, float eps, int relu) {
-  const int64_t s = blockIdx.x;
-  const int64_t c = blockIdx.y;
+  const uint32_t bid = xcd_order(blockIdx.x, gridDim.x);
+  const int64_t c = div_by(bid, by_S);
+  const int64_t s = bid - c * S;
   __shared__ float coef[2];
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < kWave) {
     double mean, m2, count;
     channel_stats(ws, c, S, mean, m2, count);
-    channel_coefs(mean, m2, count, c, gamma, beta, running_mean, running_var, save_mean,
-                  save_invstd, momentum, eps, s == 0, coef);
+    if (threadIdx.x == 0)
+      channel_coefs(mean, m2, count, c, gamma, beta, running_mean, running_var, save_mean,
+                    save_invstd, momentum, eps, s == 0, coef);
   }
   __syncthreads();
   int64_t n0, n1;
   split_range(N, S, s, n0, n1);
-  normalize_planes<VEC>(x, y, n0, n1, C, HW, c, coef[0], coef[1], relu);
+  normalize_planes<VEC>(x, y, n0, n1, C, g, c, coef[0], coef[1], relu);
 }
 
 // Small channels (N * HW <= kSmallChannel values): one launch, a workgroup
@@ -280,22 +370,47 @@ __global__ __launch_bounds__(kThreads) void bn_normalize(
 // or [4, 24, 10, 10] that chain, not the bytes, is the time (the
 // single-pass kernel adds an epoch read and a slab exchange to it).
 constexpr int64_t kSmallChannel = 16384;
+// Larger ones take the same kernel with 1024 threads: whole float4 planes up
+// to 7 a thread (28672 values; two workgroups per CU) and at least 32
+// channels, ragged ones, whose alternative reads x twice, up to 12 vectors a
+// thread.  Graph replays in us, single-pass kernel / here, inputs reused [not
+// reused]: [128, 1024, 14, 14] 56.7 / 39.3 [57.3 / 47.7], [128, 256, 14, 14]
+// 15.6 / 11.9 [16.5 / 14.8], [128, 64, 14, 14] 9.2 / 7.1 [9.6 / 8.6], but
+// [64, 512, 28, 28], 50176 values, 37.7 / 40.5 [37.8 / 52.0] and [6, 960, 72,
+// 70], 30240, 52.4 / 47.8 [52.8 / 57.8].  Split-K before / split-K now / here:
+// [512, 512, 7, 7] 95 / 34.5 / 23.0, [17, 488, 35, 37] 41.2 / 32.5 / 19.4, [21,
+// 782, 46, 43] 119 / 81 / 58, [12, 1280, 46, 45] 105 / 78 / 53; with 16 vectors
+// a thread (and spills) [5, 32, 101, 99] 22.7 / 9.7 / 12.3.
+constexpr int64_t kLargeChannel = 65536;
+constexpr int kLargeThreads = 1024;
+constexpr int64_t kLargeMinChannels = 32;
 
+// Planes that are not whole float4s, or not 16-byte aligned, are cut into
+// vectors at value alignment (PlaneGeom); planes below 9 values that are not
+// a multiple of 4, where over a third of those vectors' values would be
+// read twice, go value by value.  Workgroups in XCD order: neighbouring
+// channels share the cache lines at their planes' ends.  [128, 2048, 7, 7]
+// 39.0 us value by value -> 19.0 (5.4 TB/s).
 struct SmallGeom {
-  int total;      // float4 (VEC) or values per channel
-  int per_plane;  // HW / 4 (VEC) or HW
+  int total;      // vectors, or values, per channel
+  int per_plane;  // HW / 4 (kWhole) or HW (kValues)
   DivMagic by_plane;
+  PlaneGeom ragged;  // kRagged
 };
 
-template <bool VEC, int U>
-__global__ __launch_bounds__(kThreads) void bn_channel_small(
+enum class SmallKind { kValues, kWhole, kRagged };
+
+template <SmallKind KIND, int U, int T>
+__global__ __launch_bounds__(T) void bn_channel_small(
     const float* __restrict__ x, const float* __restrict__ gamma,
     const float* __restrict__ beta, float* __restrict__ running_mean,
     float* __restrict__ running_var, float* __restrict__ y,
     float* __restrict__ save_mean, float* __restrict__ save_invstd, SmallGeom g, int64_t C,
     float momentum, float eps, int relu) {
-  using Elem = std::conditional_t<VEC, float4, float>;
-  const int64_t c = blockIdx.x;
+  constexpr bool kVec = KIND != SmallKind::kValues;
+  constexpr bool kRagged = KIND == SmallKind::kRagged;
+  using Elem = std::conditional_t<kRagged, f32x4_t, std::conditional_t<kVec, float4, float>>;
+  const int64_t c = xcd_order(blockIdx.x, gridDim.x);
   float pg = 0.f, pb = 0.f, prm = 0.f, prv = 0.f;
   if (threadIdx.x == 0) {
     pg = gamma[c];
@@ -303,26 +418,43 @@ __global__ __launch_bounds__(kThreads) void bn_channel_small(
     prm = running_mean[c];
     prv = running_var[c];
   }
-  // Element i of the channel: plane i / per_plane, offset i % per_plane.
+  // Element i of the channel: plane i / per_plane, offset i % per_plane
+  // (in units of Elem; kRagged: the vector's value offset and its skip).
   auto offset = [&](int i) {
-    const uint32_t n = div_by(static_cast<uint32_t>(i), g.by_plane);
-    return (static_cast<int64_t>(n) * C + c) * g.per_plane +
-           (i - static_cast<int>(n) * g.per_plane);
+    if constexpr (kRagged) {
+      PlaneVec p = plane_vec(g.ragged, C * g.ragged.HW, static_cast<uint32_t>(i));
+      p.off += c * g.ragged.HW;
+      return p;
+    } else {
+      const uint32_t n = div_by(static_cast<uint32_t>(i), g.by_plane);
+      return (static_cast<int64_t>(n) * C + c) * g.per_plane +
+             (i - static_cast<int>(n) * g.per_plane);
+    }
   };
-  const Elem* xs = reinterpret_cast<const Elem*>(x);
   Elem v[U];
   bool ok[U];
+  int skip[U];
   // Unconditional loads (threads past the channel's end re-read its last
   // element and store nothing), so all of them are in flight together.
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int i = static_cast<int>(threadIdx.x) + u * kThreads;
+    const int i = static_cast<int>(threadIdx.x) + u * T;
     ok[u] = i < g.total;
-    v[u] = xs[offset(ok[u] ? i : g.total - 1)];
+    const auto at = offset(ok[u] ? i : g.total - 1);
+    if constexpr (kRagged) {
+      v[u] = *reinterpret_cast<const f32x4_a4_t*>(x + at.off);
+      skip[u] = ok[u] ? at.skip : 4;
+    } else {
+      v[u] = reinterpret_cast<const Elem*>(x)[at];
+    }
   }
   Welford acc{0.f, 0.f, 0.f};
-  absorb<U>(acc, v, ok);
-  const Welford t = block_welford(acc);
+  if constexpr (kRagged) {
+    absorb<U>(acc, v, skip);
+  } else {
+    absorb<U>(acc, v, ok);
+  }
+  const Welford t = block_welford<T>(acc);
   __shared__ float coef[2];
   if (threadIdx.x == 0)
     channel_coefs_of(static_cast<double>(t.mean), static_cast<double>(t.m2),
@@ -330,12 +462,11 @@ __global__ __launch_bounds__(kThreads) void bn_channel_small(
                      save_mean, save_invstd, momentum, eps, true, coef);
   __syncthreads();
   const float alpha = coef[0], shift = coef[1];
-  Elem* ys = reinterpret_cast<Elem*>(y);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (!ok[u]) continue;
     Elem o = v[u];
-    if constexpr (VEC) {
+    if constexpr (kVec) {
       o.x = __builtin_fmaf(o.x, alpha, shift);
       o.y = __builtin_fmaf(o.y, alpha, shift);
       o.z = __builtin_fmaf(o.z, alpha, shift);
@@ -350,45 +481,76 @@ __global__ __launch_bounds__(kThreads) void bn_channel_small(
       o = __builtin_fmaf(o, alpha, shift);
       if (relu) o = relu_f32(o);
     }
-    ys[offset(static_cast<int>(threadIdx.x) + u * kThreads)] = o;
+    const auto at = offset(static_cast<int>(threadIdx.x) + u * T);
+    if constexpr (kRagged) {
+      *reinterpret_cast<f32x4_a4_t*>(y + at.off) = o;
+    } else {
+      reinterpret_cast<Elem*>(y)[at] = o;
+    }
   }
 }
 
-template <bool VEC, int U>
+template <SmallKind KIND, int U, int T = kThreads>
 void launch_small(const float* x, const float* gamma, const float* beta, float* running_mean,
                   float* running_var, float* y, float* save_mean, float* save_invstd,
                   const SmallGeom& g, int64_t c, float momentum, float eps, int relu,
                   hipStream_t stream) {
-  bn_channel_small<VEC, U><<<dim3(static_cast<unsigned>(c)), dim3(kThreads), 0, stream>>>(
+  bn_channel_small<KIND, U, T><<<dim3(static_cast<unsigned>(c)), dim3(T), 0, stream>>>(
       x, gamma, beta, running_mean, running_var, y, save_mean, save_invstd, g, c, momentum,
       eps, relu);
 }
 
-// U = the smallest instantiated count covering the channel.
+// Launches the register-held kernel, U = the smallest instantiated count
+// covering the channel; -1 if it does not take the shape.
 int small_launch(const float* x, const float* gamma, const float* beta, float* running_mean,
                  float* running_var, float* y, float* save_mean, float* save_invstd, int64_t n,
                  int64_t c, int64_t hw, float momentum, float eps, int relu,
                  hipStream_t stream) {
-  const bool vec = hw % 4 == 0 && aligned16(x) && aligned16(y);
+  if (c > 0x7fffffff || hw > kLargeChannel || n * hw > kLargeChannel) return -1;
+  const bool whole = hw % 4 == 0 && aligned16(x) && aligned16(y);
+  const bool ragged = !whole && (hw % 4 == 0 || hw >= 9);
   SmallGeom g;
-  g.per_plane = static_cast<int>(vec ? hw / 4 : hw);
-  g.total = static_cast<int>(n) * g.per_plane;
+  g.per_plane = static_cast<int>(whole ? hw / 4 : hw);
   g.by_plane = div_magic(static_cast<uint32_t>(g.per_plane));
+  g.ragged = plane_geom(hw);
+  g.total = static_cast<int>(n) * (ragged ? g.ragged.F : g.per_plane);
+#define HIPO_BN_SMALL(K, ...)                                                        \
+  launch_small<SmallKind::K, __VA_ARGS__>(x, gamma, beta, running_mean, running_var, y, \
+                                          save_mean, save_invstd, g, c, momentum, eps,  \
+                                          relu, stream)
+  if (n * hw > kSmallChannel) {
+    const int per_thread = (g.total + kLargeThreads - 1) / kLargeThreads;
+    if (whole && c >= kLargeMinChannels && per_thread <= 7)
+      HIPO_BN_SMALL(kWhole, 7, kLargeThreads);
+    else if (ragged && per_thread <= 8)
+      HIPO_BN_SMALL(kRagged, 8, kLargeThreads);
+    else if (ragged && per_thread <= 12)
+      HIPO_BN_SMALL(kRagged, 12, kLargeThreads);
+    else
+      return -1;
+    return check_launch("batchnorm_train_fwd_f32 (channels in registers)");
+  }
   const int per_thread = (g.total + kThreads - 1) / kThreads;
-#define HIPO_BN_SMALL(V, U)                                                              \
-  launch_small<V, U>(x, gamma, beta, running_mean, running_var, y, save_mean, save_invstd, \
-                     g, c, momentum, eps, relu, stream)
-  if (vec) {
-    if (per_thread <= 1) HIPO_BN_SMALL(true, 1);
-    else if (per_thread <= 2) HIPO_BN_SMALL(true, 2);
-    else if (per_thread <= 4) HIPO_BN_SMALL(true, 4);
-    else if (per_thread <= 8) HIPO_BN_SMALL(true, 8);
-    else HIPO_BN_SMALL(true, 16);
+  if (whole) {
+    if (per_thread <= 1) HIPO_BN_SMALL(kWhole, 1);
+    else if (per_thread <= 2) HIPO_BN_SMALL(kWhole, 2);
+    else if (per_thread <= 4) HIPO_BN_SMALL(kWhole, 4);
+    else if (per_thread <= 8) HIPO_BN_SMALL(kWhole, 8);
+    else HIPO_BN_SMALL(kWhole, 16);
+  } else if (ragged) {
+    // At most 16384 values in planes of 9 or more: 12 / 9 of them in
+    // vectors, 21.3 a thread.
+    if (per_thread <= 1) HIPO_BN_SMALL(kRagged, 1);
+    else if (per_thread <= 2) HIPO_BN_SMALL(kRagged, 2);
+    else if (per_thread <= 4) HIPO_BN_SMALL(kRagged, 4);
+    else if (per_thread <= 8) HIPO_BN_SMALL(kRagged, 8);
+    else if (per_thread <= 16) HIPO_BN_SMALL(kRagged, 16);
+    else HIPO_BN_SMALL(kRagged, 24);
   } else {
-    if (per_thread <= 1) HIPO_BN_SMALL(false, 1);
-    else if (per_thread <= 4) HIPO_BN_SMALL(false, 4);
-    else if (per_thread <= 16) HIPO_BN_SMALL(false, 16);
-    else HIPO_BN_SMALL(false, 64);
+    if (per_thread <= 1) HIPO_BN_SMALL(kValues, 1);
+    else if (per_thread <= 4) HIPO_BN_SMALL(kValues, 4);
+    else if (per_thread <= 16) HIPO_BN_SMALL(kValues, 16);
+    else HIPO_BN_SMALL(kValues, 64);
   }
 #undef HIPO_BN_SMALL
   return check_launch("batchnorm_train_fwd_f32 (small channels)");
@@ -431,37 +593,31 @@ extern "C" int hipo_batchnorm_train_fwd_f32(
                need);
   HIPO_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 8 == 0,
                "batchnorm: workspace must be 8-byte aligned");
-  if (n * hw <= kSmallChannel && c <= 0x7fffffff)
-    return small_launch(x, gamma, beta, running_mean, running_var, y, save_mean, save_invstd,
-                        n, c, hw, momentum, eps, relu, stream);
+  const int held = small_launch(x, gamma, beta, running_mean, running_var, y, save_mean,
+                                save_invstd, n, c, hw, momentum, eps, relu, stream);
+  if (held >= 0) return held;
   const int fused = bn_fused_launch(x, gamma, beta, running_mean, running_var, y,
                                     save_mean, save_invstd, n, c, hw, momentum,
                                     eps, relu, workspace, stream);
   if (fused >= 0) return fused;
 
-  const bool vec = hw % 4 == 0 && aligned16(x) && aligned16(y);
-
   HIPO_REQUIRE(c <= 65535, "batchnorm: too many channels");
   const int64_t S = num_splits(n, c);
-  const dim3 grid(static_cast<unsigned>(S), static_cast<unsigned>(c));
+  const PlaneGeom g = plane_geom(hw);
+  const bool vec = hw >= 4 && hw < (int64_t{1} << 30) &&
+                   (n + S - 1) / S * g.F < (int64_t{1} << 30);
+  const dim3 grid(static_cast<unsigned>(S * c));
+  const DivMagic by_S = div_magic(static_cast<uint32_t>(S));
   float* ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + kBnCtlBytes +
                                        bn_fused_slot_bytes(n, c, hw));
-  if (vec) {
-    bn_partial_stats<true><<<grid, dim3(kThreads), 0, stream>>>(x, ws, n, c, hw, S);
-  } else {
-    bn_partial_stats<false><<<grid, dim3(kThreads), 0, stream>>>(x, ws, n, c, hw, S);
-  }
+  auto stats = vec ? bn_partial_stats<true> : bn_partial_stats<false>;
+  stats<<<grid, dim3(kThreads), 0, stream>>>(x, ws, n, c, g, S, by_S);
   int rc = check_launch("batchnorm_train_fwd_f32 (stats)");
   if (rc) return rc;
-  if (vec) {
-    bn_normalize<true><<<grid, dim3(kThreads), 0, stream>>>(
-        x, gamma, beta, running_mean, running_var, y, save_mean, save_invstd,
-        ws, n, c, hw, S, momentum, eps, relu);
-  } else {
-    bn_normalize<false><<<grid, dim3(kThreads), 0, stream>>>(
-        x, gamma, beta, running_mean, running_var, y, save_mean, save_invstd,
-        ws, n, c, hw, S, momentum, eps, relu);
-  }
+  auto normalize = vec ? bn_normalize<true> : bn_normalize<false>;
+  normalize<<<grid, dim3(kThreads), 0, stream>>>(x, gamma, beta, running_mean, running_var, y,
+                                                 save_mean, save_invstd, ws, n, c, g, S, by_S,
+                                                 momentum, eps, relu);
   return check_launch("batchnorm_train_fwd_f32 (normalize)");
 }
 

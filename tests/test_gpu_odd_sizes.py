@@ -149,3 +149,40 @@ def test_transpose_any_matrix(r, c, dtype, rocm_device):
         torch.cuda.synchronize()
         out.check(f"[{r}, {c}]")
         assert torch.equal(out.t.cpu(), x.transpose(1, 2).contiguous()), f"[{r}, {c}]"
+
+
+# (n, c, hw): planes of whole float4s and not, value by value (below 9), one
+# vector a thread and many, the 1024-thread kernel from 16385 values on (both
+# kinds, its largest), split-K past it, with one plane and with many.
+BN_TRAIN = [(3, 5, 7), (3, 5, 9), (4, 5, 12), (26, 9, 49), (334, 3, 49), (335, 3, 49), (128, 40, 196),
+            (146, 33, 196), (147, 33, 196), (1820, 2, 9), (2000, 3, 13), (17, 6, 1295), (5, 3, 9999),
+            (1, 4, 50001), (60, 2, 1023), (9000, 2, 3), (700, 2, 70)]
+
+
+@pytest.mark.parametrize("n,c,hw", BN_TRAIN)
+def test_batchnorm_train_any_plane(n, c, hw, rocm_device):
+    """fp32 statistics of exact two-pass pieces merged by Chan's formula:
+    1e-5 holds with a margin of over ten."""
+    import hip_oracles
+    import oracle as ref
+    torch.manual_seed(n + c + hw)
+    x = torch.randn(n, c, 1, hw) * 2 + 0.5
+    gamma, beta = torch.randn(c), torch.randn(c)
+    for shift, relu in ((0, True), (1, False)):
+        rm, rv = torch.randn(c), torch.rand(c) + 0.5
+        want = ref.batchnorm_train(x, gamma, beta, rm.clone(), rv.clone(), momentum=0.1, eps=1e-5,
+                                   relu=relu)
+        xd = place(x, rocm_device, shift)
+        y = Guarded(x.shape, torch.float32, rocm_device, shift)
+        side = [t.to(rocm_device) for t in (gamma, beta, rm, rv)]
+        mean, invstd = (torch.empty(c, device=rocm_device) for _ in range(2))
+        need = hip_oracles.batchnorm_workspace_bytes(n, c, hw)
+        ws = torch.zeros(need, dtype=torch.uint8, device=rocm_device)
+        ok(lib().hipo_batchnorm_train_fwd_f32(
+            xd.data_ptr(), *(t.data_ptr() for t in side), y.t.data_ptr(), mean.data_ptr(),
+            invstd.data_ptr(), n, c, hw, 0.1, 1e-5, int(relu), ws.data_ptr(), need, None))
+        torch.cuda.synchronize()
+        y.check(f"[{n}, {c}, {hw}]")
+        got = (y.t, mean, invstd, side[2], side[3])
+        for name, a, b in zip(("y", "mean", "invstd", "running_mean", "running_var"), got, want):
+            close(a, b, 1e-5, 1e-5, f"[{n}, {c}, {hw}] shift {shift} {name}")
