@@ -65,7 +65,7 @@ __device__ __forceinline__ int64_t row_group_col(int u, int waves_per_row,
          kRowGroup;
 }
 
-// Valid values in wave w's groups of a row of `cols` (cols % 8 == 0).
+// Values of a row of `cols` that wave w's groups own.
 __device__ __forceinline__ int row_wave_count(int U, int waves_per_row,
                                               const RowPlace& p, int64_t cols) {
   int n = 0;
@@ -194,7 +194,7 @@ inline int short_row_lanes(int64_t cols) {
 }
 
 // Host side: waves per row, groups per lane, rows per workgroup for a row of
-// `cols` bf16 values (cols % 8 == 0).  Groups per lane are rounded up to a
+// `cols` bf16 values.  Groups per lane are rounded up to a
 // power of two (the kernels are instantiated for 1, 2, 4, 8); returns false
 // if the row does not fit in registers (cols > 8 waves x 8 groups x 512).
 struct RowPlan {
@@ -236,6 +236,21 @@ struct RowPlan {
       LAUNCH(4, 0);                                                \
     } else {                                                       \
       LAUNCH(8, 0);                                                \
+    }                                                              \
+  } while (0)
+
+// Launch LAUNCH(U) for a row plan, waves per row from the arguments.
+#define HIPO_ROW_DISPATCH_U(plan, LAUNCH)                          \
+  do {                                                             \
+    const int u_ = (plan).groups;                                  \
+    if (u_ == 1) {                                                 \
+      LAUNCH(1);                                                   \
+    } else if (u_ == 2) {                                          \
+      LAUNCH(2);                                                   \
+    } else if (u_ == 4) {                                          \
+      LAUNCH(4);                                                   \
+    } else {                                                       \
+      LAUNCH(8);                                                   \
     }                                                              \
   } while (0)
 

@@ -2,6 +2,12 @@
 //   residual-add LayerNorm  (outputs h, y, mean, rstd)
 //   RMSNorm                 (outputs y, rstd)
 //
+// Rows that are not whole 16-byte groups, or not 16-byte aligned, take the
+// same kernels with element-aligned groups (row_layout.h, RaggedGroup), where
+// one wave per row read it three times value by value before: graph replays,
+// LayerNorm [25216, 769] 68.4 -> 31.2 us, [54972, 180] 29.3 -> 15.7, [14,
+// 4796] 31.8 -> 3.5; RMSNorm [2447, 3126] 39.9 -> 9.5, [60, 7842] 50.5 -> 3.4.
+//
 // Layout (row_layout.h): W waves per row, the row held in registers between
 // its statistics and its output, non-temporal 16-byte streaming accesses,
 // gamma / beta re-read by every row from cache.
@@ -24,7 +30,8 @@
 namespace hipo {
 namespace {
 
-template <int U, int WT>
+// RAGGED: rows of any length >= 8 and any alignment (row_layout.h).
+template <int U, int WT, bool RAGGED>
 __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
     const uint16_t* __restrict__ gamma, const uint16_t* __restrict__ beta,
@@ -38,11 +45,18 @@ __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
   const int64_t base = p.row * cols;
 
   u32x4_t hv[U], rv[U];
+  RaggedGroup rg[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t col = row_group_col(u, waves_per_row, p);
-    hv[u] = row_load_stream(x + base, col, cols);
-    rv[u] = row_load_stream(res + base, col, cols);
+    if constexpr (RAGGED) {
+      rg[u] = ragged_group(col, cols);
+      hv[u] = ragged_load_stream(x + base + rg[u].col);
+      rv[u] = ragged_load_stream(res + base + rg[u].col);
+    } else {
+      hv[u] = row_load_stream(x + base, col, cols);
+      rv[u] = row_load_stream(res + base, col, cols);
+    }
   }
 
   // h = bf16(x + residual); statistics use the bf16-rounded h.  Groups past
@@ -54,10 +68,20 @@ __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
     for (int d = 0; d < 4; ++d) {
       hv[u][d] = pack_bf16x2(bf16lo(hv[u][d]) + bf16lo(rv[u][d]),
                              bf16hi(hv[u][d]) + bf16hi(rv[u][d]));
-      sum += bf16lo(hv[u][d]) + bf16hi(hv[u][d]);
+      if constexpr (RAGGED) {
+        sum += rg[u].skip <= 2 * d ? bf16lo(hv[u][d]) : 0.f;
+        sum += rg[u].skip <= 2 * d + 1 ? bf16hi(hv[u][d]) : 0.f;
+      } else {
+        sum += bf16lo(hv[u][d]) + bf16hi(hv[u][d]);
+      }
     }
     const int64_t col = row_group_col(u, waves_per_row, p);
-    if (h != nullptr && p.valid && col < cols) row_store_stream(h + base, col, hv[u]);
+    if constexpr (RAGGED) {
+      if (h != nullptr && p.valid && rg[u].skip < kRowGroup)
+        ragged_store(h + base + rg[u].col, hv[u]);
+    } else {
+      if (h != nullptr && p.valid && col < cols) row_store_stream(h + base, col, hv[u]);
+    }
   }
   const float n = static_cast<float>(row_wave_count(U, waves_per_row, p, cols));
   const float wmean = n > 0.f ? wave_sum(sum) / n : 0.f;
@@ -67,8 +91,10 @@ __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
     const bool in = row_group_col(u, waves_per_row, p) < cols;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      const float a = in ? bf16lo(hv[u][d]) - wmean : 0.f;
-      const float b = in ? bf16hi(hv[u][d]) - wmean : 0.f;
+      const bool lo = RAGGED ? rg[u].skip <= 2 * d : in;
+      const bool hi = RAGGED ? rg[u].skip <= 2 * d + 1 : in;
+      const float a = lo ? bf16lo(hv[u][d]) - wmean : 0.f;
+      const float b = hi ? bf16hi(hv[u][d]) - wmean : 0.f;
       sq = __builtin_fmaf(a, a, sq);
       sq = __builtin_fmaf(b, b, sq);
     }
@@ -101,8 +127,10 @@ __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t col = row_group_col(u, waves_per_row, p);
-    const u32x4_t gv = row_load_cached(gamma, col, cols);
-    const u32x4_t bv = row_load_cached(beta, col, cols);
+    const u32x4_t gv =
+        RAGGED ? ragged_load_cached(gamma + rg[u].col) : row_load_cached(gamma, col, cols);
+    const u32x4_t bv =
+        RAGGED ? ragged_load_cached(beta + rg[u].col) : row_load_cached(beta, col, cols);
     u32x4_t o;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
@@ -111,7 +139,11 @@ __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
       o[d] = pack_bf16x2(__builtin_fmaf(n0, bf16lo(gv[d]), bf16lo(bv[d])),
                          __builtin_fmaf(n1, bf16hi(gv[d]), bf16hi(bv[d])));
     }
-    if (p.valid && col < cols) row_store_stream(y + base, col, o);
+    if constexpr (RAGGED) {
+      if (p.valid && rg[u].skip < kRowGroup) ragged_store(y + base + rg[u].col, o);
+    } else {
+      if (p.valid && col < cols) row_store_stream(y + base, col, o);
+    }
   }
   if (p.valid && p.w == 0 && p.lane == 0) {
     if (mean_out != nullptr) mean_out[p.row] = mean;
@@ -122,8 +154,32 @@ __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
 // MODE 0 (torch rms_norm): y = bf16(h * rstd * gamma * scale), one rounding.
 // MODE 1 (HF T5 op order): t = bf16(h * rstd); u = bf16(gamma * t);
 //                          y = scale == 1 ? u : bf16(u * scale).
+template <int MODE, bool SCALED>
+__device__ __forceinline__ u32x4_t rms_apply(u32x4_t h, u32x4_t gv, float rstd, float scale) {
+  u32x4_t o;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    float a = bf16lo(h[d]) * rstd, b = bf16hi(h[d]) * rstd;
+    if constexpr (MODE == 0) {
+      a *= bf16lo(gv[d]);
+      b *= bf16hi(gv[d]);
+      if constexpr (SCALED) {
+        a *= scale;
+        b *= scale;
+      }
+      o[d] = pack_bf16x2(a, b);
+    } else {
+      const uint32_t t = pack_bf16x2(a, b);
+      uint32_t w = pack_bf16x2(bf16lo(gv[d]) * bf16lo(t), bf16hi(gv[d]) * bf16hi(t));
+      if constexpr (SCALED) w = pack_bf16x2(bf16lo(w) * scale, bf16hi(w) * scale);
+      o[d] = w;
+    }
+  }
+  return o;
+}
+
 // With a residual, h = bf16(x + residual) (the eager bf16 add), else h = x.
-template <int U, int WT, bool RES, int MODE>
+template <int U, int WT, bool RES, int MODE, bool RAGGED>
 __global__ __launch_bounds__(kRowMaxThreads) void rmsnorm_rows(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
     const uint16_t* __restrict__ gamma, uint16_t* __restrict__ h, uint16_t* __restrict__ y,
@@ -136,20 +192,34 @@ __global__ __launch_bounds__(kRowMaxThreads) void rmsnorm_rows(
   const int64_t base = p.row * cols;
 
   u32x4_t xv[U];
+  RaggedGroup rg[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u)
-    xv[u] = row_load_stream(x + base, row_group_col(u, waves_per_row, p), cols);
+  for (int u = 0; u < U; ++u) {
+    const int64_t col = row_group_col(u, waves_per_row, p);
+    if constexpr (RAGGED) {
+      rg[u] = ragged_group(col, cols);
+      xv[u] = ragged_load_stream(x + base + rg[u].col);
+    } else {
+      xv[u] = row_load_stream(x + base, col, cols);
+    }
+  }
   if (RES) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const u32x4_t rv =
-          row_load_stream(res + base, row_group_col(u, waves_per_row, p), cols);
+          RAGGED ? ragged_load_stream(res + base + rg[u].col)
+                 : row_load_stream(res + base, row_group_col(u, waves_per_row, p), cols);
 #pragma unroll
       for (int d = 0; d < 4; ++d)
         xv[u][d] = pack_bf16x2(bf16lo(xv[u][d]) + bf16lo(rv[d]),
                                bf16hi(xv[u][d]) + bf16hi(rv[d]));
       const int64_t col = row_group_col(u, waves_per_row, p);
-      if (h != nullptr && p.valid && col < cols) row_store_stream(h + base, col, xv[u]);
+      if constexpr (RAGGED) {
+        if (h != nullptr && p.valid && rg[u].skip < kRowGroup)
+          ragged_store(h + base + rg[u].col, xv[u]);
+      } else {
+        if (h != nullptr && p.valid && col < cols) row_store_stream(h + base, col, xv[u]);
+      }
     }
   }
   float sq = 0.f;
@@ -157,8 +227,8 @@ __global__ __launch_bounds__(kRowMaxThreads) void rmsnorm_rows(
   for (int u = 0; u < U; ++u) {
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      const float a = bf16lo(xv[u][d]);
-      const float b = bf16hi(xv[u][d]);
+      const float a = !RAGGED || rg[u].skip <= 2 * d ? bf16lo(xv[u][d]) : 0.f;
+      const float b = !RAGGED || rg[u].skip <= 2 * d + 1 ? bf16hi(xv[u][d]) : 0.f;
       sq = __builtin_fmaf(a, a, sq);
       sq = __builtin_fmaf(b, b, sq);
     }
@@ -176,31 +246,17 @@ __global__ __launch_bounds__(kRowMaxThreads) void rmsnorm_rows(
   // The scale test is hoisted out of the per-element loop (one uniform
   // branch, two copies of the store loop).
   auto store = [&](auto scaled) {
-    constexpr bool kScaled = decltype(scaled)::value;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t col = row_group_col(u, waves_per_row, p);
-      const u32x4_t gv = row_load_cached(gamma, col, cols);
-      u32x4_t o;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        float a = bf16lo(xv[u][d]) * rstd, b = bf16hi(xv[u][d]) * rstd;
-        if constexpr (MODE == 0) {
-          a *= bf16lo(gv[d]);
-          b *= bf16hi(gv[d]);
-          if constexpr (kScaled) {
-            a *= scale;
-            b *= scale;
-          }
-          o[d] = pack_bf16x2(a, b);
-        } else {
-          const uint32_t t = pack_bf16x2(a, b);
-          uint32_t w = pack_bf16x2(bf16lo(gv[d]) * bf16lo(t), bf16hi(gv[d]) * bf16hi(t));
-          if constexpr (kScaled) w = pack_bf16x2(bf16lo(w) * scale, bf16hi(w) * scale);
-          o[d] = w;
-        }
+      const u32x4_t gv =
+          RAGGED ? ragged_load_cached(gamma + rg[u].col) : row_load_cached(gamma, col, cols);
+      const u32x4_t o = rms_apply<MODE, decltype(scaled)::value>(xv[u], gv, rstd, scale);
+      if constexpr (RAGGED) {
+        if (p.valid && rg[u].skip < kRowGroup) ragged_store(y + base + rg[u].col, o);
+      } else {
+        if (p.valid && col < cols) row_store_stream(y + base, col, o);
       }
-      if (p.valid && col < cols) row_store_stream(y + base, col, o);
     }
   };
   if (scale != 1.0f) {
@@ -437,7 +493,8 @@ __global__ __launch_bounds__(W * NR * 64) void residual_layernorm_k(
 // DPP-and-readlane sums: 19.7, 19.9), and at 2048 values one wave per row
 // with 4 groups lost to the row kernel's two waves with 2 (20.4 against
 // 19.2 us).
-template <int L, int U>
+// RAGGED: rows of any length >= 8 and any alignment (row_layout.h).
+template <int L, int U, bool RAGGED>
 __global__ __launch_bounds__(256) void residual_layernorm_seg(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
     const uint16_t* __restrict__ gamma, const uint16_t* __restrict__ beta,
@@ -448,24 +505,45 @@ __global__ __launch_bounds__(256) void residual_layernorm_seg(
   const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + threadIdx.x / L;
   const bool valid = row < rows;
   const int64_t base = (valid ? row : rows - 1) * cols;
-  const int groups = cols / kRowGroup;
+  const int groups = RAGGED ? (cols + kRowGroup - 1) / kRowGroup : cols / kRowGroup;
 
   u32x4_t hv[U], rv[U], gv[U], bv[U];
-  bool in[U];
+  int at[U];    // column of the group held
+  int skip[U];  // its values from `skip` on count (8: none)
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int g = u * L + l;
-    in[u] = g < groups;
-    const int col = (in[u] ? g : groups - 1) * kRowGroup;
-    hv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(x + base + col));
-    rv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(res + base + col));
+    const int first = g * kRowGroup;
+    const int last = RAGGED ? cols - kRowGroup : (groups - 1) * kRowGroup;
+    at[u] = first < last ? first : last;
+    skip[u] = g < groups ? first - at[u] : kRowGroup;
+    if constexpr (RAGGED) {
+      hv[u] = ragged_load_stream(x + base + at[u]);
+      rv[u] = ragged_load_stream(res + base + at[u]);
+    } else {
+      hv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(x + base + at[u]));
+      rv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(res + base + at[u]));
+    }
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int col = (in[u] ? u * L + l : groups - 1) * kRowGroup;
-    gv[u] = *reinterpret_cast<const u32x4_t*>(gamma + col);
-    bv[u] = *reinterpret_cast<const u32x4_t*>(beta + col);
+    if constexpr (RAGGED) {
+      gv[u] = ragged_load_cached(gamma + at[u]);
+      bv[u] = ragged_load_cached(beta + at[u]);
+    } else {
+      gv[u] = *reinterpret_cast<const u32x4_t*>(gamma + at[u]);
+      bv[u] = *reinterpret_cast<const u32x4_t*>(beta + at[u]);
+    }
   }
+  // Whether value e of group u counts; a whole row's groups count or not as one.
+  auto counts = [&](int u, int e) { return RAGGED ? e >= skip[u] : skip[u] == 0; };
+  auto store = [&](uint16_t* row_out, int u, u32x4_t v) {
+    if constexpr (RAGGED) {
+      if (valid && skip[u] < kRowGroup) ragged_store(row_out + at[u], v);
+    } else {
+      if (valid && skip[u] == 0) row_store_stream(row_out, at[u], v);
+    }
+  };
 
   // h = bf16(x + residual); the statistics use the bf16-rounded h.
   float sum = 0.f;
@@ -475,10 +553,14 @@ __global__ __launch_bounds__(256) void residual_layernorm_seg(
     for (int d = 0; d < 4; ++d) {
       hv[u][d] = pack_bf16x2(bf16lo(hv[u][d]) + bf16lo(rv[u][d]),
                              bf16hi(hv[u][d]) + bf16hi(rv[u][d]));
-      if (in[u]) sum += bf16lo(hv[u][d]) + bf16hi(hv[u][d]);
+      if constexpr (RAGGED) {
+        sum += (counts(u, 2 * d) ? bf16lo(hv[u][d]) : 0.f) +
+               (counts(u, 2 * d + 1) ? bf16hi(hv[u][d]) : 0.f);
+      } else {
+        if (counts(u, 0)) sum += bf16lo(hv[u][d]) + bf16hi(hv[u][d]);
+      }
     }
-    if (h != nullptr && valid && in[u])
-      row_store_stream(h + base, static_cast<int64_t>(u * L + l) * kRowGroup, hv[u]);
+    if (h != nullptr) store(h + base, u, hv[u]);
   }
   const float inv_n = 1.0f / static_cast<float>(cols);
   const float mean = seg_sum<L>(sum) * inv_n;
@@ -489,7 +571,12 @@ __global__ __launch_bounds__(256) void residual_layernorm_seg(
     for (int d = 0; d < 4; ++d) {
       const float a = bf16lo(hv[u][d]) - mean;
       const float b = bf16hi(hv[u][d]) - mean;
-      if (in[u]) sq = __builtin_fmaf(a, a, __builtin_fmaf(b, b, sq));
+      if constexpr (RAGGED) {
+        if (counts(u, 2 * d)) sq = __builtin_fmaf(a, a, sq);
+        if (counts(u, 2 * d + 1)) sq = __builtin_fmaf(b, b, sq);
+      } else {
+        if (counts(u, 0)) sq = __builtin_fmaf(a, a, __builtin_fmaf(b, b, sq));
+      }
     }
   }
   const float rstd = 1.0f / __builtin_sqrtf(seg_sum<L>(sq) * inv_n + eps);
@@ -504,7 +591,7 @@ __global__ __launch_bounds__(256) void residual_layernorm_seg(
       o[d] = pack_bf16x2(__builtin_fmaf(n0, bf16lo(gv[u][d]), bf16lo(bv[u][d])),
                          __builtin_fmaf(n1, bf16hi(gv[u][d]), bf16hi(bv[u][d])));
     }
-    if (valid && in[u]) row_store_stream(y + base, static_cast<int64_t>(u * L + l) * kRowGroup, o);
+    store(y + base, u, o);
   }
   if (valid && l == 0) {
     if (mean_out != nullptr) mean_out[row] = mean;
@@ -518,8 +605,8 @@ struct SegPlan {
 
 SegPlan seg_plan(int64_t rows, int64_t cols) {
   SegPlan p;
-  if (cols % kRowGroup != 0 || cols <= 0 || cols > 1536) return p;
-  const int g = static_cast<int>(cols / kRowGroup);
+  if (cols < kRowGroup || cols > 1536) return p;
+  const int g = static_cast<int>((cols + kRowGroup - 1) / kRowGroup);
   if (g > kWave && rows < 16384) return p;  // the row kernel's 8-row workgroups win there
   if (g <= kWave) {
     p.lanes = 8;
@@ -532,22 +619,23 @@ SegPlan seg_plan(int64_t rows, int64_t cols) {
   return p;
 }
 
-template <int L, int U>
+template <int L, int U, bool RAGGED>
 void launch_seg(int64_t rows, hipStream_t stream, const uint16_t* x, const uint16_t* residual,
                 const uint16_t* gamma, const uint16_t* beta, uint16_t* h, uint16_t* y,
                 float* mean, float* rstd, int cols, float eps) {
   constexpr int kRowsPerBlock = 256 / L;
-  residual_layernorm_seg<L, U>
+  residual_layernorm_seg<L, U, RAGGED>
       <<<dim3(static_cast<unsigned>((rows + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(256), 0,
          stream>>>(x, residual, gamma, beta, h, y, mean, rstd, rows, cols, eps);
 }
 
 // Dispatch over the (L, U) pairs seg_plan returns.
+template <bool RAGGED>
 void launch_seg_plan(const SegPlan& sp, int64_t rows, hipStream_t stream, const uint16_t* x,
                      const uint16_t* residual, const uint16_t* gamma, const uint16_t* beta,
                      uint16_t* h, uint16_t* y, float* mean, float* rstd, int cols, float eps) {
 #define HIPO_SEG(L_, U_) \
-  launch_seg<L_, U_>(rows, stream, x, residual, gamma, beta, h, y, mean, rstd, cols, eps)
+  launch_seg<L_, U_, RAGGED>(rows, stream, x, residual, gamma, beta, h, y, mean, rstd, cols, eps)
   if (sp.groups == 1) {
     switch (sp.lanes) {
       case 8: HIPO_SEG(8, 1); break;
@@ -589,31 +677,44 @@ extern "C" int hipo_residual_layernorm_bf16(
   HIPO_REQUIRE(cols > 0, "residual_layernorm: cols must be > 0");
   HIPO_REQUIRE(x && residual && gamma && beta && y,
                "residual_layernorm: null pointer");
+  // Rows of 8 to 32768 values are held in registers: the aligned kernels for
+  // whole 16-byte groups at 16-byte alignment, their ragged forms otherwise.
   RowPlan plan;
-  const bool vec = cols % 8 == 0 && row_plan(cols, plan) && aligned16(x) &&
-                   aligned16(residual) && aligned16(gamma) && aligned16(beta) &&
-                   (h == nullptr || aligned16(h)) && aligned16(y);
+  const bool held = cols >= kRowGroup && row_plan(cols, plan);
+  const bool vec = held && cols % 8 == 0 && aligned16(x) && aligned16(residual) &&
+                   aligned16(gamma) && aligned16(beta) && (h == nullptr || aligned16(h)) &&
+                   aligned16(y);
   constexpr int kRowsPerBlock = kLnSlots * kLayerNormRowsPerWave;
   if (vec && cols == 4096 && (rows + kRowsPerBlock - 1) / kRowsPerBlock <= 0x7fffffff) {
     residual_layernorm_k<4096, kLnWaves, kLnSlots, kLayerNormRowsPerWave, kLnStage>
         <<<dim3(static_cast<unsigned>((rows + kRowsPerBlock - 1) / kRowsPerBlock)),
            dim3(kLnWaves * kLnSlots * kWave), 0, stream>>>(x, residual, gamma, beta, h, y, mean,
                                                            rstd, rows, eps);
-  } else if (const SegPlan sp = vec ? seg_plan(rows, cols) : SegPlan{};
+  } else if (const SegPlan sp = held ? seg_plan(rows, cols) : SegPlan{};
              sp.lanes > 0 && (rows + 256 / sp.lanes - 1) / (256 / sp.lanes) <= 0x7fffffff) {
-    launch_seg_plan(sp, rows, stream, x, residual, gamma, beta, h, y, mean, rstd,
-                    static_cast<int>(cols), eps);
-  } else if (vec) {
+    auto launch = vec ? launch_seg_plan<false> : launch_seg_plan<true>;
+    launch(sp, rows, stream, x, residual, gamma, beta, h, y, mean, rstd, static_cast<int>(cols),
+           eps);
+  } else if (held) {
     const int64_t blocks = (rows + plan.rows_per_block - 1) / plan.rows_per_block;
     HIPO_REQUIRE(blocks <= 0x7fffffff, "residual_layernorm: too many rows");
     const dim3 grid(static_cast<unsigned>(blocks));
     const dim3 block(plan.threads());
-#define HIPO_LN(U_, W_)                                                              \
-  residual_layernorm_rows<U_, W_><<<grid, block, 0, stream>>>(                       \
+#define HIPO_LN(U_, W_)                                                                \
+  residual_layernorm_rows<U_, W_, false><<<grid, block, 0, stream>>>(                  \
       x, residual, gamma, beta, h, y, mean, rstd, rows, cols, eps, plan.waves_per_row, \
       plan.rows_per_block)
-    HIPO_ROW_DISPATCH(plan, HIPO_LN);
+#define HIPO_LN_RAGGED(U_)                                                             \
+  residual_layernorm_rows<U_, 0, true><<<grid, block, 0, stream>>>(                    \
+      x, residual, gamma, beta, h, y, mean, rstd, rows, cols, eps, plan.waves_per_row, \
+      plan.rows_per_block)
+    if (vec) {
+      HIPO_ROW_DISPATCH(plan, HIPO_LN);
+    } else {
+      HIPO_ROW_DISPATCH_U(plan, HIPO_LN_RAGGED);
+    }
 #undef HIPO_LN
+#undef HIPO_LN_RAGGED
   } else {
     const int64_t blocks = (rows + 3) / 4;
     HIPO_REQUIRE(blocks <= 0x7fffffff, "residual_layernorm: too many rows");
@@ -626,18 +727,101 @@ extern "C" int hipo_residual_layernorm_bf16(
 namespace hipo {
 namespace {
 
+// Rows of at most 512 values (head norms: 64, 128): a row owns L = 8..64
+// lanes, one 16-byte group each, so a load instruction of a wave covers 64 / L
+// rows, where the row kernel leaves the lanes past a row's end idle.  Same
+// arithmetic, the sum of squares over the row's lanes by seg_sum.  Graph
+// replays, the row kernel -> here (two rows, four rows per lane): [16000,
+// 128] 5.6 -> 3.3 us (3.4, 3.6), [131072, 128] 32.9 -> 12.5 (13.6, 13.0),
+// [65536, 64] with residual and h 20.2 -> 7.3 (7.2, 6.9), [32768, 256] 11.0 ->
+// 7.6 (7.5, 7.4), [1000, 128] 2.27 -> 2.06 (2.32, 2.89), [32768, 512] with a
+// residual 18.7 -> 17.4 (18.4, 18.6).
+constexpr int kSegThreads = 256;
+
+template <int L, bool RES, int MODE, bool RAGGED>
+__global__ __launch_bounds__(kSegThreads) void rmsnorm_seg(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
+    const uint16_t* __restrict__ gamma, uint16_t* __restrict__ h, uint16_t* __restrict__ y,
+    float* __restrict__ rstd_out, int64_t rows, int cols, float eps, float scale) {
+  const int l = static_cast<int>(threadIdx.x) & (L - 1);
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * (kSegThreads / L) + threadIdx.x / L;
+  const int first = l * kRowGroup;
+  const int at = first < cols - kRowGroup ? first : cols - kRowGroup;
+  const int skip = first - at;  // >= 8: no group of the row
+  const bool own = row < rows && skip < kRowGroup;
+  const int64_t off = (row < rows ? row : rows - 1) * cols + at;
+  auto load = [&](const uint16_t* p) {
+    if constexpr (RAGGED) return ragged_load_stream(p + off);
+    else return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p + off));
+  };
+  auto store = [&](uint16_t* p, u32x4_t v) {
+    if (!own) return;
+    if constexpr (RAGGED) ragged_store(p + off, v);
+    else row_store_stream(p, off, v);
+  };
+  u32x4_t hv = load(x);
+  if constexpr (RES) {
+    const u32x4_t rv = load(res);
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      hv[d] = pack_bf16x2(bf16lo(hv[d]) + bf16lo(rv[d]), bf16hi(hv[d]) + bf16hi(rv[d]));
+    if (h != nullptr) store(h, hv);
+  }
+  const u32x4_t gv = RAGGED ? ragged_load_cached(gamma + at)
+                            : *reinterpret_cast<const u32x4_t*>(gamma + at);
+  float sq = 0.f;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const float a = skip <= (RAGGED ? 2 * d : 0) ? bf16lo(hv[d]) : 0.f;
+    const float b = skip <= (RAGGED ? 2 * d + 1 : 0) ? bf16hi(hv[d]) : 0.f;
+    sq = __builtin_fmaf(a, a, sq);
+    sq = __builtin_fmaf(b, b, sq);
+  }
+  const float rstd = 1.0f / __builtin_sqrtf(seg_sum<L>(sq) / static_cast<float>(cols) + eps);
+  store(y, scale != 1.0f ? rms_apply<MODE, true>(hv, gv, rstd, scale)
+                         : rms_apply<MODE, false>(hv, gv, rstd, scale));
+  if (rstd_out != nullptr && row < rows && l == 0) rstd_out[row] = rstd;
+}
+
+template <bool RES, int MODE, bool RAGGED>
+void launch_rmsnorm_seg(int lanes, hipStream_t stream, const uint16_t* x,
+                        const uint16_t* residual, const uint16_t* gamma, uint16_t* h,
+                        uint16_t* y, float* rstd, int64_t rows, int cols, float eps,
+                        float scale) {
+  const int64_t per_block = kSegThreads / lanes;
+  const dim3 grid(static_cast<unsigned>((rows + per_block - 1) / per_block));
+#define HIPO_RMS_SEG(L_)                                                      \
+  rmsnorm_seg<L_, RES, MODE, RAGGED><<<grid, dim3(kSegThreads), 0, stream>>>( \
+      x, residual, gamma, h, y, rstd, rows, cols, eps, scale)
+  switch (lanes) {
+    case 8: HIPO_RMS_SEG(8); break;
+    case 16: HIPO_RMS_SEG(16); break;
+    case 32: HIPO_RMS_SEG(32); break;
+    default: HIPO_RMS_SEG(64); break;
+  }
+#undef HIPO_RMS_SEG
+}
+
 template <bool RES, int MODE>
-void launch_rmsnorm(const RowPlan& plan, dim3 grid, hipStream_t stream,
+void launch_rmsnorm(const RowPlan& plan, bool vec, dim3 grid, hipStream_t stream,
                     const uint16_t* x, const uint16_t* residual,
                     const uint16_t* gamma, uint16_t* h, uint16_t* y, float* rstd,
                     int64_t rows, int64_t cols, float eps, float scale) {
   const dim3 block(plan.threads());
   const int w = plan.waves_per_row, r = plan.rows_per_block;
-#define HIPO_RMS(U_, W_)                                            \
-  rmsnorm_rows<U_, W_, RES, MODE><<<grid, block, 0, stream>>>(      \
+#define HIPO_RMS(U_, W_)                                               \
+  rmsnorm_rows<U_, W_, RES, MODE, false><<<grid, block, 0, stream>>>(  \
       x, residual, gamma, h, y, rstd, rows, cols, eps, scale, w, r)
-  HIPO_ROW_DISPATCH(plan, HIPO_RMS);
+#define HIPO_RMS_RAGGED(U_)                                            \
+  rmsnorm_rows<U_, 0, RES, MODE, true><<<grid, block, 0, stream>>>(    \
+      x, residual, gamma, h, y, rstd, rows, cols, eps, scale, w, r)
+  if (vec) {
+    HIPO_ROW_DISPATCH(plan, HIPO_RMS);
+  } else {
+    HIPO_ROW_DISPATCH_U(plan, HIPO_RMS_RAGGED);
+  }
 #undef HIPO_RMS
+#undef HIPO_RMS_RAGGED
 }
 
 int rmsnorm_impl(const uint16_t* x, const uint16_t* residual, const uint16_t* gamma,
@@ -651,20 +835,40 @@ int rmsnorm_impl(const uint16_t* x, const uint16_t* residual, const uint16_t* ga
   HIPO_REQUIRE(x && gamma && y && (rstd || !require_rstd), "%s: null pointer", what);
   HIPO_REQUIRE(h == nullptr || residual != nullptr, "%s: h needs a residual", what);
   HIPO_REQUIRE(mode == 0 || mode == 1, "%s: mode must be 0 or 1", what);
+  // As for the LayerNorm: registers for 8 to 32768 values, ragged forms for
+  // rows that are not whole 16-byte groups or not 16-byte aligned.
   RowPlan plan;
-  const bool vec = cols % 8 == 0 && row_plan(cols, plan) && aligned16(x) &&
-                   aligned16(gamma) && aligned16(y) &&
+  const bool held = cols >= kRowGroup && row_plan(cols, plan);
+  const bool vec = held && cols % 8 == 0 && aligned16(x) && aligned16(gamma) && aligned16(y) &&
                    (residual == nullptr || aligned16(residual)) && (h == nullptr || aligned16(h));
-  if (vec) {
+  const int lanes = std::max(8, short_row_lanes(cols));
+  const int64_t seg_rows = kSegThreads / lanes;
+  if (held && cols <= kRowSweep && (rows + seg_rows - 1) / seg_rows <= 0x7fffffff) {
+    const int c = static_cast<int>(cols);
+#define HIPO_RMS_SEG_CALL(RES_, MODE_)                                                         \
+  do {                                                                                         \
+    auto launch = vec ? launch_rmsnorm_seg<RES_, MODE_, false>                                 \
+                      : launch_rmsnorm_seg<RES_, MODE_, true>;                                 \
+    launch(lanes, stream, x, residual, gamma, h, y, rstd, rows, c, eps, scale);                \
+  } while (0)
+    if (residual != nullptr) {
+      if (mode == 0) HIPO_RMS_SEG_CALL(true, 0);
+      else HIPO_RMS_SEG_CALL(true, 1);
+    } else {
+      if (mode == 0) HIPO_RMS_SEG_CALL(false, 0);
+      else HIPO_RMS_SEG_CALL(false, 1);
+    }
+#undef HIPO_RMS_SEG_CALL
+  } else if (held) {
     const int64_t blocks = (rows + plan.rows_per_block - 1) / plan.rows_per_block;
     HIPO_REQUIRE(blocks <= 0x7fffffff, "%s: too many rows", what);
     const dim3 grid(static_cast<unsigned>(blocks));
     if (residual != nullptr) {
-      if (mode == 0) launch_rmsnorm<true, 0>(plan, grid, stream, x, residual, gamma, h, y, rstd, rows, cols, eps, scale);
-      else launch_rmsnorm<true, 1>(plan, grid, stream, x, residual, gamma, h, y, rstd, rows, cols, eps, scale);
+      if (mode == 0) launch_rmsnorm<true, 0>(plan, vec, grid, stream, x, residual, gamma, h, y, rstd, rows, cols, eps, scale);
+      else launch_rmsnorm<true, 1>(plan, vec, grid, stream, x, residual, gamma, h, y, rstd, rows, cols, eps, scale);
     } else {
-      if (mode == 0) launch_rmsnorm<false, 0>(plan, grid, stream, x, residual, gamma, nullptr, y, rstd, rows, cols, eps, scale);
-      else launch_rmsnorm<false, 1>(plan, grid, stream, x, residual, gamma, nullptr, y, rstd, rows, cols, eps, scale);
+      if (mode == 0) launch_rmsnorm<false, 0>(plan, vec, grid, stream, x, residual, gamma, nullptr, y, rstd, rows, cols, eps, scale);
+      else launch_rmsnorm<false, 1>(plan, vec, grid, stream, x, residual, gamma, nullptr, y, rstd, rows, cols, eps, scale);
     }
   } else {
     const int64_t blocks = (rows + 3) / 4;

@@ -186,3 +186,54 @@ def test_batchnorm_train_any_plane(n, c, hw, rocm_device):
         got = (y.t, mean, invstd, side[2], side[3])
         for name, a, b in zip(("y", "mean", "invstd", "running_mean", "running_var"), got, want):
             close(a, b, 1e-5, 1e-5, f"[{n}, {c}, {hw}] shift {shift} {name}")
+
+
+# One group, one value more and less; the ends of the lane counts and of the
+# short-row kernels (512, 1536); several waves and groups per row; value by
+# value (below 8).
+NORM_COLS = [7, 8, 9, 63, 64, 65, 100, 128, 180, 257, 511, 512, 513, 769, 1025, 1535, 2530, 4096,
+             4796, 7842, 16385]
+
+
+@pytest.mark.parametrize("cols", NORM_COLS)
+def test_norms_any_row_length(cols, rocm_device):
+    """Statistics 1e-5; bf16 results within 2^-7 (two ulps where kernel and
+    oracle round to different sides twice), 1e-2 near zero for LayerNorm,
+    whose terms cancel there."""
+    import oracle as ref
+    torch.manual_seed(cols)
+    L = lib()
+    for rows in ((3, 16400) if cols in (513, 769, 1535) else (1, 37)):
+        x, r = (torch.randn(rows, cols).to(torch.bfloat16) for _ in range(2))
+        g, b = (1 + 0.1 * torch.randn(cols)).to(torch.bfloat16), torch.randn(cols).to(torch.bfloat16)
+        hw, yw, mw, sw = ref.residual_layernorm(x, r, g, b, 1e-5)
+        for shift in (0, 1):
+            what = f"[{rows}, {cols}] shift {shift}"
+            xd, rd, gd, bd = (place(t, rocm_device, shift) for t in (x, r, g, b))
+            h, y = (Guarded((rows, cols), torch.bfloat16, rocm_device, shift) for _ in range(2))
+            mean, rstd = (Guarded((rows,), torch.float32, rocm_device) for _ in range(2))
+            ok(L.hipo_residual_layernorm_bf16(
+                xd.data_ptr(), rd.data_ptr(), gd.data_ptr(), bd.data_ptr(), h.t.data_ptr(),
+                y.t.data_ptr(), mean.t.data_ptr(), rstd.t.data_ptr(), rows, cols, 1e-5, None))
+            torch.cuda.synchronize()
+            for o in (h, y, mean, rstd):
+                o.check("layernorm " + what)
+            assert torch.equal(h.t.cpu(), hw), what
+            close(y.t, yw, 2 ** -7, 1e-2, "layernorm y " + what)
+            close(mean.t, mw, 1e-5, 1e-5, "mean " + what)
+            close(rstd.t, sw, 1e-5, 1e-5, "rstd " + what)
+            for mode, scale, res in ((0, 1.0, None), (1, 0.125, rd), (0, 0.5, rd), (1, 1.0, None)):
+                want = ref.rmsnorm_ex(x, g, 1e-6, residual=None if res is None else r,
+                                      scale=scale, mode=mode)
+                h, y = (Guarded((rows, cols), torch.bfloat16, rocm_device, shift)
+                        for _ in range(2))
+                ok(L.hipo_rmsnorm_ex_bf16(
+                    xd.data_ptr(), None if res is None else res.data_ptr(), gd.data_ptr(),
+                    None if res is None else h.t.data_ptr(), y.t.data_ptr(), rstd.t.data_ptr(),
+                    rows, cols, 1e-6, scale, mode, None))
+                torch.cuda.synchronize()
+                for o in (h, y, rstd):
+                    o.check(f"rmsnorm mode {mode} " + what)
+                if res is not None:
+                    assert torch.equal(h.t.cpu(), hw), what
+                close(y.t, want[0], 2 ** -6 if mode else 2 ** -7, 1e-6, f"rmsnorm {mode} " + what)
