@@ -136,19 +136,40 @@ def _require(cond: bool, msg: str) -> None:
         raise ValueError(msg)
 
 
+_IS_ROCM = torch.version.hip is not None
+
+
 def _require_rocm(*tensors: torch.Tensor) -> torch.device:
     dev = tensors[0].device
     for t in tensors:
-        _require(isinstance(t, torch.Tensor), "expected tensors")
-        _require(t.device.type == "cuda",
-                 f"hip_oracles runs on the ROCm device only, got a {t.device} tensor")
-        _require(t.device == dev, "all operands must be on one device")
-    _require(torch.version.hip is not None, "torch is not a ROCm build")
+        if not isinstance(t, torch.Tensor):
+            raise ValueError("expected tensors")
+        if not t.is_cuda:
+            raise ValueError(f"hip_oracles runs on the ROCm device only, got a {t.device} tensor")
+        if t.device != dev:
+            raise ValueError("all operands must be on one device")
+    _require(_IS_ROCM, "torch is not a ROCm build")
     return dev
 
 
-def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+# The current device's index and a device's current stream as plain integers,
+# without the torch.cuda.device context and the torch.cuda.Stream object that
+# cost a call 1.2 and 1.8 us of its host time (row_mean at [300, 1000] 9.3 ->
+# 5.6 us a call, of which the launch is 2.9).
+_current_device = torch._C._cuda_getDevice if torch.cuda._is_compiled() else None
+_raw_stream = torch._C._cuda_getCurrentRawStream if torch.cuda._is_compiled() else None
+
+
+def _call(fn, what: str, dev: torch.device, *args) -> None:
+    """fn(*args, stream) on dev's current stream, with dev current."""
+    index = dev.index
+    if index == _current_device():
+        rc = fn(*args, _raw_stream(index))
+    else:
+        with torch.cuda.device(dev):
+            rc = fn(*args, _raw_stream(index))
+    if rc != 0:
+        _check(rc, what)
 
 
 def _ptr(t: torch.Tensor) -> int:
@@ -161,23 +182,21 @@ def _ptr(t: torch.Tensor) -> int:
 
 def row_mean(x: torch.Tensor) -> torch.Tensor:
     """fp32 mean over the last dim of a 2-D fp32 tensor -> [rows]."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dtype == torch.float32 and x.dim() == 2, "row_mean: x must be 2-D fp32")
     _require(x.stride(1) == 1 or x.shape[1] <= 1, "row_mean: last dim must be contiguous")
     rows, cols = x.shape
     out = torch.empty(rows, dtype=torch.float32, device=dev)
     row_stride = x.stride(0) if rows > 1 else cols
-    with torch.cuda.device(dev):
-        _check(lib.hipo_row_mean_f32(_ptr(x), _ptr(out), rows, cols,
-                                     max(row_stride, cols), _stream(dev)),
-               "row_mean")
+    _call(lib.hipo_row_mean_f32, "row_mean", dev, _ptr(x), _ptr(out), rows, cols,
+          max(row_stride, cols))
     return out
 
 
 def bias_gelu_nchw_to_nhwc(x: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     """gelu_tanh(x + bias[None,:,None,None]) written channels-last (bf16)."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x, bias)
     _require(x.dtype == torch.bfloat16 and bias.dtype == torch.bfloat16,
              "bias_gelu: bf16 operands required")
@@ -186,10 +205,8 @@ def bias_gelu_nchw_to_nhwc(x: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     _require(bias.shape == (c,) and bias.is_contiguous(), "bias_gelu: bias must be [C]")
     out = torch.empty((n, c, h, w), dtype=torch.bfloat16, device=dev,
                       memory_format=torch.channels_last)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_bias_gelu_nchw_to_nhwc_bf16(_ptr(x), _ptr(bias), _ptr(out),
-                                                    n, c, h * w, _stream(dev)),
-               "bias_gelu_nchw_to_nhwc")
+    _call(lib.hipo_bias_gelu_nchw_to_nhwc_bf16, "bias_gelu_nchw_to_nhwc", dev, _ptr(x),
+          _ptr(bias), _ptr(out), n, c, h * w)
     return out
 
 
@@ -197,21 +214,20 @@ def gelu_tanh(x: torch.Tensor) -> torch.Tensor:
     """0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))) of a contiguous bf16
     or fp32 tensor, same shape: bf16 correctly rounded per element, fp32 as
     x / (1 + e^(-2u)) to a few ulps."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dtype in (torch.bfloat16, torch.float32), "gelu_tanh: bf16 or fp32 x required")
     _require(x.is_contiguous(), "gelu_tanh: x must be contiguous")
     y = torch.empty_like(x, memory_format=torch.contiguous_format)
     fn = lib.hipo_gelu_tanh_bf16 if x.dtype == torch.bfloat16 else lib.hipo_gelu_tanh_f32
-    with torch.cuda.device(dev):
-        _check(fn(_ptr(x), _ptr(y), x.numel(), _stream(dev)), "gelu_tanh")
+    _call(fn, "gelu_tanh", dev, _ptr(x), _ptr(y), x.numel())
     return y
 
 
 def transpose_last2(x: torch.Tensor) -> torch.Tensor:
     """x.transpose(-2, -1).contiguous() for a contiguous tensor of >= 2 dims
     with 2- or 4-byte elements, moved bit for bit."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dim() >= 2 and x.is_contiguous(), "transpose_last2: contiguous x, >= 2 dims")
     _require(x.element_size() in (2, 4), "transpose_last2: 2- or 4-byte elements required")
@@ -220,25 +236,23 @@ def transpose_last2(x: torch.Tensor) -> torch.Tensor:
     batch = 1
     for d in lead:
         batch *= d
-    with torch.cuda.device(dev):
-        _check(lib.hipo_transpose_last2(_ptr(x), _ptr(y), batch, rows, cols,
-                                        x.element_size(), _stream(dev)), "transpose_last2")
+    _call(lib.hipo_transpose_last2, "transpose_last2", dev, _ptr(x), _ptr(y), batch, rows, cols,
+          x.element_size())
     return y
 
 
 def row_mean_bf16(x: torch.Tensor, *, relu: bool = False) -> torch.Tensor:
     """bf16 mean over the last dim of a contiguous 2-D bf16 tensor (fp32 sum,
     one rounding), of relu(x) with relu=True -> [rows] bf16."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous(),
              "row_mean_bf16: x must be contiguous 2-D bf16")
     rows, cols = x.shape
     _require(cols >= 1 or rows == 0, "row_mean_bf16: mean over zero elements")
     out = torch.empty(rows, dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_row_mean_bf16(_ptr(x), _ptr(out), rows, cols, 1 if relu else 0,
-                                      _stream(dev)), "row_mean_bf16")
+    _call(lib.hipo_row_mean_bf16, "row_mean_bf16", dev, _ptr(x), _ptr(out), rows, cols,
+          1 if relu else 0)
     return out
 
 
@@ -247,7 +261,7 @@ def gelu_erf_bwd_colsum(grad: torch.Tensor, x: torch.Tensor):
     x [rows, cols] (cols a multiple of 8): y = bf16(grad * d(x)) with d the
     correctly rounded fp32 GELU'(x), and colsum = bf16(sum over rows of y)
     as fp32.  Returns (y [rows, cols] bf16, colsum [cols] fp32)."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(grad, x)
     _require(grad.dtype == torch.bfloat16 and x.dtype == torch.bfloat16,
              "gelu_erf_bwd: bf16 operands required")
@@ -259,16 +273,14 @@ def gelu_erf_bwd_colsum(grad: torch.Tensor, x: torch.Tensor):
     colsum = torch.empty(cols, dtype=torch.float32, device=dev)
     need = int(lib.hipo_gelu_erf_bwd_colsum_workspace_bytes(rows, cols))
     ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-    with torch.cuda.device(dev):
-        _check(lib.hipo_gelu_erf_bwd_colsum_bf16(
-            _ptr(grad), _ptr(x), _ptr(y), _ptr(colsum), rows, cols,
-            None if ws is None else _ptr(ws), need, _stream(dev)), "gelu_erf_bwd_colsum")
+    _call(lib.hipo_gelu_erf_bwd_colsum_bf16, "gelu_erf_bwd_colsum", dev, _ptr(grad), _ptr(x),
+          _ptr(y), _ptr(colsum), rows, cols, None if ws is None else _ptr(ws), need)
     return y, colsum
 
 
 def scaled_masked_softmax(x: torch.Tensor, mask: torch.Tensor, scale: float) -> torch.Tensor:
     """softmax(x * scale + mask, -1) for bf16 x [B, Q, K], mask [Q, K]."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x, mask)
     _require(x.dtype == torch.bfloat16 and mask.dtype == torch.bfloat16,
              "masked_softmax: bf16 operands required")
@@ -282,11 +294,8 @@ def scaled_masked_softmax(x: torch.Tensor, mask: torch.Tensor, scale: float) -> 
         mask = mask.contiguous()
     mstride = mask.stride(0) if q > 1 else k
     out = torch.empty_like(x)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_scaled_masked_softmax_bf16(_ptr(x), _ptr(mask), _ptr(out),
-                                                   b, q, k, mstride,
-                                                   float(scale), _stream(dev)),
-               "scaled_masked_softmax")
+    _call(lib.hipo_scaled_masked_softmax_bf16, "scaled_masked_softmax", dev, _ptr(x), _ptr(mask),
+          _ptr(out), b, q, k, mstride, float(scale))
     return out
 
 
@@ -300,7 +309,7 @@ def softmax_lastdim(x: torch.Tensor) -> torch.Tensor:
     with scale 1 and one zero mask row (s = fma(x, 1, 0) = x exactly).  The
     zero row is allocated on a device's first call with that K, which
     therefore must not be inside a graph capture."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dtype == torch.bfloat16, "softmax: bf16 operand required")
     _require(x.dim() >= 1 and x.is_contiguous(), "softmax: x must be contiguous")
@@ -314,11 +323,8 @@ def softmax_lastdim(x: torch.Tensor) -> torch.Tensor:
         _require(not torch.cuda.is_current_stream_capturing(),
                  "softmax: the first call for this K must run outside graph capture")
         zero = _zero_rows[key] = torch.zeros(k, dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_scaled_masked_softmax_bf16(_ptr(x), _ptr(zero), _ptr(out),
-                                                   x.numel() // k, 1, k, k, 1.0,
-                                                   _stream(dev)),
-               "softmax_lastdim")
+    _call(lib.hipo_scaled_masked_softmax_bf16, "softmax_lastdim", dev, _ptr(x), _ptr(zero),
+          _ptr(out), x.numel() // k, 1, k, k, 1.0)
     return out
 
 
@@ -326,7 +332,7 @@ def residual_layernorm(x, residual, gamma, beta, eps: float, *, outputs: str = "
     """(h, y, mean, rstd) of LayerNorm(x + residual) over the last dim;
     outputs="y" returns y alone and writes nothing else, outputs="hy"
     returns (h, y) and writes no statistics."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x, residual, gamma, beta)
     for t in (x, residual, gamma, beta):
         _require(t.dtype == torch.bfloat16 and t.is_contiguous(),
@@ -347,11 +353,8 @@ def residual_layernorm(x, residual, gamma, beta, eps: float, *, outputs: str = "
         ptrs = (_ptr(h), None, None)
     else:
         ptrs = (None, None, None)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_residual_layernorm_bf16(
-            _ptr(x), _ptr(residual), _ptr(gamma), _ptr(beta), ptrs[0], _ptr(y),
-            ptrs[1], ptrs[2], rows, cols, float(eps), _stream(dev)),
-            "residual_layernorm")
+    _call(lib.hipo_residual_layernorm_bf16, "residual_layernorm", dev, _ptr(x), _ptr(residual),
+          _ptr(gamma), _ptr(beta), ptrs[0], _ptr(y), ptrs[1], ptrs[2], rows, cols, float(eps))
     if outputs == "all":
         return h, y, mean, rstd
     return (h, y) if outputs == "hy" else y
@@ -359,7 +362,7 @@ def residual_layernorm(x, residual, gamma, beta, eps: float, *, outputs: str = "
 
 def rmsnorm(x, gamma, eps: float):
     """(y, rstd) of RMSNorm(x) over the last dim."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x, gamma)
     for t in (x, gamma):
         _require(t.dtype == torch.bfloat16 and t.is_contiguous(),
@@ -369,10 +372,8 @@ def rmsnorm(x, gamma, eps: float):
     _require(gamma.shape == (cols,), "rmsnorm: gamma must be [C]")
     y = torch.empty_like(x)
     rstd = torch.empty(rows, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_rmsnorm_bf16(_ptr(x), _ptr(gamma), _ptr(y), _ptr(rstd),
-                                     rows, cols, float(eps), _stream(dev)),
-               "rmsnorm")
+    _call(lib.hipo_rmsnorm_bf16, "rmsnorm", dev, _ptr(x), _ptr(gamma), _ptr(y), _ptr(rstd),
+          rows, cols, float(eps))
     return y, rstd
 
 
@@ -398,11 +399,10 @@ def rmsnorm_ex(x, gamma, eps: float, *, residual=None, scale: float = 1.0, mode:
     y = torch.empty_like(x)
     h = torch.empty_like(x) if want_h else None
     rstd = torch.empty(rows, dtype=torch.float32, device=dev) if want_rstd else None
-    with torch.cuda.device(dev):
-        _check(lib.hipo_rmsnorm_ex_bf16(
-            _ptr(x), None if residual is None else _ptr(residual), _ptr(gamma),
-            None if h is None else _ptr(h), _ptr(y), None if rstd is None else _ptr(rstd),
-            rows, cols, float(eps), float(scale), int(mode), _stream(dev)), "rmsnorm_ex")
+    _call(lib.hipo_rmsnorm_ex_bf16, "rmsnorm_ex", dev, _ptr(x),
+          None if residual is None else _ptr(residual), _ptr(gamma),
+          None if h is None else _ptr(h), _ptr(y), None if rstd is None else _ptr(rstd),
+          rows, cols, float(eps), float(scale), int(mode))
     out = (y, rstd) if want_rstd else (y,)
     out = ((h,) + out) if want_h else out
     return out if len(out) > 1 else out[0]
@@ -412,7 +412,7 @@ def scaled_bias_softmax(x, bias, scale: float, heads: int):
     """softmax(x * scale + bias, -1) for bf16 x [B, Q, K] and a bias
     [B / heads, Q, K] (any layout with unit inner stride and 8-aligned row and
     batch strides) shared by `heads` consecutive batch entries."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x, bias)
     _require(x.dtype == torch.bfloat16 and bias.dtype == torch.bfloat16,
              "bias_softmax: bf16 operands required")
@@ -426,18 +426,15 @@ def scaled_bias_softmax(x, bias, scale: float, heads: int):
     rs = bias.stride(1) if q > 1 else k
     bs = bias.stride(0) if b // heads > 1 else 0
     out = torch.empty_like(x)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_scaled_bias_softmax_bf16(_ptr(x), _ptr(bias), _ptr(out), b, q, k,
-                                                 rs, bs, heads, float(scale),
-                                                 _stream(dev)),
-               "scaled_bias_softmax")
+    _call(lib.hipo_scaled_bias_softmax_bf16, "scaled_bias_softmax", dev, _ptr(x), _ptr(bias),
+          _ptr(out), b, q, k, rs, bs, heads, float(scale))
     return out
 
 
 def spatial_mean_nhwc(x, keepdim: bool = True):
     """Mean over H, W of a channels-last bf16 [N, C, H, W] tensor ->
     [N, C, 1, 1] (keepdim) or [N, C], contiguous bf16."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dtype == torch.bfloat16 and x.dim() == 4, "spatial_mean: bf16 NCHW tensor")
     n, c, h, w = x.shape
@@ -446,11 +443,8 @@ def spatial_mean_nhwc(x, keepdim: bool = True):
     out = torch.empty((n, c, 1, 1) if keepdim else (n, c), dtype=torch.bfloat16, device=dev)
     need = int(lib.hipo_spatial_mean_workspace_bytes(n, h * w, c))
     ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev) if need else None
-    with torch.cuda.device(dev):
-        _check(lib.hipo_spatial_mean_nhwc_bf16(_ptr(x), _ptr(out), n, h * w, c,
-                                               None if ws is None else _ptr(ws), need,
-                                               _stream(dev)),
-               "spatial_mean_nhwc")
+    _call(lib.hipo_spatial_mean_nhwc_bf16, "spatial_mean_nhwc", dev, _ptr(x), _ptr(out),
+          n, h * w, c, None if ws is None else _ptr(ws), need)
     return out
 
 
@@ -506,7 +500,7 @@ def batchnorm_train(x, gamma, beta, running_mean, running_var, *, momentum: floa
     batchnorm_workspace_bytes(n, c, h*w) bytes, reused unmodified across calls
     that are ordered on one stream.  Default: the device's shared workspace
     (callers issuing BatchNorm on several streams at once pass their own)."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x, gamma, beta, running_mean, running_var)
     _require(x.dim() == 4 and x.dtype == torch.float32 and x.is_contiguous(),
              "batchnorm: x must be contiguous NCHW fp32")
@@ -526,13 +520,10 @@ def batchnorm_train(x, gamma, beta, running_mean, running_var, *, momentum: floa
     y = torch.empty_like(x)
     save_mean = torch.empty(c, dtype=torch.float32, device=dev)
     save_invstd = torch.empty(c, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_batchnorm_train_fwd_f32(
-            _ptr(x), _ptr(gamma), _ptr(beta), _ptr(running_mean), _ptr(running_var),
-            _ptr(y), _ptr(save_mean), _ptr(save_invstd), n, c, h * w,
-            float(momentum), float(eps), 1 if relu else 0,
-            _ptr(workspace), workspace.numel() * workspace.element_size(), _stream(dev)),
-            "batchnorm_train")
+    _call(lib.hipo_batchnorm_train_fwd_f32, "batchnorm_train", dev, _ptr(x), _ptr(gamma),
+          _ptr(beta), _ptr(running_mean), _ptr(running_var), _ptr(y), _ptr(save_mean),
+          _ptr(save_invstd), n, c, h * w, float(momentum), float(eps), 1 if relu else 0,
+          _ptr(workspace), workspace.numel() * workspace.element_size())
     return y, save_mean, save_invstd
 
 
@@ -541,15 +532,14 @@ def flat_copy(src: torch.Tensor, dst: torch.Tensor, read_bytes: int | None = Non
     """Measurement yardstick: read `read_bytes` of src and write `write_bytes`
     of dst in one launch with the oracle kernels' access style (default: all
     of each).  Sizes are multiples of 1024 bytes."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(src, dst)
     _require(src.is_contiguous() and dst.is_contiguous(), "flat_copy: contiguous buffers")
     rb = src.numel() * src.element_size() if read_bytes is None else int(read_bytes)
     wb = dst.numel() * dst.element_size() if write_bytes is None else int(write_bytes)
     _require(rb <= src.numel() * src.element_size() and wb <= dst.numel() * dst.element_size(),
              "flat_copy: sizes exceed the buffers")
-    with torch.cuda.device(dev):
-        _check(lib.hipo_flat_copy(_ptr(src), rb, _ptr(dst), wb, _stream(dev)), "flat_copy")
+    _call(lib.hipo_flat_copy, "flat_copy", dev, _ptr(src), rb, _ptr(dst), wb)
 
 
 def flat_copy2(src0: torch.Tensor, src1: torch.Tensor, dst0: torch.Tensor,
@@ -557,15 +547,14 @@ def flat_copy2(src0: torch.Tensor, src1: torch.Tensor, dst0: torch.Tensor,
     """Measurement yardstick: copy src0 -> dst0 and src1 -> dst1 in one
     launch, four streams in lockstep (the residual LayerNorm's pattern).  All
     four buffers contiguous, the same size, a multiple of 1024 bytes."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(src0, src1, dst0, dst1)
     nb = src0.numel() * src0.element_size()
     for t in (src0, src1, dst0, dst1):
         _require(t.is_contiguous() and t.numel() * t.element_size() == nb,
                  "flat_copy2: four contiguous buffers of one size")
-    with torch.cuda.device(dev):
-        _check(lib.hipo_flat_copy2(_ptr(src0), _ptr(src1), _ptr(dst0), _ptr(dst1), nb,
-                                   _stream(dev)), "flat_copy2")
+    _call(lib.hipo_flat_copy2, "flat_copy2", dev, _ptr(src0), _ptr(src1), _ptr(dst0), _ptr(dst1),
+          nb)
 
 
 def hold_copy(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -573,7 +562,7 @@ def hold_copy(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     the single-pass BatchNorm kernel's access pattern (slabs held in
     registers from their loads to their stores, no exchange, no arithmetic
     on the values)."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dtype == torch.float32 and x.dim() == 4 and x.is_contiguous(),
              "hold_copy: a contiguous fp32 [N, C, H, W] tensor required")
@@ -581,8 +570,7 @@ def hold_copy(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     _require(y.shape == x.shape and y.dtype == x.dtype and y.is_contiguous(),
              "hold_copy: out must match x")
     n, c, h, w = x.shape
-    with torch.cuda.device(dev):
-        _check(lib.hipo_hold_copy_f32(_ptr(x), _ptr(y), n, c, h * w, _stream(dev)), "hold_copy")
+    _call(lib.hipo_hold_copy_f32, "hold_copy", dev, _ptr(x), _ptr(y), n, c, h * w)
     return y
 
 
@@ -604,7 +592,7 @@ def batchnorm_nhwc_act_pad(x, gamma, beta, running_mean, running_var, *, momentu
     border.  Returns (save_mean [1, C, 1, 1], save_rstd [1, C, 1, 1], out
     [N, C, H + pad_bottom, W + pad_right] channels-last bf16); running_mean
     / running_var are updated in place."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dim() == 4 and x.dtype == torch.bfloat16
              and x.is_contiguous(memory_format=torch.channels_last),
@@ -618,12 +606,10 @@ def batchnorm_nhwc_act_pad(x, gamma, beta, running_mean, running_var, *, momentu
     save_rstd = torch.empty((1, c, 1, 1), dtype=torch.float32, device=dev)
     need = int(lib.hipo_batchnorm_nhwc_workspace_bytes(n, h, w, c))
     ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_batchnorm_nhwc_act_pad_bf16(
-            _ptr(x), _ptr(gamma), _ptr(beta), _ptr(running_mean), _ptr(running_var),
-            _ptr(save_mean), _ptr(save_rstd), _ptr(out), n, h, w, c, int(pad_bottom),
-            int(pad_right), float(momentum), float(eps), float(var_scale), _BN_ACTS[act],
-            _ptr(ws), ws.numel(), _stream(dev)), "batchnorm_nhwc_act_pad")
+    _call(lib.hipo_batchnorm_nhwc_act_pad_bf16, "batchnorm_nhwc_act_pad", dev, _ptr(x),
+          _ptr(gamma), _ptr(beta), _ptr(running_mean), _ptr(running_var), _ptr(save_mean),
+          _ptr(save_rstd), _ptr(out), n, h, w, c, int(pad_bottom), int(pad_right), float(momentum),
+          float(eps), float(var_scale), _BN_ACTS[act], _ptr(ws), ws.numel())
     return save_mean, save_rstd, out
 
 
@@ -633,7 +619,7 @@ def batchnorm_nchw_act_mean(x, gamma, beta, running_mean, running_var, *, moment
     statistics, an activation and the mean over H, W.  Returns (save_mean
     [1, C, 1, 1], save_rstd [1, C, 1, 1], out [N, C] bf16); running_mean /
     running_var are updated in place."""
-    lib = load_library()
+    lib = _lib or load_library()
     dev = _require_rocm(x)
     _require(x.dim() == 4 and x.dtype == torch.bfloat16 and x.is_contiguous(),
              "batchnorm_nchw: x must be a contiguous NCHW bf16 tensor")
@@ -645,12 +631,10 @@ def batchnorm_nchw_act_mean(x, gamma, beta, running_mean, running_var, *, moment
     save_rstd = torch.empty((1, c, 1, 1), dtype=torch.float32, device=dev)
     need = int(lib.hipo_batchnorm_nchw_mean_workspace_bytes(n, c, h * w))
     ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
-        _check(lib.hipo_batchnorm_nchw_act_mean_bf16(
-            _ptr(x), _ptr(gamma), _ptr(beta), _ptr(running_mean), _ptr(running_var),
-            _ptr(save_mean), _ptr(save_rstd), _ptr(out), n, c, h * w, float(momentum),
-            float(eps), float(var_scale), _BN_ACTS[act], _ptr(ws), ws.numel(), _stream(dev)),
-            "batchnorm_nchw_act_mean")
+    _call(lib.hipo_batchnorm_nchw_act_mean_bf16, "batchnorm_nchw_act_mean", dev, _ptr(x),
+          _ptr(gamma), _ptr(beta), _ptr(running_mean), _ptr(running_var), _ptr(save_mean),
+          _ptr(save_rstd), _ptr(out), n, c, h * w, float(momentum), float(eps), float(var_scale),
+          _BN_ACTS[act], _ptr(ws), ws.numel())
     return save_mean, save_rstd, out
 
 
