@@ -237,3 +237,29 @@ def test_norms_any_row_length(cols, rocm_device):
                 if res is not None:
                     assert torch.equal(h.t.cpu(), hw), what
                 close(y.t, want[0], 2 ** -6 if mode else 2 ** -7, 1e-6, f"rmsnorm {mode} " + what)
+
+
+# (n, c, hw): one group, one channel more and less, channel counts over several
+# blocks of groups, one position, fewer positions than rows per instruction.
+SPATIAL = [(2, 7, 9), (2, 8, 9), (3, 9, 1), (3, 15, 49), (4, 29, 3190), (2, 61, 700), (130, 1001, 49),
+           (6, 1759, 196), (1, 514, 50), (2, 8193, 4), (300, 33, 100)]
+
+
+@pytest.mark.parametrize("n,c,hw", SPATIAL)
+def test_spatial_mean_any_channels(n, c, hw, rocm_device):
+    """fp32 sums of up to 3190 bf16 values rounded once: one bf16 ulp, 2^-8,
+    and 1e-5 near zero."""
+    import oracle as ref
+    torch.manual_seed(n + c + hw)
+    x = torch.randn(n, hw, c).to(torch.bfloat16)
+    want = ref.spatial_mean_nhwc(x.view(n, hw, 1, c).permute(0, 3, 1, 2)).reshape(n, c)
+    for shift in (0, 1):
+        xd = place(x, rocm_device, shift)
+        out = Guarded((n, c), torch.bfloat16, rocm_device, shift)
+        need = lib().hipo_spatial_mean_workspace_bytes(n, hw, c)
+        ws = torch.empty(max(need, 1), dtype=torch.uint8, device=rocm_device)
+        ok(lib().hipo_spatial_mean_nhwc_bf16(xd.data_ptr(), out.t.data_ptr(), n, hw, c,
+                                             ws.data_ptr() if need else None, need, None))
+        torch.cuda.synchronize()
+        out.check(f"[{n}, {c}, {hw}]")
+        close(out.t, want, 2 ** -8, 1e-5, f"[{n}, {c}, {hw}] shift {shift}")
