@@ -149,16 +149,31 @@ __device__ __forceinline__ void unpack8(const u32x4_t v, float (&f)[8]) {
 // (all of x when it fits there).
 // ---------------------------------------------------------------------------
 
+// RAGGED: any C >= 8, any alignment.  The last group of a row ends with it
+// (channels it shares with its neighbour get the same values from both) and
+// accesses are element-aligned.
+template <bool RAGGED>
+__device__ __forceinline__ int64_t group_channel(int g, int64_t C) {
+  return RAGGED ? std::min<int64_t>(8 * static_cast<int64_t>(g), C - 8) : 8 * g;
+}
+
+template <bool RAGGED>
+__device__ __forceinline__ u32x4_t group_load(const uint16_t* p) {
+  if constexpr (RAGGED) return *reinterpret_cast<const u32x4_a2_t*>(p);
+  else return *reinterpret_cast<const u32x4_t*>(p);
+}
+
 // Workgroup s reduces rows [s*L, min(M, (s+1)*L)): sums of (x - shift) and
 // (x - shift)^2 per channel, shift = the slice's first row, with kStatUnroll
 // loads in flight per thread; the R = T / G row partials of a group are added
 // by a fixed-order halving tree in LDS (R is a power of two) and turned into
 // (mean, M2) for the slice.
 constexpr int kStatUnroll = 8;
+template <bool RAGGED>
 __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_partial(
     const uint16_t* __restrict__ x, float2* __restrict__ part, int64_t M, int64_t C, int G,
     int64_t L) {
-  extern __shared__ float lds[];  // [T / 2][16]
+  extern __shared__ float lds[];  // [16][T / 2]
   const int T = blockDim.x;
   const int t = threadIdx.x;
   const int g = t % G;
@@ -167,10 +182,10 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_partial(
   const int64_t s = blockIdx.x;
   const int64_t p0 = s * L;
   const int64_t p1 = std::min<int64_t>(M, p0 + L);
-  const u32x4_t* xv = reinterpret_cast<const u32x4_t*>(x) + g;
-  const int64_t G64 = G;
+  const int64_t c0 = group_channel<RAGGED>(g, C);
+  const uint16_t* xc = x + c0;
 
-  const u32x4_t shv = xv[p0 * G64];
+  const u32x4_t shv = group_load<RAGGED>(xc + p0 * C);
   float shift[8];
   unpack8(shv, shift);
   float s1[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -182,7 +197,7 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_partial(
       // Rows past the slice re-read its first row and count as the shift
       // (a zero deviation).
       const int64_t pu = p + static_cast<int64_t>(u) * R;
-      v[u] = xv[(pu < p1 ? pu : p0) * G64];
+      v[u] = group_load<RAGGED>(xc + (pu < p1 ? pu : p0) * C);
       if (pu >= p1) v[u] = shv;
     }
 #pragma unroll
@@ -198,35 +213,36 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_partial(
     }
   }
   // At each level rows [half, 2 half) store to slot (r - half) * G + g and
-  // rows [0, half) add the slot of row r + half of their group.
+  // rows [0, half) add the slot of row r + half of their group.  Value e of
+  // slot i is at lds[e * T / 2 + i]: consecutive lanes, consecutive banks.
+  const int slots = T / 2;
   for (int half = R / 2; half > 0; half /= 2) {
     if (r >= half && r < 2 * half) {
-      float* slot = lds + ((r - half) * G + g) * 16;
+      float* slot = lds + (r - half) * G + g;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        slot[e] = s1[e];
-        slot[8 + e] = s2[e];
+        slot[e * slots] = s1[e];
+        slot[(8 + e) * slots] = s2[e];
       }
     }
     __syncthreads();
     if (r < half) {
-      const float* slot = lds + (r * G + g) * 16;
+      const float* slot = lds + r * G + g;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        s1[e] += slot[e];
-        s2[e] += slot[8 + e];
+        s1[e] += slot[e * slots];
+        s2[e] += slot[(8 + e) * slots];
       }
     }
     __syncthreads();
   }
   if (t >= G) return;
   const float n = static_cast<float>(p1 - p0);
-  const int64_t S = gridDim.x;
-  float2* dst = part + (8 * g) * S + s;
+  float2* dst = part + s * C + c0;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float d = s1[e] / n;
-    dst[e * S] = make_float2(shift[e] + d, fmaxf(s2[e] - s1[e] * d, 0.f));
+    dst[e] = make_float2(shift[e] + d, fmaxf(s2[e] - s1[e] * d, 0.f));
   }
 }
 
@@ -234,30 +250,30 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_partial(
 // normalised, activated x row (n, ho, wo) when ho < H and wo < W, else zeros.
 // Workgroup b writes rows [b'*R*kApplyUnroll, (b'+1)*R*kApplyUnroll),
 // b' = gridDim.x - 1 - b (reverse order, see above).
-constexpr int kApplyUnroll = 4;
-template <int ACT>
+template <int ACT, bool RAGGED, int kApplyUnroll>
 __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_apply_pad(
     const uint16_t* __restrict__ x, const float* __restrict__ mean,
     const float* __restrict__ rstd, const float* __restrict__ gamma,
     const float* __restrict__ beta, uint16_t* __restrict__ out, uint32_t rows_out, uint32_t H,
-    uint32_t W, uint32_t Ho, uint32_t Wo, DivMagic image_div, DivMagic row_div, int G) {
+    uint32_t W, uint32_t Ho, uint32_t Wo, DivMagic image_div, DivMagic row_div, int64_t C,
+    int G) {
   const int T = blockDim.x;
   const int t = threadIdx.x;
   const int g = t % G;
   const int r = t / G;
   const int R = T / G;
+  const int64_t c0 = group_channel<RAGGED>(g, C);
   float m[8], rs[8], ga[8], be[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    m[e] = mean[8 * g + e];
-    rs[e] = rstd[8 * g + e];
-    ga[e] = gamma[8 * g + e];
-    be[e] = beta[8 * g + e];
+    m[e] = mean[c0 + e];
+    rs[e] = rstd[c0 + e];
+    ga[e] = gamma[c0 + e];
+    be[e] = beta[c0 + e];
   }
-  const u32x4_t* xv = reinterpret_cast<const u32x4_t*>(x) + g;
-  u32x4_t* ov = reinterpret_cast<u32x4_t*>(out) + g;
+  const uint16_t* xc = x + c0;
+  uint16_t* oc = out + c0;
   const uint32_t o0 = (gridDim.x - 1 - blockIdx.x) * static_cast<uint32_t>(R * kApplyUnroll) + r;
-  const int64_t G64 = G;
   u32x4_t v[kApplyUnroll];
   bool inside[kApplyUnroll];
 #pragma unroll
@@ -270,7 +286,7 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_apply_pad(
     inside[u] = o < rows_out && ho < H && wo < W;
     // Padding and rows past the end read row 0 (in bounds) and store zeros.
     const int64_t src = inside[u] ? (static_cast<int64_t>(img) * H + ho) * W + wo : 0;
-    v[u] = xv[src * G64];
+    v[u] = group_load<RAGGED>(xc + src * C);
   }
 #pragma unroll
   for (int u = 0; u < kApplyUnroll; ++u) {
@@ -285,11 +301,16 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_apply_pad(
     u32x4_t w;
 #pragma unroll
     for (int d = 0; d < 4; ++d) w[d] = pack_bf16x2(f[2 * d], f[2 * d + 1]);
-    __builtin_nontemporal_store(w, ov + static_cast<int64_t>(o) * G64);
+    uint16_t* dst = oc + static_cast<int64_t>(o) * C;
+    if constexpr (RAGGED) {
+      *reinterpret_cast<u32x4_a2_t*>(dst) = w;
+    } else {
+      __builtin_nontemporal_store(w, reinterpret_cast<u32x4_t*>(dst));
+    }
   }
 }
 
-// Any C / alignment: one thread per (slice, channel).
+// C < 8, or too many rows for the kernel above: one thread per (slice, channel).
 __global__ __launch_bounds__(256) void bn_nhwc_partial_scalar(
     const uint16_t* __restrict__ x, float2* __restrict__ part, int64_t M, int64_t C, int64_t L) {
   const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -306,7 +327,7 @@ __global__ __launch_bounds__(256) void bn_nhwc_partial_scalar(
   }
   const float n = static_cast<float>(p1 - p0);
   const float d = s1 / n;
-  part[c * static_cast<int64_t>(gridDim.y) + s] = make_float2(shift + d, fmaxf(s2 - s1 * d, 0.f));
+  part[s * C + c] = make_float2(shift + d, fmaxf(s2 - s1 * d, 0.f));
 }
 
 __global__ __launch_bounds__(256) void bn_nhwc_apply_pad_scalar(
@@ -785,138 +806,123 @@ __global__ __launch_bounds__(kChanThreads) void bn_nchw_channels(
 }
 
 // ---------------------------------------------------------------------------
-// Per-channel merge.  The workspace is channel-major: part[c * S + s] is
-// slice s of channel c, which holds (min(units, (s+1)*per) - s*per) * mult
-// values with mean m_s and M2_s.  In fp64, about the shift K = m_0:
-// S1 = sum n_s (m_s - K), S2 = sum M2_s + n_s (m_s - K)^2 -- a plain sum, no
-// divisions.  A workgroup of kFinalThreads threads per channel: thread t
-// adds slices t, t + kFinalThreads, ... (the first kFinalLoads of them
-// loaded at once), a butterfly adds the lanes of each wave, and thread 0
-// adds the waves in order.  mean = K + S1 / N, M2 = S2 - S1^2 / N.
+// Per-channel merge of the channels-last slices.  The workspace is slice-
+// major, part[s * C + c], so the statistics workgroups write and the merge
+// reads contiguous runs.  Slice s holds n_s = min(M, (s+1) * per) - s * per
+// values with mean m_s and M2_s.  In fp64, about the shift K = m_0: S1 = sum
+// n_s (m_s - K), S2 = sum M2_s + n_s (m_s - K)^2 -- a plain sum, no divisions.
+// A workgroup takes kFinalCols channels; thread j * kFinalCols + l adds
+// slices j, j + kFinalLanes, ... of channel l, kFinalLoads loads in flight,
+// and the lanes of a channel are added by a halving tree in LDS.  mean = K +
+// S1 / N, M2 = S2 - S1^2 / N.
 // ---------------------------------------------------------------------------
 constexpr int kFinalThreads = 256;
-constexpr int kFinalLoads = 4;
+constexpr int kFinalCols = 4;
+constexpr int kFinalLanes = kFinalThreads / kFinalCols;
+constexpr int kFinalLoads = 8;
 
 __global__ __launch_bounds__(kFinalThreads) void bn_finalize(
-    const float2* __restrict__ part, int64_t slices, int64_t units, int64_t per, int64_t mult,
+    const float2* __restrict__ part, int64_t slices, int64_t M, int64_t per, int64_t C,
     float* __restrict__ running_mean, float* __restrict__ running_var,
     float* __restrict__ save_mean, float* __restrict__ save_rstd, float momentum, float eps,
     float var_scale) {
-  __shared__ double wsum[kFinalThreads / kWave][3];
-  const int64_t c = blockIdx.x;
+  __shared__ double red[3][kFinalThreads];
   const int t = threadIdx.x;
-  const int lane = t & (kWave - 1);
-  const float2* pc = part + c * slices;
+  const int j = t / kFinalCols;
+  const int64_t c = static_cast<int64_t>(blockIdx.x) * kFinalCols + t % kFinalCols;
+  const float2* pc = part + (c < C ? c : C - 1);
+  const bool owner = j == 0 && c < C;
+  const float rm = owner ? running_mean[c] : 0.f;
+  const float rv = owner ? running_var[c] : 0.f;
   const double K = static_cast<double>(pc[0].x);
   double n = 0.0, s1 = 0.0, s2 = 0.0;
-  auto add = [&](int64_t s, float2 p) {
-    const double cnt =
-        s < slices
-            ? static_cast<double>((std::min<int64_t>(units, (s + 1) * per) - s * per) * mult)
-            : 0.0;
-    const double d = static_cast<double>(p.x) - K;
-    n += cnt;
-    s1 = __builtin_fma(cnt, d, s1);
-    s2 += cnt > 0.0 ? __builtin_fma(cnt * d, d, static_cast<double>(p.y)) : 0.0;
-  };
-  float2 v[kFinalLoads];
+  for (int64_t s0 = j; s0 < slices; s0 += int64_t{kFinalLanes} * kFinalLoads) {
+    float2 v[kFinalLoads];
 #pragma unroll
-  for (int k = 0; k < kFinalLoads; ++k) {
-    const int64_t s = t + static_cast<int64_t>(k) * kFinalThreads;
-    v[k] = pc[s < slices ? s : 0];
-  }
+    for (int k = 0; k < kFinalLoads; ++k) {
+      const int64_t s = s0 + int64_t{k} * kFinalLanes;
+      v[k] = pc[(s < slices ? s : 0) * C];
+    }
 #pragma unroll
-  for (int k = 0; k < kFinalLoads; ++k) add(t + static_cast<int64_t>(k) * kFinalThreads, v[k]);
-  for (int64_t s = t + int64_t{kFinalLoads} * kFinalThreads; s < slices; s += kFinalThreads)
-    add(s, pc[s]);
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    // (lower lane) + (upper lane) in both lanes: the same rounding everywhere
-    const double n2 = __shfl_xor(n, off), a2 = __shfl_xor(s1, off), b2 = __shfl_xor(s2, off);
-    const bool upper = (lane & off) != 0;
-    n = upper ? n2 + n : n + n2;
-    s1 = upper ? a2 + s1 : s1 + a2;
-    s2 = upper ? b2 + s2 : s2 + b2;
+    for (int k = 0; k < kFinalLoads; ++k) {
+      const int64_t s = s0 + int64_t{k} * kFinalLanes;
+      if (s >= slices) continue;
+      const double cnt = static_cast<double>(std::min<int64_t>(M, (s + 1) * per) - s * per);
+      const double d = static_cast<double>(v[k].x) - K;
+      n += cnt;
+      s1 = __builtin_fma(cnt, d, s1);
+      s2 += __builtin_fma(cnt * d, d, static_cast<double>(v[k].y));
+    }
   }
-  if (lane == 0) {
-    wsum[t / kWave][0] = n;
-    wsum[t / kWave][1] = s1;
-    wsum[t / kWave][2] = s2;
-  }
+  red[0][t] = n;
+  red[1][t] = s1;
+  red[2][t] = s2;
   __syncthreads();
-  if (t != 0) return;
-  for (int w = 1; w < kFinalThreads / kWave; ++w) {
-    n += wsum[w][0];
-    s1 += wsum[w][1];
-    s2 += wsum[w][2];
+  for (int half = kFinalLanes / 2; half > 0; half /= 2) {
+    if (j < half) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) red[q][t] += red[q][t + half * kFinalCols];
+    }
+    __syncthreads();
   }
+  if (!owner) return;
+  n = red[0][t];
+  s1 = red[1][t];
+  s2 = red[2][t];
   const double dm = s1 / n;
   const float mean_f = static_cast<float>(K + dm);
   const float var_f = static_cast<float>(std::max(0.0, s2 - s1 * dm) / n);
   save_mean[c] = mean_f;
   save_rstd[c] = 1.0f / __builtin_sqrtf(__fadd_rn(var_f, eps));
   const float keep = 1.0f - momentum;
-  running_mean[c] = __fadd_rn(__fmul_rn(mean_f, momentum), __fmul_rn(running_mean[c], keep));
+  running_mean[c] = __fadd_rn(__fmul_rn(mean_f, momentum), __fmul_rn(rm, keep));
   running_var[c] = __fadd_rn(__fmul_rn(__fmul_rn(var_f, var_scale), momentum),
-                             __fmul_rn(running_var[c], keep));
-}
-
-int64_t gcd64(int64_t a, int64_t b) {
-  while (b) {
-    const int64_t t = a % b;
-    a = b;
-    b = t;
-  }
-  return a;
+                             __fmul_rn(rv, keep));
 }
 
 // Channels-last plan: threads per workgroup (0: scalar kernels), rows per
-// slice and slice count.  Slices of a multiple of 512 rows, at most about
-// 512 of them; the slicing does not depend on the kernel choice, so the
-// workspace size is a function of the shape alone.  The workspace traffic
-// (8 B per channel per slice) stays under 1 % of x for the corpus shapes.
-// Measured on MI355X (statistics kernel, [128, 240, 28, 28] / [128, 96,
-// 112, 112]): 512-row slices, at most 512 of them, 8 non-temporal loads in
-// flight per thread: 15.2 / 49.9 us; at most 1024 / 256 / 128 slices:
-// 61.8 / 53.6 / 84.8 us on the second shape; 256-row slices, 4 or 16 loads,
-// or cached loads: 21-27 / 55-64 us.  Whole call (three launches, graph
-// loop): 44.0 / 160.2 us as planned; 128- or 64-row slices with up to 1024
-// or 2048 of them 71-100 / 167-184 us; 2 or 1 rows per thread in the
-// epilogue instead of kApplyUnroll = 4: 44.1-51.2 / 168.6-203.5 us.  With
-// the SiLU fast form, one call after a 1 GiB cache flush (the runner's
-// protocol), [128, 240, 28, 28] / [128, 96, 112, 112]: 47.2 / 161-163 us
-// with 960-thread workgroups and non-temporal loads; 42.5 / 162.5 with 480
-// threads (G * R above); 38.4 / 161.5 with 480 threads, cached loads and
-// the reversed epilogue (shipped); 256-row slices on top: 40.7 / 162.6.
+// slice and slice count.  A workgroup has R rows of G = ceil(C / 8) groups
+// per instruction, R a power of two, up to 256 threads (the last wave may be
+// partial).  Slices are whole sweeps of R * kStatUnroll rows, at most about
+// 512 of them; where that gives under 192, the sweeps are cut into shorter
+// slices, of 64 rows at least: a launch of a dozen workgroups, one per 512
+// rows, took twice as long.  The slicing depends on the shape alone, and so
+// does the workspace size; its traffic (8 B per channel per slice) stays
+// under 3 % of x.
+// Graph replays of the whole call in us, before (512-row slices, 480-512
+// threads, a slice stride between a workgroup's results) -> now: [128, 240,
+// 28, 28] 33.0 -> 31.5, [128, 96, 112, 112] 159.0 -> 157.7, [29, 896, 14, 14]
+// 32.5 -> 17.1, [128, 1024, 7, 7] 33.5 -> 17.4, [11, 664, 67, 66] 46.4 -> 38.1;
+// C not a multiple of 8, which went one channel per thread, [6, 103, 28, 28]
+// 59 -> 11.2, [8, 28, 112, 112] 85 -> 14.6.  At [128, 240, 28, 28]: up to
+// 1024 slices 34.6, 2048 42.2; 480 / 960 threads 32.2 / 37.3; 16 loads in
+// flight 32.1; non-temporal loads 38.4 (the epilogue's second read then
+// misses the Infinity Cache).  What is left there is two reads and a write
+// (150 MB) and three dependent launches.
+constexpr int kNhwcThreads = 256;
+constexpr int64_t kNhwcMinSlice = 64;
+constexpr int64_t kNhwcMaxSlices = 512;
+constexpr int64_t kNhwcFewSlices = 192;
+
 struct NhwcPlan {
   int threads = 0;
   int64_t slice_len = 0;
   int64_t slices = 0;
 };
 
-constexpr int64_t kNhwcSliceStep = 512;
-constexpr int64_t kNhwcMaxSlices = 512;
-
 NhwcPlan nhwc_plan(int64_t M, int64_t C, bool vec_ok) {
   NhwcPlan plan;
   if (M <= 0 || C <= 0) return plan;
-  if (vec_ok && C % 8 == 0 && C / 8 <= kMaxThreads) {
-    const int64_t G = C / 8;
-    const int64_t lcm = G / gcd64(G, kWave) * kWave;
-    if (lcm <= 512) {
-      plan.threads = static_cast<int>(lcm * (512 / lcm));
-    } else {
-      // Whole waves would take lcm threads (960 for C = 240): one such
-      // workgroup per CU at the kernels' register use.  G * R threads with
-      // a partial last wave fit two or three per CU instead.
-      int64_t R = 1;
-      while (G * R * 2 <= 512) R *= 2;
-      plan.threads = static_cast<int>(G * R);
-    }
-  }
-  const int64_t want = (M + kNhwcMaxSlices - 1) / kNhwcMaxSlices;
-  plan.slice_len = (want + kNhwcSliceStep - 1) / kNhwcSliceStep * kNhwcSliceStep;
-  plan.slices = (M + plan.slice_len - 1) / plan.slice_len;
+  const int64_t G = (C + 7) / 8;
+  int64_t R = 1;
+  while (G * R * 2 <= kNhwcThreads) R *= 2;
+  if (vec_ok && C >= 8 && G <= kMaxThreads) plan.threads = static_cast<int>(G * R);
+  const int64_t sweep = R * kStatUnroll;
+  int64_t len = std::max<int64_t>(kNhwcMinSlice, (M + kNhwcMaxSlices - 1) / kNhwcMaxSlices);
+  len = (len + sweep - 1) / sweep * sweep;
+  while (len > kNhwcMinSlice && M / len < kNhwcFewSlices) len /= 2;
+  plan.slice_len = len;
+  plan.slices = (M + len - 1) / len;
   return plan;
 }
 
@@ -950,42 +956,50 @@ extern "C" int hipo_batchnorm_nhwc_act_pad_bf16(
   const int64_t M = n * h * w;
   const int64_t Ho = h + pad_bottom, Wo = w + pad_right;
   const int64_t rows_out = n * Ho * Wo;
-  const bool vec_ok = aligned16(x) && aligned16(out) && rows_out < (int64_t{1} << 31) &&
-                      M < (int64_t{1} << 31);
-  const NhwcPlan plan = nhwc_plan(M, c, vec_ok);
+  const bool small_rows = rows_out < (int64_t{1} << 31) && M < (int64_t{1} << 31);
+  const bool whole = c % 8 == 0 && aligned16(x) && aligned16(out);
+  const NhwcPlan plan = nhwc_plan(M, c, small_rows);
   const size_t need = static_cast<size_t>(plan.slices * c) * sizeof(float2);
   HIPO_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
                "%s: workspace of %zu bytes (16-byte aligned), need %zu", what, workspace_bytes,
                need);
   HIPO_REQUIRE(plan.slices <= 65535 || plan.threads > 0, "%s: too many rows", what);
   float2* part = static_cast<float2*>(workspace);
+  const int G = static_cast<int>((c + 7) / 8);
   if (plan.threads > 0) {
-    const int G = static_cast<int>(c / 8);
     const int R = plan.threads / G;
-    HIPO_REQUIRE((R & (R - 1)) == 0, "%s: rows per instruction %d not a power of two", what, R);
     const size_t lds = R > 1 ? static_cast<size_t>(plan.threads / 2) * 16 * sizeof(float) : 0;
-    bn_nhwc_partial<<<dim3(static_cast<unsigned>(plan.slices)), dim3(plan.threads), lds,
-                      stream>>>(x, part, M, c, G, plan.slice_len);
+    auto kernel = whole ? bn_nhwc_partial<false> : bn_nhwc_partial<true>;
+    kernel<<<dim3(static_cast<unsigned>(plan.slices)), dim3(plan.threads), lds, stream>>>(
+        x, part, M, c, G, plan.slice_len);
   } else {
     bn_nhwc_partial_scalar<<<dim3(static_cast<unsigned>((c + 255) / 256),
                                   static_cast<unsigned>(plan.slices)),
                              dim3(256), 0, stream>>>(x, part, M, c, plan.slice_len);
   }
-  bn_finalize<<<dim3(static_cast<unsigned>(c)), dim3(kFinalThreads), 0, stream>>>(
-      part, plan.slices, M, plan.slice_len, 1, running_mean, running_var, save_mean, save_rstd,
-      momentum, eps, var_scale);
+  bn_finalize<<<dim3(static_cast<unsigned>((c + kFinalCols - 1) / kFinalCols)),
+                dim3(kFinalThreads), 0, stream>>>(part, plan.slices, M, plan.slice_len, c,
+                                                  running_mean, running_var, save_mean,
+                                                  save_rstd, momentum, eps, var_scale);
   if (plan.threads > 0) {
-    const int G = static_cast<int>(c / 8);
-    const int64_t rows_per_block = static_cast<int64_t>(plan.threads / G) * kApplyUnroll;
-    const int64_t blocks = (rows_out + rows_per_block - 1) / rows_per_block;
-    auto kernel = act == kActSilu   ? bn_nhwc_apply_pad<kActSilu>
-                  : act == kActRelu ? bn_nhwc_apply_pad<kActRelu>
-                                    : bn_nhwc_apply_pad<kActNone>;
+    // Four rows per thread, two where four would leave under 1024 workgroups.
+    const int64_t R = plan.threads / G;
+    const int unroll = (rows_out + 4 * R - 1) / (4 * R) < 1024 ? 2 : 4;
+    const int64_t blocks = (rows_out + unroll * R - 1) / (unroll * R);
+#define HIPO_APPLY(ACT_)                                               \
+  (unroll == 2 ? (whole ? bn_nhwc_apply_pad<ACT_, false, 2>            \
+                        : bn_nhwc_apply_pad<ACT_, true, 2>)            \
+               : (whole ? bn_nhwc_apply_pad<ACT_, false, 4>            \
+                        : bn_nhwc_apply_pad<ACT_, true, 4>))
+    auto kernel = act == kActSilu   ? HIPO_APPLY(kActSilu)
+                  : act == kActRelu ? HIPO_APPLY(kActRelu)
+                                    : HIPO_APPLY(kActNone);
+#undef HIPO_APPLY
     kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(plan.threads), 0, stream>>>(
         x, save_mean, save_rstd, gamma, beta, out, static_cast<uint32_t>(rows_out),
         static_cast<uint32_t>(h), static_cast<uint32_t>(w), static_cast<uint32_t>(Ho),
         static_cast<uint32_t>(Wo), div_magic(static_cast<uint32_t>(Ho * Wo)),
-        div_magic(static_cast<uint32_t>(Wo)), G);
+        div_magic(static_cast<uint32_t>(Wo)), c, G);
   } else {
     const int64_t total = rows_out * c;
     HIPO_REQUIRE((total + 255) / 256 <= 0x7fffffff, "%s: too large", what);

@@ -263,3 +263,44 @@ def test_spatial_mean_any_channels(n, c, hw, rocm_device):
         torch.cuda.synchronize()
         out.check(f"[{n}, {c}, {hw}]")
         close(out.t, want, 2 ** -8, 1e-5, f"[{n}, {c}, {hw}] shift {shift}")
+
+
+# (n, c, h, w, pad): one group, a channel more and less, several groups with a
+# remainder, one row a workgroup and many, more groups than threads.
+BN_NHWC = [(2, 7, 3, 3, 1), (2, 8, 3, 3, 0), (3, 9, 5, 4, 1), (2, 28, 20, 21, 1), (4, 103, 9, 9, 0),
+           (2, 664, 6, 5, 1), (3, 2049, 3, 2, 1), (40, 33, 31, 30, 0), (1, 8200, 2, 2, 0)]
+
+
+@pytest.mark.parametrize("n,c,h,w,pad", BN_NHWC)
+def test_batchnorm_nhwc_any_channels(n, c, h, w, pad, rocm_device):
+    """Statistics 1e-5.  y = act(t), t rounded to bf16, where kernel and oracle
+    may land on neighbouring values: one ulp, up to 2^-7 of t; 1e-5 near zero,
+    where the affine form cancels.  SiLU carries that ulp at a relative slope
+    of at most 1.1 for t > 0 and rounds again, two ulps, 2^-6; for t < 0 the
+    ulp moves it by at most 2^-7 max |t silu'(t)| = 2^-7 * 0.25 = 2e-3."""
+    import oracle as ref
+    torch.manual_seed(n * c + h)
+    x = torch.randn(n, h, w, c).to(torch.bfloat16)
+    gamma, beta, rm, rv = torch.randn(c), torch.randn(c), torch.randn(c), torch.rand(c) + 0.5
+    for shift, act, code in ((0, "silu", 2), (1, "relu", 1), (1, "none", 0)):
+        sm, sr, yw, rmw, rvw = ref.batchnorm_nhwc_act_pad(
+            x.permute(0, 3, 1, 2), gamma, beta, rm, rv, momentum=0.1, eps=1e-3, var_scale=1.25,
+            act=act, pad_bottom=pad, pad_right=pad)
+        xd = place(x, rocm_device, shift)
+        out = Guarded((n, h + pad, w + pad, c), torch.bfloat16, rocm_device, shift)
+        side = [t.to(rocm_device) for t in (gamma, beta, rm, rv)]
+        mean, rstd = (Guarded((c,), torch.float32, rocm_device) for _ in range(2))
+        need = lib().hipo_batchnorm_nhwc_workspace_bytes(n, h, w, c)
+        ws = Guarded((need // 4,), torch.float32, rocm_device)
+        ok(lib().hipo_batchnorm_nhwc_act_pad_bf16(
+            xd.data_ptr(), *(t.data_ptr() for t in side), mean.t.data_ptr(), rstd.t.data_ptr(),
+            out.t.data_ptr(), n, h, w, c, pad, pad, 0.1, 1e-3, 1.25, code, ws.t.data_ptr(), need,
+            None))
+        torch.cuda.synchronize()
+        what = f"[{n}, {c}, {h}, {w}] {act}"
+        for o in (out, mean, rstd, ws):
+            o.check(what)
+        rtol, atol = (2 ** -6, 2e-3) if act == "silu" else (2 ** -7, 1e-5)
+        close(out.t, yw.permute(0, 2, 3, 1), rtol, atol, what)
+        for a, b in ((mean.t, sm), (rstd.t, sr), (side[2], rmw), (side[3], rvw)):
+            close(a, b.reshape(-1), 1e-5, 1e-5, what)
