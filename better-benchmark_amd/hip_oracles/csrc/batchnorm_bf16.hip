@@ -882,30 +882,32 @@ __global__ __launch_bounds__(kFinalThreads) void bn_finalize(
 
 // Channels-last plan: threads per workgroup (0: scalar kernels), rows per
 // slice and slice count.  A workgroup has R rows of G = ceil(C / 8) groups
-// per instruction, R a power of two, up to 256 threads (the last wave may be
-// partial).  Slices are whole sweeps of R * kStatUnroll rows, at most about
-// 512 of them; where that gives under 192, the sweeps are cut into shorter
-// slices, of 64 rows at least: a launch of a dozen workgroups, one per 512
-// rows, took twice as long.  The slicing depends on the shape alone, and so
+// per instruction, R a power of two, up to 512 threads in the statistics pass
+// and 256 in the epilogue (the last wave may be partial).  Slices are of a multiple of 512 rows, at most about 512 of them;
+// where that gives under 192, they are halved, down to 64 rows: a launch of a
+// dozen workgroups, one per 512 rows, took twice as long.  The slicing depends on the shape alone, and so
 // does the workspace size; its traffic (8 B per channel per slice) stays
 // under 3 % of x.
-// Graph replays of the whole call in us, before (512-row slices, 480-512
-// threads, a slice stride between a workgroup's results) -> now: [128, 240,
-// 28, 28] 33.0 -> 31.5, [128, 96, 112, 112] 159.0 -> 157.7, [29, 896, 14, 14]
-// 32.5 -> 17.1, [128, 1024, 7, 7] 33.5 -> 17.4, [11, 664, 67, 66] 46.4 -> 38.1;
-// C not a multiple of 8, which went one channel per thread, [6, 103, 28, 28]
-// 59 -> 11.2, [8, 28, 112, 112] 85 -> 14.6.  At [128, 240, 28, 28]: up to
-// 1024 slices 34.6, 2048 42.2; 480 / 960 threads 32.2 / 37.3; 16 loads in
-// flight 32.1; non-temporal loads 38.4 (the epilogue's second read then
-// misses the Infinity Cache).  What is left there is two reads and a write
-// (150 MB) and three dependent launches.
-constexpr int kNhwcThreads = 256;
+// Graph replays of the whole call in us, before (at least 512-row slices, a
+// slice stride between a workgroup's results) -> now: [128, 240, 28, 28] 33.0
+// -> 31.6, [128, 96, 112, 112] 159.0 -> 156.7, [29, 896, 14, 14] 32.5 -> 16.3,
+// [128, 1024, 7, 7] 33.6 -> 16.7, [11, 664, 67, 66] 46.4 -> 39.0; C not a
+// multiple of 8, which went one channel per thread, [6, 103, 28, 28] 59 ->
+// 12.0, [8, 28, 112, 112] 86 -> 14.9.  At [128, 240, 28, 28]: 392 slices 32.1,
+// 784 34.6, 1568 42.2; statistics with 256 / 1024 threads 32.4 / 32.1; 16
+// loads in flight 32.1; non-temporal loads 38.4 (the epilogue's second read
+// then misses the Infinity Cache).  What is left there is two reads and a
+// write (150 MB) and three dependent launches.
+constexpr int kNhwcStatThreads = 512;
+constexpr int kNhwcApplyThreads = 256;
+constexpr int64_t kNhwcSliceStep = 512;
 constexpr int64_t kNhwcMinSlice = 64;
 constexpr int64_t kNhwcMaxSlices = 512;
 constexpr int64_t kNhwcFewSlices = 192;
 
 struct NhwcPlan {
-  int threads = 0;
+  int threads = 0;  // of the epilogue
+  int stat_threads = 0;
   int64_t slice_len = 0;
   int64_t slices = 0;
 };
@@ -914,12 +916,15 @@ NhwcPlan nhwc_plan(int64_t M, int64_t C, bool vec_ok) {
   NhwcPlan plan;
   if (M <= 0 || C <= 0) return plan;
   const int64_t G = (C + 7) / 8;
-  int64_t R = 1;
-  while (G * R * 2 <= kNhwcThreads) R *= 2;
-  if (vec_ok && C >= 8 && G <= kMaxThreads) plan.threads = static_cast<int>(G * R);
-  const int64_t sweep = R * kStatUnroll;
-  int64_t len = std::max<int64_t>(kNhwcMinSlice, (M + kNhwcMaxSlices - 1) / kNhwcMaxSlices);
-  len = (len + sweep - 1) / sweep * sweep;
+  if (vec_ok && C >= 8 && G <= kMaxThreads) {
+    int64_t R = 1;
+    while (G * R * 2 <= kNhwcApplyThreads) R *= 2;
+    plan.threads = static_cast<int>(G * R);
+    while (G * R * 2 <= kNhwcStatThreads) R *= 2;
+    plan.stat_threads = static_cast<int>(G * R);
+  }
+  const int64_t want = (M + kNhwcMaxSlices - 1) / kNhwcMaxSlices;
+  int64_t len = (want + kNhwcSliceStep - 1) / kNhwcSliceStep * kNhwcSliceStep;
   while (len > kNhwcMinSlice && M / len < kNhwcFewSlices) len /= 2;
   plan.slice_len = len;
   plan.slices = (M + len - 1) / len;
@@ -967,10 +972,10 @@ extern "C" int hipo_batchnorm_nhwc_act_pad_bf16(
   float2* part = static_cast<float2*>(workspace);
   const int G = static_cast<int>((c + 7) / 8);
   if (plan.threads > 0) {
-    const int R = plan.threads / G;
-    const size_t lds = R > 1 ? static_cast<size_t>(plan.threads / 2) * 16 * sizeof(float) : 0;
+    const int T = plan.stat_threads;
+    const size_t lds = T > G ? static_cast<size_t>(T / 2) * 16 * sizeof(float) : 0;
     auto kernel = whole ? bn_nhwc_partial<false> : bn_nhwc_partial<true>;
-    kernel<<<dim3(static_cast<unsigned>(plan.slices)), dim3(plan.threads), lds, stream>>>(
+    kernel<<<dim3(static_cast<unsigned>(plan.slices)), dim3(T), lds, stream>>>(
         x, part, M, c, G, plan.slice_len);
   } else {
     bn_nhwc_partial_scalar<<<dim3(static_cast<unsigned>((c + 255) / 256),
