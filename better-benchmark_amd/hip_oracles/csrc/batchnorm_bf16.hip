@@ -27,7 +27,7 @@
 // launch instead (bn_nchw_channels): x read once, no workspace.
 #include <algorithm>
 
-#include "hipo_common.h"
+#include "row_layout.h"
 
 namespace hipo {
 namespace {
@@ -352,7 +352,8 @@ __global__ __launch_bounds__(256) void bn_nhwc_apply_pad_scalar(
 }
 
 // ---------------------------------------------------------------------------
-// NCHW, general shapes: a workgroup of kNchwImages waves covers a block of
+// NCHW, planes below 8 values of fewer than 8 channels (and grids past the
+// index range): a workgroup of kNchwImages waves covers a block of
 // 64 channels (lane = channel) of kNchwImages consecutive images (wave =
 // image); each lane reads its channel's HW values from memory.
 // ---------------------------------------------------------------------------
@@ -465,8 +466,7 @@ __global__ __launch_bounds__(kNchwImages * kWave) void bn_nchw_small_hw(
 }
 
 // ---------------------------------------------------------------------------
-// NCHW with small planes (C % 8 == 0, HW <= kPlanesMaxHw, x 16-byte
-// aligned): a wave covers 8 consecutive channels of the kNchwImages images
+// NCHW with small planes (C >= 8, HW <= kPlanesMaxHw): a wave covers 8 consecutive channels of the kNchwImages images
 // of one slice -- per image, 8 consecutive H x W planes: 16 * HW bytes, a
 // whole number of 16-byte vectors whatever HW is.  The wave issues all its
 // non-temporal 16-byte loads at once, stages the planes in LDS, and reduces
@@ -484,11 +484,14 @@ constexpr int kPlaneWaves = 4;
 constexpr int kPlaneChannels = 8;  // per wave
 constexpr int kPlanesMaxHw = 128;
 
+// RAGGED: any C >= 8, any alignment: the last wave's 8 channels end with the
+// tensor's (the channels it shares with its neighbour it loads and reduces,
+// but does not write), and the loads are element-aligned.
 // HWB: plane-size bucket (8, 16, 32, 64 or 128 >= HW): each lane holds
 // HWB / 8 values of a plane, and a wave loads at most 4 * HWB / 64 vectors
 // per lane, so both loops have fixed trip counts and their loads issue
 // together.
-template <int MODE, int HWB>
+template <int MODE, int HWB, bool RAGGED>
 __global__ __launch_bounds__(kPlaneWaves * kWave) void bn_nchw_planes(
     const uint16_t* __restrict__ x, float2* __restrict__ part, NchwMerge mg,
     const float* __restrict__ gamma, const float* __restrict__ beta,
@@ -500,12 +503,15 @@ __global__ __launch_bounds__(kPlaneWaves * kWave) void bn_nchw_planes(
   const int w = threadIdx.x >> 6;
   const int r = lane >> 3;
   const int k = lane & 7;
-  const int64_t c0 = (static_cast<int64_t>(blockIdx.x) * kPlaneWaves + w) * kPlaneChannels;
-  const bool wave_ok = c0 < C;  // wave-uniform; C % 8 == 0, so all 8 channels exist
+  const int64_t c_first = (static_cast<int64_t>(blockIdx.x) * kPlaneWaves + w) * kPlaneChannels;
+  const bool wave_ok = c_first < C;  // wave-uniform
+  const int64_t c0 =
+      RAGGED ? std::min<int64_t>(c_first, C - kPlaneChannels) : c_first;  // all 8 exist
   const int64_t s = blockIdx.y;
   const int64_t n0 = s * kNchwImages;
   const int imgs = static_cast<int>(N - n0 < kNchwImages ? N - n0 : kNchwImages);
   const int64_t c = c0 + r;
+  const bool own = !RAGGED || c >= c_first;  // this wave writes channel c
   u32x4_t* lds = reinterpret_cast<u32x4_t*>(stage[w]);
 
   // The slice's planes of these 8 channels: image im's block of 8 planes is
@@ -542,7 +548,11 @@ __global__ __launch_bounds__(kPlaneWaves * kWave) void bn_nchw_planes(
     const int i = i0 < nvec ? i0 : nvec - 1;
     const int im = static_cast<int>(div_by(static_cast<uint32_t>(i), by_hw));
     const int64_t off = static_cast<int64_t>(im) * C * HW + static_cast<int64_t>(i - im * HW) * 8;
-    v[q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(xb + off));
+    if constexpr (RAGGED) {
+      v[q] = *reinterpret_cast<const u32x4_a2_t*>(xb + off);
+    } else {
+      v[q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(xb + off));
+    }
   }
 
   float mc = 0.f, rc = 0.f;
@@ -570,7 +580,7 @@ __global__ __launch_bounds__(kPlaneWaves * kWave) void bn_nchw_planes(
       mc = static_cast<float>(K + dm);
       const float var_f = static_cast<float>(std::max(0.0, s2 - s1 * dm) / n);
       rc = 1.0f / __builtin_sqrtf(__fadd_rn(var_f, mg.eps));
-      if (s == 0 && k == 0) {
+      if (s == 0 && k == 0 && own) {
         mg.save_mean[c] = mc;
         mg.save_rstd[c] = rc;
         const float keep = 1.0f - mg.momentum;
@@ -621,7 +631,7 @@ __global__ __launch_bounds__(kPlaneWaves * kWave) void bn_nchw_planes(
       }
       chan_merge(cnt, mean, m2, static_cast<float>(HW), mu, sum8(q2));
     }
-    if (k == 0) part[c * static_cast<int64_t>(gridDim.y) + s] = make_float2(mean, m2);
+    if (k == 0 && own) part[c * static_cast<int64_t>(gridDim.y) + s] = make_float2(mean, m2);
   } else {
 #pragma unroll
     for (int im = 0; im < kNchwImages; ++im) {
@@ -631,8 +641,164 @@ __global__ __launch_bounds__(kPlaneWaves * kWave) void bn_nchw_planes(
       for (int t = 0; t < kVals; ++t)
         sum += k + 8 * t < HW ? round_bf16(bn_act(val[im][t], mc, rc, gc, bc, act)) : 0.f;
       sum = sum8(sum);
-      if (k == 0)
+      if (k == 0 && own)
         out[(n0 + im) * C + c] =
+            static_cast<uint16_t>(pack_bf16x2(sum / static_cast<float>(HW), 0.f) & 0xffffu);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// NCHW with larger planes (HW >= 8, any C and alignment): a wave per channel
+// and slice of kNchwImages images, a workgroup for kWideWaves consecutive
+// channels of one slice (consecutive planes in memory).  L lanes hold a
+// plane, or a chunk of L * U * 8 values of it, as U element-aligned 16-byte
+// groups each, the plane's last group moved back to its end (RaggedGroup); 64
+// / L planes go side by side, and the loads of all the slice's planes go out
+// together.  Neighbouring planes share cache lines, so the loads are cached
+// and the workgroups, channel fastest, run in XCD order.
+// MODE 0: each chunk's exact two-pass (mean, M2), merged over the chunks and
+//   then over the slice's images in order -> part[c * slices + s].
+// MODE 1: the channel's slices merged in fp64 about the shift m_0 (lanes
+//   strided over the slices, wave_sum: the same in every wave; the waves of
+//   slice 0 write save_* and the running statistics), then
+//   out[n, c] = bf16(sum_hw act(bn(x)) / HW).
+// Against a lane per channel reading its plane value by value, graph replays:
+// [30, 232, 28, 28] 362 -> 12.0 us, [128, 512, 14, 14] 120 -> 29.8, [4, 504, 14,
+// 14] 92 -> 7.0.  One plane per wave, with the merge repeated for each: 13.3,
+// 88, 7.6.
+// ---------------------------------------------------------------------------
+constexpr int kWideWaves = 4;
+
+template <int MODE, int ACT, int L, int U>
+__global__ __launch_bounds__(kWideWaves * kWave) void bn_nchw_wide(
+    const uint16_t* __restrict__ x, float2* __restrict__ part, NchwMerge mg,
+    const float* __restrict__ gamma, const float* __restrict__ beta,
+    uint16_t* __restrict__ out, int64_t N, int64_t C, int64_t HW, int64_t slices,
+    uint32_t cblocks, DivMagic by_cblocks) {
+  constexpr int kSide = kWave / L;               // planes side by side
+  constexpr int kTurns = kNchwImages / kSide;    // turn i holds images kSide i + lane / L
+  const int lane = threadIdx.x & (kWave - 1);
+  const int l = lane & (L - 1);
+  const uint32_t bid = xcd_order(blockIdx.x, gridDim.x);
+  const int64_t s = div_by(bid, by_cblocks);
+  const int64_t c = (bid - s * cblocks) * kWideWaves + (threadIdx.x >> 6);
+  if (c >= C) return;  // wave-uniform; no barrier follows
+  const int imgs = static_cast<int>(std::min<int64_t>(kNchwImages, N - s * kNchwImages));
+  const uint16_t* plane[kTurns];
+#pragma unroll
+  for (int i = 0; i < kTurns; ++i) {
+    const int im = kSide * i + lane / L;  // past the last image: the last one again
+    plane[i] = x + ((s * kNchwImages + (im < imgs ? im : imgs - 1)) * C + c) * HW;
+  }
+
+  float mc = 0.f, rc = 0.f, g = 0.f, b = 0.f;
+  if constexpr (MODE == 1) {
+    const float2* pc = mg.part + c * slices;
+    const double K = static_cast<double>(pc[0].x);
+    double n = 0.0, s1 = 0.0, s2 = 0.0;
+    for (int64_t t = lane; t < slices; t += kWave) {
+      const int64_t hi = (t + 1) * kNchwImages < N ? (t + 1) * kNchwImages : N;
+      const double cnt = static_cast<double>((hi - t * kNchwImages) * HW);
+      const float2 pv = pc[t];
+      const double d = static_cast<double>(pv.x) - K;
+      n += cnt;
+      s1 = __builtin_fma(cnt, d, s1);
+      s2 += __builtin_fma(cnt * d, d, static_cast<double>(pv.y));
+    }
+    n = wave_sum(n);
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    const double dm = s1 / n;
+    mc = static_cast<float>(K + dm);
+    const float var_f = static_cast<float>(std::max(0.0, s2 - s1 * dm) / n);
+    rc = 1.0f / __builtin_sqrtf(__fadd_rn(var_f, mg.eps));
+    g = gamma[c];
+    b = beta[c];
+    if (s == 0 && lane == 0) {
+      mg.save_mean[c] = mc;
+      mg.save_rstd[c] = rc;
+      const float keep = 1.0f - mg.momentum;
+      mg.running_mean[c] =
+          __fadd_rn(__fmul_rn(mc, mg.momentum), __fmul_rn(mg.running_mean[c], keep));
+      mg.running_var[c] = __fadd_rn(__fmul_rn(__fmul_rn(var_f, mg.var_scale), mg.momentum),
+                                    __fmul_rn(mg.running_var[c], keep));
+    }
+  }
+
+  float mean[kTurns], m2[kTurns];  // MODE 0
+  float total[kTurns];             // MODE 1
+  float cnt = 0.f;
+#pragma unroll
+  for (int i = 0; i < kTurns; ++i) mean[i] = m2[i] = total[i] = 0.f;
+  for (int64_t base = 0; base < HW; base += L * U * kRowGroup) {
+    u32x4_t v[kTurns][U];
+    int skip[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const RaggedGroup rg = ragged_group(base + (u * L + l) * kRowGroup, HW);
+      skip[u] = rg.skip;
+#pragma unroll
+      for (int i = 0; i < kTurns; ++i) v[i][u] = ragged_load_cached(plane[i] + rg.col);
+    }
+    const float n = static_cast<float>(std::min<int64_t>(HW - base, L * U * kRowGroup));
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+      if constexpr (MODE == 0) {
+        float sum = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float f[8];
+          unpack8(v[i][u], f);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) sum += e >= skip[u] ? f[e] : 0.f;
+        }
+        const float mu = seg_sum<L>(sum) / n;
+        float q = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float f[8];
+          unpack8(v[i][u], f);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float d = e >= skip[u] ? f[e] - mu : 0.f;
+            q = __builtin_fmaf(d, d, q);
+          }
+        }
+        float have = cnt;
+        chan_merge(have, mean[i], m2[i], n, mu, seg_sum<L>(q));
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float f[8];
+          unpack8(v[i][u], f);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] = bn_affine(f[e], mc, rc, g, b);
+          bn_act_x8<ACT>(f);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) total[i] += e >= skip[u] ? round_bf16(f[e]) : 0.f;
+        }
+      }
+    }
+    cnt += n;
+  }
+  if constexpr (MODE == 0) {
+    float n = 0.f, mm = 0.f, mq = 0.f;
+#pragma unroll
+    for (int im = 0; im < kNchwImages; ++im) {
+      if (im >= imgs) break;  // wave-uniform
+      const int from = im % kSide * L;  // a lane of the image's segment
+      chan_merge(n, mm, mq, cnt, lane_value(mean[im / kSide], from),
+                 lane_value(m2[im / kSide], from));
+    }
+    if (lane == 0) part[c * slices + s] = make_float2(mm, mq);
+  } else {
+#pragma unroll
+    for (int i = 0; i < kTurns; ++i) {
+      const float sum = seg_sum<L>(total[i]);
+      const int im = kSide * i + lane / L;
+      if (im < imgs && l == 0)
+        out[(s * kNchwImages + im) * C + c] =
             static_cast<uint16_t>(pack_bf16x2(sum / static_cast<float>(HW), 0.f) & 0xffffu);
     }
   }
@@ -1076,18 +1242,20 @@ extern "C" int hipo_batchnorm_nchw_act_mean_bf16(
   const NchwMerge none{};
   const NchwMerge mg{part, slices, running_mean, running_var, save_mean, save_rstd,
                      momentum, eps, var_scale};
-  if (c % kPlaneChannels == 0 && hw <= kPlanesMaxHw && aligned16(x)) {
+  if (c >= kPlaneChannels && hw <= kPlanesMaxHw) {
     const int64_t cb = (c + kPlaneWaves * kPlaneChannels - 1) / (kPlaneWaves * kPlaneChannels);
     const dim3 grid(static_cast<unsigned>(cb), static_cast<unsigned>(slices));
     const dim3 block(kPlaneWaves * kWave);
     const int h = static_cast<int>(hw);
     const DivMagic by_hw = div_magic(static_cast<uint32_t>(hw));
+    const bool whole = c % kPlaneChannels == 0 && aligned16(x);
 #define HIPO_PLANES(B_)                                                                      \
   do {                                                                                       \
-    bn_nchw_planes<0, B_><<<grid, block, 0, stream>>>(x, part, none, nullptr, nullptr,        \
-                                                      nullptr, n, c, h, by_hw, act);         \
-    bn_nchw_planes<1, B_><<<grid, block, 0, stream>>>(x, nullptr, mg, gamma, beta, out, n, c, \
-                                                      h, by_hw, act);                        \
+    auto stats = whole ? bn_nchw_planes<0, B_, false> : bn_nchw_planes<0, B_, true>;          \
+    auto apply = whole ? bn_nchw_planes<1, B_, false> : bn_nchw_planes<1, B_, true>;          \
+    stats<<<grid, block, 0, stream>>>(x, part, none, nullptr, nullptr, nullptr, n, c, h,      \
+                                      by_hw, act);                                           \
+    apply<<<grid, block, 0, stream>>>(x, nullptr, mg, gamma, beta, out, n, c, h, by_hw, act); \
   } while (0)
     if (hw <= 8) {
       HIPO_PLANES(8);
@@ -1101,6 +1269,30 @@ extern "C" int hipo_batchnorm_nchw_act_mean_bf16(
       HIPO_PLANES(128);
     }
 #undef HIPO_PLANES
+  } else if (const int64_t cb = (c + kWideWaves - 1) / kWideWaves;
+             hw >= kRowGroup && cb < (int64_t{1} << 31) / slices) {
+    const dim3 grid(static_cast<unsigned>(cb * slices)), block(kWideWaves * kWave);
+    const auto cblocks = static_cast<uint32_t>(cb);
+    const DivMagic by_cb = div_magic(cblocks);
+    // The fewest lanes and groups that hold a plane; beyond 1024 values, chunks.
+#define HIPO_WIDE(L_, U_)                                                                    \
+  do {                                                                                       \
+    bn_nchw_wide<0, kActNone, L_, U_><<<grid, block, 0, stream>>>(                           \
+        x, part, none, nullptr, nullptr, nullptr, n, c, hw, slices, cblocks, by_cb);         \
+    auto apply = act == kActSilu   ? bn_nchw_wide<1, kActSilu, L_, U_>                       \
+                 : act == kActRelu ? bn_nchw_wide<1, kActRelu, L_, U_>                       \
+                                   : bn_nchw_wide<1, kActNone, L_, U_>;                      \
+    apply<<<grid, block, 0, stream>>>(x, nullptr, mg, gamma, beta, out, n, c, hw, slices,    \
+                                      cblocks, by_cb);                                       \
+  } while (0)
+    if (hw <= 32 * kRowGroup) {
+      HIPO_WIDE(32, 1);
+    } else if (hw <= 64 * kRowGroup) {
+      HIPO_WIDE(64, 1);
+    } else {
+      HIPO_WIDE(64, 2);
+    }
+#undef HIPO_WIDE
   } else {
     const dim3 grid(static_cast<unsigned>((c + kNchwChannels - 1) / kNchwChannels),
                     static_cast<unsigned>(slices));

@@ -304,3 +304,44 @@ def test_batchnorm_nhwc_any_channels(n, c, h, w, pad, rocm_device):
         close(out.t, yw.permute(0, 2, 3, 1), rtol, atol, what)
         for a, b in ((mean.t, sm), (rstd.t, sr), (side[2], rmw), (side[3], rvw)):
             close(a, b.reshape(-1), 1e-5, 1e-5, what)
+
+
+# (n, c, h, w): the small-plane kernel with a channel block moved back and with
+# misaligned x (the one-launch kernel needs C % 4 == 0), planes over 128 values
+# at the ends of the lane counts (256, 512, 1024) and in several chunks,
+# fewer channels than a block, fewer values than a group, a partial slice.
+BN_NCHW = [(5, 9, 5, 5), (6, 15, 8, 16), (3, 125, 7, 7), (2, 3, 3, 2), (2, 3, 3, 3), (5, 6, 3, 43),
+           (4, 8, 16, 16), (9, 11, 1, 257), (7, 10, 16, 32), (3, 5, 1, 513), (2, 9, 28, 28),
+           (1, 2, 32, 32), (6, 7, 25, 41), (2, 3, 60, 61), (300, 2, 12, 12)]
+
+
+@pytest.mark.parametrize("n,c,h,w", BN_NCHW)
+def test_batchnorm_nchw_mean_any_plane(n, c, h, w, rocm_device):
+    """Statistics 1e-5.  A mean of up to 3660 activations, each of which may
+    sit one bf16 ulp off the oracle's at a rounding boundary (rarely, and up
+    or down alike), rounded once more: 2^-7, and 1e-4 near zero."""
+    import oracle as ref
+    torch.manual_seed(n + c + h)
+    x = torch.randn(n, c, h, w).to(torch.bfloat16)
+    gamma, beta, rm, rv = torch.randn(c), torch.randn(c), torch.randn(c), torch.rand(c) + 0.5
+    for shift, act, code in ((0, "silu", 2), (1, "relu", 1), (1, "none", 0)):
+        sm, sr, yw, rmw, rvw = ref.batchnorm_nchw_act_mean(
+            x, gamma, beta, rm, rv, momentum=0.1, eps=1e-5, var_scale=1.25, act=act)
+        xd = place(x, rocm_device, shift)
+        out = Guarded((n, c), torch.bfloat16, rocm_device, shift)
+        side = [Guarded((c,), torch.float32, rocm_device) for _ in range(4)]
+        for g, t in zip(side, (gamma, beta, rm, rv)):
+            g.t.copy_(t)
+        mean, rstd = (Guarded((c,), torch.float32, rocm_device) for _ in range(2))
+        need = lib().hipo_batchnorm_nchw_mean_workspace_bytes(n, c, h * w)
+        ws = Guarded((need // 4,), torch.float32, rocm_device)
+        ok(lib().hipo_batchnorm_nchw_act_mean_bf16(
+            xd.data_ptr(), *(g.t.data_ptr() for g in side), mean.t.data_ptr(), rstd.t.data_ptr(),
+            out.t.data_ptr(), n, c, h * w, 0.1, 1e-5, 1.25, code, ws.t.data_ptr(), need, None))
+        torch.cuda.synchronize()
+        what = f"[{n}, {c}, {h}, {w}] {act}"
+        for o in (out, mean, rstd, ws, *side):
+            o.check(what)
+        close(out.t, yw, 2 ** -7, 1e-4, what)
+        for a, b in ((mean.t, sm), (rstd.t, sr), (side[2].t, rmw), (side[3].t, rvw)):
+            close(a, b.reshape(-1), 1e-5, 1e-5, what)
