@@ -353,6 +353,19 @@ BwdPlan bwd_plan(int64_t rows, int64_t cols) {
   return p;
 }
 
+// Rows per block as launched: the plan's, which sizes the workspace, rounded
+// up to whole passes of the 16 waves, a multiple of 32 rows (fewer row blocks,
+// so the workspace holds them).  A last pass that only some rows fill reads
+// and looks up as much as a full one.  Graph replays, the plan's rows -> here:
+// [25216, 3072] 73 -> 96, 91.6 -> 88.5 us; [8192, 6144] 48 -> 64, 65.2 -> 59.5;
+// [28000, 2880] 82 -> 96, 98.0 -> 93.2; [16384, 4608] 72 -> 96, 87.1 -> 86.4.
+// Powers of two instead: 86.9 at the first, but 91.3 at the last.
+int64_t bwd_launch_rows(const BwdPlan& p) {
+  if (p.threads != 1024 || p.rows_per_block > 128) return p.rows_per_block;
+  constexpr int64_t kPass = 16 * kRows;
+  return (p.rows_per_block + kPass - 1) / kPass * kPass;
+}
+
 }  // namespace
 }  // namespace hipo
 
@@ -395,15 +408,15 @@ extern "C" int hipo_gelu_erf_bwd_colsum_bf16(const uint16_t* grad, const uint16_
       static_cast<size_t>(p.row_blocks) * static_cast<size_t>(cols) * sizeof(double);
   HIPO_REQUIRE(workspace_bytes >= need, "gelu_erf_bwd: workspace of %zu bytes, need %zu",
                workspace_bytes, need);
-  const dim3 grid(static_cast<unsigned>(p.col_blocks), static_cast<unsigned>(p.row_blocks));
+  const int64_t rpb = bwd_launch_rows(p);
+  const int row_blocks = static_cast<int>((rows + rpb - 1) / rpb);
+  const dim3 grid(static_cast<unsigned>(p.col_blocks), static_cast<unsigned>(row_blocks));
   double* partial = static_cast<double*>(workspace);
   if (p.threads == 1024)
-    gelu_erf_bwd_tiles<1024><<<grid, 1024, 0, stream>>>(grad, x, y, partial, rows, c,
-                                                        p.rows_per_block);
+    gelu_erf_bwd_tiles<1024><<<grid, 1024, 0, stream>>>(grad, x, y, partial, rows, c, rpb);
   else
-    gelu_erf_bwd_tiles<256><<<grid, 256, 0, stream>>>(grad, x, y, partial, rows, c,
-                                                      p.rows_per_block);
+    gelu_erf_bwd_tiles<256><<<grid, 256, 0, stream>>>(grad, x, y, partial, rows, c, rpb);
   const int rc = check_launch("gelu_erf_bwd_colsum_bf16");
   if (rc != 0) return rc;
-  return launch_finish(partial, colsum, p.row_blocks, cols, stream);
+  return launch_finish(partial, colsum, row_blocks, cols, stream);
 }

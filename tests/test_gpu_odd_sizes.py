@@ -345,3 +345,19 @@ def test_batchnorm_nchw_mean_any_plane(n, c, h, w, rocm_device):
         close(out.t, yw, 2 ** -7, 1e-4, what)
         for a, b in ((mean.t, sm), (rstd.t, sr), (side[2].t, rmw), (side[3].t, rvw)):
             close(a, b.reshape(-1), 1e-5, 1e-5, what)
+
+
+# Rows per block rounded up from 65..96 and 33..63 rows, the last block and
+# the last pass of a block partly filled.
+@pytest.mark.parametrize("rows,cols", [(25000, 3072), (5001, 6144), (1025, 4104)])
+def test_gelu_bwd_row_blocks(rows, cols, rocm_device):
+    """y is one fp32 product of the same operands, the column sum one rounding
+    of an fp64 sum that is exact here: bit for bit."""
+    import hip_oracles
+    import oracle as ref
+    torch.manual_seed(rows)
+    g, x = (torch.randn(rows, cols).to(torch.bfloat16) for _ in range(2))
+    yw, cw = ref.gelu_erf_bwd_colsum(g, x)
+    y, colsum = hip_oracles.gelu_erf_bwd_colsum(g.to(rocm_device), x.to(rocm_device))
+    assert torch.equal(y.cpu(), yw)
+    assert torch.equal(colsum.cpu(), cw)
