@@ -15,17 +15,22 @@
 // HBM-bound: algorithmic bytes per row = 4*cols (read) + 4 (write).
 #include <algorithm>
 
-#include "hipo_common.h"
+#include "row_layout.h"
 
 namespace hipo {
 namespace {
 
 constexpr int kMaxWaves = 8;  // per workgroup
 constexpr int kMaxThreads = kMaxWaves * kWave;
+constexpr int64_t kRaggedMinCols = 1024;
+constexpr int64_t kRaggedMaxRows = 2048;
 
 // WT > 0: waves per row (and rows per workgroup, kMaxWaves / WT) fixed at
 // compile time; WT = 0: both from the arguments.
-template <int U, int WT>
+// RAGGED: rows of any length >= 4, any stride and alignment: a row's last
+// float4 moves back to end with it, where its first values, its neighbour's,
+// count as zero; loads at element alignment.
+template <int U, int WT, bool RAGGED>
 __global__ __launch_bounds__(kMaxThreads) void row_mean_f32_vec4(
     const float* __restrict__ x, float* __restrict__ out, int64_t rows,
     int64_t cols, int64_t row_stride, int w_arg, int rpb_arg) {
@@ -40,9 +45,9 @@ __global__ __launch_bounds__(kMaxThreads) void row_mean_f32_vec4(
   // Waves past the last row still take part in the barrier; they read the
   // last row and write nothing.
   const bool valid = row < rows;
-  const f32x4_t* p =
-      reinterpret_cast<const f32x4_t*>(x + (valid ? row : rows - 1) * row_stride);
-  const int64_t nvec = cols >> 2;
+  const float* xr = x + (valid ? row : rows - 1) * row_stride;
+  const f32x4_t* p = reinterpret_cast<const f32x4_t*>(xr);
+  const int64_t nvec = RAGGED ? (cols + 3) >> 2 : cols >> 2;
   const int64_t step = static_cast<int64_t>(waves_per_row) * kWave;
 
   const int64_t sweeps = (nvec + step * U - 1) / (step * U);
@@ -56,8 +61,16 @@ __global__ __launch_bounds__(kMaxThreads) void row_mean_f32_vec4(
       // Out-of-row slots load the row's last float4 (in bounds, no branch
       // around the load) and are zeroed.
       const int64_t i = base + u * step;
-      v[u] = __builtin_nontemporal_load(p + (i < nvec ? i : nvec - 1));
-      if (i >= nvec) v[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (RAGGED) {
+        const int64_t at = i * 4 < cols - 4 ? i * 4 : cols - 4;
+        const int64_t skip = i * 4 - at;  // >= 4: past the row
+        v[u] = *reinterpret_cast<const f32x4_a4_t*>(xr + at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u][e] = e >= skip ? v[u][e] : 0.f;
+      } else {
+        v[u] = __builtin_nontemporal_load(p + (i < nvec ? i : nvec - 1));
+        if (i >= nvec) v[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) acc += v[u];
@@ -73,7 +86,8 @@ __global__ __launch_bounds__(kMaxThreads) void row_mean_f32_vec4(
   if (valid && w == 0 && lane == 0) out[row] = s / static_cast<float>(cols);
 }
 
-// Any alignment / any cols: scalar loads, one wave per row.
+// Any alignment, any cols: scalar loads, one wave per row (many rows, or short
+// ones; see the entry point).
 __global__ __launch_bounds__(256) void row_mean_f32_scalar(
     const float* __restrict__ x, float* __restrict__ out, int64_t rows,
     int64_t cols, int64_t row_stride) {
@@ -171,30 +185,61 @@ __global__ __launch_bounds__(kBf16Waves * kWave) void row_mean_bf16_short(
   if (k == 0 && r < nrows) out[row0 + r] = round_to_bf16(s / static_cast<float>(cols));
 }
 
-template <bool RELU, bool VEC>
-__global__ __launch_bounds__(256) void row_mean_bf16_long(const uint16_t* __restrict__ x,
-                                                          uint16_t* __restrict__ out,
-                                                          int64_t rows, int64_t cols) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;  // wave-uniform; no barrier follows
-  const uint16_t* p = x + row * cols;
+// Longer rows, and short ones off 16-byte alignment, cols >= 8: W waves per
+// row as in row_mean_f32_vec4, U 16-byte loads per lane in flight; RAGGED: any
+// length and alignment, the row's last group moved back to end with it
+// (RaggedGroup), element-aligned cached loads.  Against one wave per row with
+// one load in flight, graph replays: [2000, 16001] 74.5 -> 12.0 us, [20, 16000]
+// 7.0 -> 3.0, [16000, 777] 10.7 -> 6.3, [8000, 4096] 11.7 -> 11.8.
+template <bool RELU, int U, bool RAGGED>
+__global__ __launch_bounds__(kMaxThreads) void row_mean_bf16_rows(
+    const uint16_t* __restrict__ x, uint16_t* __restrict__ out, int64_t rows, int64_t cols,
+    int waves_per_row, int rows_per_block) {
+  __shared__ float part[kMaxWaves];
+  const RowPlace p = row_place(waves_per_row, rows_per_block, rows);
+  const uint16_t* xr = x + p.row * cols;
+  const int64_t sweep = static_cast<int64_t>(waves_per_row) * kRowSweep;
   float acc = 0.0f;
-  if constexpr (VEC) {
-    const u32x4_t* pv = reinterpret_cast<const u32x4_t*>(p);
-    for (int64_t i = lane; i < cols / 8; i += kWave) {
-      const u32x4_t w = __builtin_nontemporal_load(pv + i);
-      float t = 0.0f;
+  for (int64_t base = 0; base < cols; base += sweep * U) {
+    u32x4_t v[U];
+    int skip[U];
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        t += act_relu<RELU>(bf16lo(w[q])) + act_relu<RELU>(bf16hi(w[q]));
-      acc += t;
+    for (int u = 0; u < U; ++u) {
+      const RaggedGroup rg = ragged_group(base + row_group_col(u, waves_per_row, p), cols);
+      v[u] = RAGGED ? ragged_load_cached(xr + rg.col)
+                    : __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(xr + rg.col));
+      skip[u] = rg.skip;
     }
-  } else {
-    for (int64_t i = lane; i < cols; i += kWave) acc += act_relu<RELU>(bf16_to_f32(p[i]));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        acc += skip[u] <= 2 * d ? act_relu<RELU>(bf16lo(v[u][d])) : 0.0f;
+        acc += skip[u] <= 2 * d + 1 ? act_relu<RELU>(bf16hi(v[u][d])) : 0.0f;
+      }
+    }
   }
-  const float s = wave_sum(acc);
-  if (lane == 0) out[row] = round_to_bf16(s / static_cast<float>(cols));
+  float s = wave_sum(acc);
+  if (waves_per_row > 1) {
+    if (p.lane == 0) part[p.wave] = s;
+    __syncthreads();
+    const int first = p.wave - p.w;
+    s = part[first];
+    for (int k = 1; k < waves_per_row; ++k) s += part[first + k];
+  }
+  if (p.valid && p.w == 0 && p.lane == 0) out[p.row] = round_to_bf16(s / static_cast<float>(cols));
+}
+
+// Fewer than 8 values off 16-byte alignment: a lane per row.
+template <bool RELU>
+__global__ __launch_bounds__(256) void row_mean_bf16_scalar(const uint16_t* __restrict__ x,
+                                                            uint16_t* __restrict__ out,
+                                                            int64_t rows, int64_t cols) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (row >= rows) return;
+  float acc = 0.0f;
+  for (int64_t i = 0; i < cols; ++i) acc += act_relu<RELU>(bf16_to_f32(x[row * cols + i]));
+  out[row] = round_to_bf16(acc / static_cast<float>(cols));
 }
 
 }  // namespace
@@ -210,12 +255,16 @@ extern "C" int hipo_row_mean_f32(const float* x, float* out, int64_t rows,
                (long long)row_stride, (long long)cols);
   if (rows == 0) return 0;
   HIPO_REQUIRE(x != nullptr && out != nullptr, "row_mean: null pointer");
-  const bool vec = cols >= 4 && (cols % 4 == 0) && (row_stride % 4 == 0) &&
-                   aligned16(x);
-  if (vec) {
+  const bool vec = (cols % 4 == 0) && (row_stride % 4 == 0) && aligned16(x);
+  // Rows off the vector path: one wave per row with 4-byte loads is as fast
+  // where the rows alone fill the chip, and faster for short ones ([65536, 17]
+  // 9.2 us against 11.2, [4000, 4097] 11.2 against 12.2); few long rows take
+  // several waves each ([24, 8707] 7.2 -> 3.1 us).
+  const bool ragged = !vec && cols >= kRaggedMinCols && rows < kRaggedMaxRows;
+  if (cols >= 4 && (vec || ragged)) {
     // About 2 KiB per wave: W = ceil(nvec / 128) waves per row (at most 8),
     // U = float4 per lane per sweep.
-    const int64_t nvec = cols / 4;
+    const int64_t nvec = (cols + 3) / 4;
     const int waves = static_cast<int>(
         std::min<int64_t>(kMaxWaves, (nvec + 2 * kWave - 1) / (2 * kWave)));
     const int64_t per_lane = (nvec + int64_t{waves} * kWave - 1) / (int64_t{waves} * kWave);
@@ -224,8 +273,11 @@ extern "C" int hipo_row_mean_f32(const float* x, float* out, int64_t rows,
     HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean: too many rows");
     const dim3 grid(static_cast<unsigned>(blocks)), block(waves * rpb * kWave);
 #define HIPO_MEAN(U_, W_)                                                            \
-  row_mean_f32_vec4<U_, W_><<<grid, block, 0, stream>>>(x, out, rows, cols, row_stride, \
-                                                        waves, rpb)
+  row_mean_f32_vec4<U_, W_, false><<<grid, block, 0, stream>>>(x, out, rows, cols,   \
+                                                               row_stride, waves, rpb)
+#define HIPO_MEAN_RAGGED(U_)                                                         \
+  row_mean_f32_vec4<U_, 0, true><<<grid, block, 0, stream>>>(x, out, rows, cols,     \
+                                                             row_stride, waves, rpb)
 #define HIPO_MEAN_W(U_)                                  \
   switch (waves) {                                       \
     case 1: HIPO_MEAN(U_, 1); break;                     \
@@ -234,13 +286,18 @@ extern "C" int hipo_row_mean_f32(const float* x, float* out, int64_t rows,
     case 8: HIPO_MEAN(U_, 8); break;                     \
     default: HIPO_MEAN(U_, 0); break;                    \
   }
-    if (per_lane <= 1) {
+    if (!vec) {
+      if (per_lane <= 1) HIPO_MEAN_RAGGED(1);
+      else if (per_lane <= 2) HIPO_MEAN_RAGGED(2);
+      else HIPO_MEAN_RAGGED(4);
+    } else if (per_lane <= 1) {
       HIPO_MEAN_W(1);
     } else if (per_lane <= 2) {
       HIPO_MEAN_W(2);
     } else {
       HIPO_MEAN_W(4);
     }
+#undef HIPO_MEAN_RAGGED
 #undef HIPO_MEAN_W
 #undef HIPO_MEAN
   } else {
@@ -280,16 +337,26 @@ extern "C" int hipo_row_mean_bf16(const uint16_t* x, uint16_t* out, int64_t rows
     }
 #undef HIPO_RMB
   } else {
-    const bool vec = cols % 8 == 0 && aligned16(x);
-    const int64_t blocks = (rows + 3) / 4;
-    HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
-    const dim3 grid(static_cast<unsigned>(blocks)), block(256);
-    if (vec) {
-      if (act) row_mean_bf16_long<true, true><<<grid, block, 0, stream>>>(x, out, rows, cols);
-      else row_mean_bf16_long<false, true><<<grid, block, 0, stream>>>(x, out, rows, cols);
+    if (cols >= kRowGroup) {
+      const int waves = static_cast<int>(
+          std::min<int64_t>(kMaxWaves, (cols + 2 * kRowSweep - 1) / (2 * kRowSweep)));
+      const int rpb = kMaxWaves / waves;
+      const int64_t blocks = (rows + rpb - 1) / rpb;
+      HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
+      const bool ragged = cols % 8 != 0 || !aligned16(x);
+      const bool two = cols <= int64_t{waves} * 2 * kRowSweep;  // one sweep of 2 loads
+#define HIPO_RMB(ACT_)                                                                \
+  (two ? (ragged ? row_mean_bf16_rows<ACT_, 2, true> : row_mean_bf16_rows<ACT_, 2, false>) \
+       : (ragged ? row_mean_bf16_rows<ACT_, 4, true> : row_mean_bf16_rows<ACT_, 4, false>))
+      auto kernel = act ? HIPO_RMB(true) : HIPO_RMB(false);
+#undef HIPO_RMB
+      kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(waves * rpb * kWave), 0, stream>>>(
+          x, out, rows, cols, waves, rpb);
     } else {
-      if (act) row_mean_bf16_long<true, false><<<grid, block, 0, stream>>>(x, out, rows, cols);
-      else row_mean_bf16_long<false, false><<<grid, block, 0, stream>>>(x, out, rows, cols);
+      const int64_t blocks = (rows + 255) / 256;
+      HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
+      auto kernel = act ? row_mean_bf16_scalar<true> : row_mean_bf16_scalar<false>;
+      kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(x, out, rows, cols);
     }
   }
   return check_launch("row_mean_bf16");

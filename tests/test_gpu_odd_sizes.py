@@ -361,3 +361,31 @@ def test_gelu_bwd_row_blocks(rows, cols, rocm_device):
     y, colsum = hip_oracles.gelu_erf_bwd_colsum(g.to(rocm_device), x.to(rocm_device))
     assert torch.equal(y.cpu(), yw)
     assert torch.equal(colsum.cpu(), cw)
+
+
+# Below a vector, one vector, one value more and less, several waves per row
+# and more than one sweep; a row stride past the row.
+@pytest.mark.parametrize("cols", [1, 3, 4, 5, 7, 8, 9, 255, 257, 333, 511, 513, 777, 1025, 4097,
+                                  8707, 33000])
+def test_row_mean_any_row_length(cols, rocm_device):
+    """fp32 sums in another order: 1e-5.  bf16: one rounding of an fp32 mean,
+    one ulp, 2^-7, and 1e-5 near zero."""
+    import oracle as ref
+    torch.manual_seed(cols)
+    rows = 11
+    x = torch.randn(rows, cols + 3)
+    xb = torch.randn(rows, cols).to(torch.bfloat16)
+    for shift in (0, 1):
+        xd = place(x, rocm_device, shift)
+        out = Guarded((rows,), torch.float32, rocm_device)
+        ok(lib().hipo_row_mean_f32(xd.data_ptr(), out.t.data_ptr(), rows, cols, cols + 3, None))
+        torch.cuda.synchronize()
+        out.check(f"f32 {cols}")
+        close(out.t, ref.row_mean(x[:, :cols].contiguous()), 1e-5, 1e-5, f"f32 {cols}")
+        xd = place(xb, rocm_device, shift)
+        for relu in (0, 1):
+            out = Guarded((rows,), torch.bfloat16, rocm_device)
+            ok(lib().hipo_row_mean_bf16(xd.data_ptr(), out.t.data_ptr(), rows, cols, relu, None))
+            torch.cuda.synchronize()
+            out.check(f"bf16 {cols}")
+            close(out.t, ref.row_mean_bf16(xb, relu=bool(relu)), 2 ** -7, 1e-5, f"bf16 {cols}")
