@@ -259,7 +259,8 @@ size_t hipo_batchnorm_workspace_bytes(int64_t n, int64_t c, int64_t hw);
  *   running_var  = (1 - momentum) running_var
  *                  + momentum var * count / (count - 1)     (in place)
  * x, y are contiguous [n, c, hw]; gamma, beta, running_*, save_* are [c].
- * Channels of at most 16384 values (n * hw) run as one launch with a
+ * Channels of at most 16384 values (n * hw), and of up to 28672 (49152 where
+ * hw is not a multiple of 4) where that is faster, run as one launch with a
  * workgroup per channel that holds it in registers (reads x once, uses no
  * workspace); larger ones as one persistent kernel that reads x once (HW a
  * multiple of 4, 16-byte aligned x / y, x under 4 GiB), others as two
