@@ -606,6 +606,10 @@ extern "C" int hipo_batchnorm_train_fwd_f32(
   const PlaneGeom g = plane_geom(hw);
   const bool vec = hw >= 4 && hw < (int64_t{1} << 30) &&
                    (n + S - 1) / S * g.F < (int64_t{1} << 30);
+  // In place (y == x), planes whose last vector is moved back go value by
+  // value in the second pass: the values it shares with its neighbour would
+  // be read by one thread after the other stored them.
+  const bool apply_vec = vec && (hw % 4 == 0 || y != x);
   const dim3 grid(static_cast<unsigned>(S * c));
   const DivMagic by_S = div_magic(static_cast<uint32_t>(S));
   float* ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + kBnCtlBytes +
@@ -614,7 +618,7 @@ extern "C" int hipo_batchnorm_train_fwd_f32(
   stats<<<grid, dim3(kThreads), 0, stream>>>(x, ws, n, c, g, S, by_S);
   int rc = check_launch("batchnorm_train_fwd_f32 (stats)");
   if (rc) return rc;
-  auto normalize = vec ? bn_normalize<true> : bn_normalize<false>;
+  auto normalize = apply_vec ? bn_normalize<true> : bn_normalize<false>;
   normalize<<<grid, dim3(kThreads), 0, stream>>>(x, gamma, beta, running_mean, running_var, y,
                                                  save_mean, save_invstd, ws, n, c, g, S, by_S,
                                                  momentum, eps, relu);

@@ -258,7 +258,8 @@ size_t hipo_batchnorm_workspace_bytes(int64_t n, int64_t c, int64_t hw);
  *   running_mean = (1 - momentum) running_mean + momentum mean
  *   running_var  = (1 - momentum) running_var
  *                  + momentum var * count / (count - 1)     (in place)
- * x, y are contiguous [n, c, hw]; gamma, beta, running_*, save_* are [c].
+ * x, y are contiguous [n, c, hw]; y may be x itself (in place), and does
+ * not overlap it otherwise; gamma, beta, running_*, save_* are [c].
  * Channels of at most 16384 values (n * hw), and of up to 28672 (49152 where
  * hw is not a multiple of 4) where that is faster, run as one launch with a
  * workgroup per channel that holds it in registers (reads x once, uses no

@@ -1,0 +1,48 @@
+"""Calls whose output is one of the inputs, through the C entry points: the
+results are those of the same call with a separate output, bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def lib():
+    import hip_oracles
+    return hip_oracles.load_library()
+
+
+def ok(rc):
+    assert rc == 0, lib().hipo_last_error()
+
+
+def same(got, want, what):
+    torch.cuda.synchronize()
+    assert torch.equal(got.cpu(), want.cpu()), what
+
+
+# Value by value; register-held planes of whole vectors and not, 256 and 1024
+# threads; the single-pass kernel; split-K with whole vectors (x off alignment)
+# and with planes whose last vector is moved back.
+@pytest.mark.parametrize("n,c,hw,shift", [
+    (3, 5, 7, 0), (26, 9, 49, 0), (335, 3, 49, 0), (128, 40, 196, 0), (16, 8, 3136, 0),
+    (16, 8, 3136, 1), (60, 2, 1023, 0), (1, 4, 50001, 0), (700, 2, 70, 0), (400, 4, 131, 1)])
+def test_batchnorm_train_in_place(n, c, hw, shift, rocm_device):
+    torch.manual_seed(n + c + hw)
+    x = torch.randn(n * c * hw + shift, device=rocm_device) * 2 + 0.5
+    gamma, beta = torch.randn(c, device=rocm_device), torch.randn(c, device=rocm_device)
+    outs = []
+    for in_place in (False, True):
+        xd = x.clone()[shift:]
+        y = xd if in_place else torch.empty_like(x)[shift:]
+        rm, rv = torch.zeros(c, device=rocm_device), torch.ones(c, device=rocm_device)
+        mean, invstd = torch.empty_like(rm), torch.empty_like(rm)
+        need = lib().hipo_batchnorm_workspace_bytes(n, c, hw)
+        ws = torch.zeros(need, dtype=torch.uint8, device=rocm_device)
+        ok(lib().hipo_batchnorm_train_fwd_f32(
+            xd.data_ptr(), gamma.data_ptr(), beta.data_ptr(), rm.data_ptr(), rv.data_ptr(),
+            y.data_ptr(), mean.data_ptr(), invstd.data_ptr(), n, c, hw, 0.1, 1e-5, 1,
+            ws.data_ptr(), need, None))
+        torch.cuda.synchronize()
+        outs.append((y.clone(), mean, invstd, rm, rv))
+    for name, a, b in zip(("y", "mean", "invstd", "running_mean", "running_var"), *outs):
+        same(b, a, f"[{n}, {c}, {hw}] {name}")
