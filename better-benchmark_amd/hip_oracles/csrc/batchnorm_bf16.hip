@@ -310,7 +310,8 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_apply_pad(
   }
 }
 
-// C < 8, or too many rows for the kernel above: one thread per (slice, channel).
+// C < 8, or too many rows for the kernels above: one thread per (slice,
+// channel), and per output value (also in place with C not a multiple of 8).
 __global__ __launch_bounds__(256) void bn_nhwc_partial_scalar(
     const uint16_t* __restrict__ x, float2* __restrict__ part, int64_t M, int64_t C, int64_t L) {
   const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1152,7 +1153,10 @@ extern "C" int hipo_batchnorm_nhwc_act_pad_bf16(
                 dim3(kFinalThreads), 0, stream>>>(part, plan.slices, M, plan.slice_len, c,
                                                   running_mean, running_var, save_mean,
                                                   save_rstd, momentum, eps, var_scale);
-  if (plan.threads > 0) {
+  // In place (out == x, no padding), channels past the last whole group go
+  // one by one: the group moved back over them would read, in its first
+  // channels, what its neighbour may have stored already.
+  if (plan.threads > 0 && (c % 8 == 0 || out != x)) {
     // Four rows per thread, two where four would leave under 1024 workgroups.
     const int64_t R = plan.threads / G;
     const int unroll = (rows_out + 4 * R - 1) / (4 * R) < 1024 ? 2 : 4;

@@ -209,7 +209,8 @@ size_t hipo_batchnorm_nhwc_workspace_bytes(int64_t n, int64_t h, int64_t w, int6
 /*
  * x is [n, c, h, w] stored channels-last (physical [n, h, w, c]); out is
  * [n, c, h + pad_bottom, w + pad_right] stored channels-last, y in the
- * top-left h x w window and zeros in the padding.
+ * top-left h x w window and zeros in the padding.  Without padding out may be
+ * x itself; it does not overlap x otherwise.
  * Replaces the Triton body of oracle_forward in
  * repros/canonical/var_mean_ceb5c315290a/oracle.py:238 (split-K statistics,
  * then the normalise + SiLU + pad epilogue; eps 1e-3, SiLU, pad 1).

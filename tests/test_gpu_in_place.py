@@ -46,3 +46,29 @@ def test_batchnorm_train_in_place(n, c, hw, shift, rocm_device):
         outs.append((y.clone(), mean, invstd, rm, rv))
     for name, a, b in zip(("y", "mean", "invstd", "running_mean", "running_var"), *outs):
         same(b, a, f"[{n}, {c}, {hw}] {name}")
+
+
+@pytest.mark.parametrize("c", [5, 8, 72, 103, 1001])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_batchnorm_nhwc_in_place(c, shift, rocm_device):
+    """No padding: out has x's shape."""
+    n, h, w = 6, 20, 31
+    torch.manual_seed(c)
+    x = (torch.randn(n * h * w * c + shift, device=rocm_device) * 2 + 0.5).to(torch.bfloat16)
+    gamma, beta = torch.randn(c, device=rocm_device), torch.randn(c, device=rocm_device)
+    outs = []
+    for in_place in (False, True):
+        xd = x.clone()[shift:]
+        y = xd if in_place else torch.empty_like(x)[shift:]
+        rm, rv = torch.zeros(c, device=rocm_device), torch.ones(c, device=rocm_device)
+        mean, rstd = torch.empty_like(rm), torch.empty_like(rm)
+        need = lib().hipo_batchnorm_nhwc_workspace_bytes(n, h, w, c)
+        ws = torch.empty(need, dtype=torch.uint8, device=rocm_device)
+        ok(lib().hipo_batchnorm_nhwc_act_pad_bf16(
+            xd.data_ptr(), gamma.data_ptr(), beta.data_ptr(), rm.data_ptr(), rv.data_ptr(),
+            mean.data_ptr(), rstd.data_ptr(), y.data_ptr(), n, h, w, c, 0, 0, 0.1, 1e-5, 1.0, 1,
+            ws.data_ptr(), need, None))
+        torch.cuda.synchronize()
+        outs.append((y.clone(), mean, rstd, rm, rv))
+    for name, a, b in zip(("out", "mean", "rstd", "running_mean", "running_var"), *outs):
+        same(b, a, f"C {c} shift {shift} {name}")
