@@ -75,11 +75,8 @@ __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
         sum += bf16lo(hv[u][d]) + bf16hi(hv[u][d]);
       }
     }
-    const int64_t col = row_group_col(u, waves_per_row, p);
-    if constexpr (RAGGED) {
-      if (h != nullptr && p.valid && rg[u].skip < kRowGroup)
-        ragged_store(h + base + rg[u].col, hv[u]);
-    } else {
+    if constexpr (!RAGGED) {
+      const int64_t col = row_group_col(u, waves_per_row, p);
       if (h != nullptr && p.valid && col < cols) row_store_stream(h + base, col, hv[u]);
     }
   }
@@ -123,6 +120,14 @@ __global__ __launch_bounds__(kRowMaxThreads) void residual_layernorm_rows(
   const float mean = t.mean;
   const float rstd = 1.0f / __builtin_sqrtf(t.m2 / static_cast<float>(cols) + eps);
   const float shift = -mean * rstd;
+  // Ragged rows store h here, past the row's barrier: a group moved back reads
+  // values that another wave owns, and h may be x or the residual.
+  if constexpr (RAGGED) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (h != nullptr && p.valid && rg[u].skip < kRowGroup)
+        ragged_store(h + base + rg[u].col, hv[u]);
+  }
 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -213,11 +218,8 @@ __global__ __launch_bounds__(kRowMaxThreads) void rmsnorm_rows(
       for (int d = 0; d < 4; ++d)
         xv[u][d] = pack_bf16x2(bf16lo(xv[u][d]) + bf16lo(rv[d]),
                                bf16hi(xv[u][d]) + bf16hi(rv[d]));
-      const int64_t col = row_group_col(u, waves_per_row, p);
-      if constexpr (RAGGED) {
-        if (h != nullptr && p.valid && rg[u].skip < kRowGroup)
-          ragged_store(h + base + rg[u].col, xv[u]);
-      } else {
+      if constexpr (!RAGGED) {
+        const int64_t col = row_group_col(u, waves_per_row, p);
         if (h != nullptr && p.valid && col < cols) row_store_stream(h + base, col, xv[u]);
       }
     }
@@ -242,6 +244,12 @@ __global__ __launch_bounds__(kRowMaxThreads) void rmsnorm_rows(
     for (int k = 1; k < waves_per_row; ++k) sq += part[first + k];
   }
   const float rstd = 1.0f / __builtin_sqrtf(sq / static_cast<float>(cols) + eps);
+  if constexpr (RES && RAGGED) {  // past the barrier, as in residual_layernorm_rows
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (h != nullptr && p.valid && rg[u].skip < kRowGroup)
+        ragged_store(h + base + rg[u].col, xv[u]);
+  }
 
   // The scale test is hoisted out of the per-element loop (one uniform
   // branch, two copies of the store loop).
@@ -280,24 +288,29 @@ __global__ __launch_bounds__(256) void residual_layernorm_rows_scalar(
       static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int64_t base = row * cols;
+  auto add = [&](int64_t j) {
+    return round_bf16(bf16_to_f32(x[base + j]) + bf16_to_f32(res[base + j]));
+  };
   float sum = 0.f;
   for (int64_t j = lane; j < cols; j += kWave) {
-    const float hv = round_bf16(bf16_to_f32(x[base + j]) + bf16_to_f32(res[base + j]));
+    const float hv = add(j);
     if (h != nullptr) h[base + j] = static_cast<uint16_t>(pack_bf16x2(hv, 0.f) & 0xffffu);
     sum += hv;
   }
+  // From here on h where it was written (by this lane): it may be x or the
+  // residual.
+  auto again = [&](int64_t j) { return h != nullptr ? bf16_to_f32(h[base + j]) : add(j); };
   const float mean = wave_sum(sum) / static_cast<float>(cols);
   float sq = 0.f;
   for (int64_t j = lane; j < cols; j += kWave) {
-    const float a =
-        round_bf16(bf16_to_f32(x[base + j]) + bf16_to_f32(res[base + j])) - mean;
+    const float a = again(j) - mean;
     sq = __builtin_fmaf(a, a, sq);
   }
   const float rstd =
       1.0f / __builtin_sqrtf(wave_sum(sq) / static_cast<float>(cols) + eps);
   const float shift = -mean * rstd;
   for (int64_t j = lane; j < cols; j += kWave) {
-    const float hv = round_bf16(bf16_to_f32(x[base + j]) + bf16_to_f32(res[base + j]));
+    const float hv = again(j);
     const float v = __builtin_fmaf(__builtin_fmaf(hv, rstd, shift),
                                    bf16_to_f32(gamma[j]), bf16_to_f32(beta[j]));
     y[base + j] = static_cast<uint16_t>(pack_bf16x2(v, 0.f) & 0xffffu);
@@ -330,7 +343,8 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_scalar(
   const float rstd =
       1.0f / __builtin_sqrtf(wave_sum(sq) / static_cast<float>(cols) + eps);
   for (int64_t j = lane; j < cols; j += kWave) {
-    float v = hval(j) * rstd;
+    // h where this lane wrote it: it may be x or the residual.
+    float v = (h != nullptr ? bf16_to_f32(h[base + j]) : hval(j)) * rstd;
     if (mode == 0) {
       v = v * bf16_to_f32(gamma[j]);
       if (scale != 1.0f) v *= scale;
@@ -560,10 +574,17 @@ __global__ __launch_bounds__(256) void residual_layernorm_seg(
         if (counts(u, 0)) sum += bf16lo(hv[u][d]) + bf16hi(hv[u][d]);
       }
     }
-    if (h != nullptr) store(h + base, u, hv[u]);
+    if (!RAGGED && h != nullptr) store(h + base, u, hv[u]);
   }
   const float inv_n = 1.0f / static_cast<float>(cols);
   const float mean = seg_sum<L>(sum) * inv_n;
+  // Ragged rows: past the loads of all the row's groups (the sum waits for
+  // them), for h may be x or the residual.
+  if constexpr (RAGGED) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (h != nullptr) store(h + base, u, hv[u]);
+  }
   float sq = 0.f;
 #pragma unroll
   for (int u = 0; u < U; ++u) {

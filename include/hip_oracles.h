@@ -96,7 +96,9 @@ int hipo_scaled_masked_softmax_bf16(const uint16_t* x, const uint16_t* mask,
  *   h = bf16(x + residual);  mean, var = fp32 stats of h (population var)
  *   rstd = 1/sqrt(var + eps);  y = bf16((h - mean) * rstd * gamma + beta)
  * x, residual, h, y are [rows, cols] contiguous; gamma, beta are [cols];
- * mean, rstd are fp32 [rows].  h, mean and rstd may be NULL: that output is
+ * mean, rstd are fp32 [rows].  h, and y, may be x or the residual itself
+ * (not both of them the same tensor), and overlap no operand otherwise.
+ * h, mean and rstd may be NULL: that output is
  * not written (the reference's var_mean_80e7ff4dee7f returns y only).
  * Replaces the Triton body of oracle_forward in
  * repros/canonical/var_mean_80e7ff4dee7f/oracle.py:122
@@ -116,6 +118,7 @@ int hipo_residual_layernorm_bf16(const uint16_t* x, const uint16_t* residual,
  *   rstd = 1/sqrt(mean(x^2) + eps)   (fp32)
  *   y = bf16(x * rstd * gamma)       (fp32 arithmetic, one rounding)
  * x, y are [rows, cols] contiguous; gamma is [cols]; rstd is fp32 [rows].
+ * y may be x itself, and does not overlap it otherwise.
  * Replaces the Triton body of oracle_forward in
  * repros/canonical/mean_4462ce967d63/oracle.py:65.
  */
@@ -131,7 +134,8 @@ int hipo_rmsnorm_bf16(const uint16_t* x, const uint16_t* gamma, uint16_t* y,
  *   mode 1: t = bf16(h * rstd); u = bf16(gamma * t);
  *           y = scale == 1 ? u : bf16(u * scale)   (HF T5 LayerNorm op order)
  * residual, h and rstd may be NULL (h, the bf16 sum, only with a
- * residual).  Shapes as hipo_rmsnorm_bf16.
+ * residual).  Shapes as hipo_rmsnorm_bf16; h and y may be x or the residual
+ * as in hipo_residual_layernorm_bf16.
  * Replaces the Triton body of oracle_forward in
  * repros/canonical/mean_4462ce967d63/oracle.py:65 (T5: residual, eps 1e-6,
  * mode 1, scale 0.04419417382415922) and of the residual-RMSNorm families

@@ -72,3 +72,39 @@ def test_batchnorm_nhwc_in_place(c, shift, rocm_device):
         outs.append((y.clone(), mean, rstd, rm, rv))
     for name, a, b in zip(("out", "mean", "rstd", "running_mean", "running_var"), *outs):
         same(b, a, f"C {c} shift {shift} {name}")
+
+
+# Value by value; one row to a part of a wave, with one and two groups a lane;
+# several waves a row with the last group moved back over a wave's first
+# values (cols % 512 in 1..7), over its own wave's, and not at all; rows longer
+# than the registers hold.
+@pytest.mark.parametrize("cols", [5, 64, 197, 513, 769, 1543, 2049, 2055, 4096, 4097, 8195, 33001])
+def test_norms_in_place(cols, rocm_device):
+    """h over x and over the residual, y over x: as with separate outputs."""
+    rows, bf = 37, torch.bfloat16
+    torch.manual_seed(cols)
+    x, r = (torch.randn(rows, cols, device=rocm_device).to(bf) for _ in range(2))
+    gamma, beta = (torch.randn(cols, device=rocm_device).to(bf) for _ in range(2))
+
+    def run(op, where):
+        xd, rd = x.clone(), r.clone()
+        spare = [torch.empty_like(x) for _ in range(2)]
+        h, y = {"apart": spare, "h=x": (xd, spare[0]), "h=res": (rd, spare[0]),
+                "y=x": (spare[0], xd)}[where]
+        mean, rstd = (torch.empty(rows, device=rocm_device) for _ in range(2))
+        if op == "layernorm":
+            ok(lib().hipo_residual_layernorm_bf16(
+                xd.data_ptr(), rd.data_ptr(), gamma.data_ptr(), beta.data_ptr(), h.data_ptr(),
+                y.data_ptr(), mean.data_ptr(), rstd.data_ptr(), rows, cols, 1e-5, None))
+        else:
+            ok(lib().hipo_rmsnorm_ex_bf16(
+                xd.data_ptr(), rd.data_ptr(), gamma.data_ptr(), h.data_ptr(), y.data_ptr(),
+                rstd.data_ptr(), rows, cols, 1e-5, 0.5, 1, None))
+        torch.cuda.synchronize()
+        return h, y, rstd
+
+    for op in ("layernorm", "rmsnorm"):
+        want = run(op, "apart")
+        for where in ("h=x", "h=res", "y=x"):
+            for name, a, b in zip(("h", "y", "rstd"), run(op, where), want):
+                same(a, b, f"{op} cols {cols} {where} {name}")
