@@ -229,7 +229,8 @@ __global__ __launch_bounds__(kThreads) void bn_partial_stats(
 }
 
 // Merge the S partial triples of channel c in fp64 about the first one's
-// mean K: with d_s = mean_s - K, S1 = sum n_s d_s and S2 = sum M2_s + n_s
+// mean K (0 where that is not finite: mean_s - K of an infinite one would be
+// NaN): with d_s = mean_s - K, S1 = sum n_s d_s and S2 = sum M2_s + n_s
 // d_s^2, mean = K + S1 / N and M2 = S2 - S1^2 / N.  One wave: lane l adds
 // splits l, l + 64, ... in order, then wave_sum (a fixed order).  All 64
 // lanes active; every lane returns the result.
@@ -237,7 +238,7 @@ __device__ void channel_stats(const float* __restrict__ ws, int64_t c,
                               int64_t S, double& mean, double& m2,
                               double& count) {
   const float* p = ws + c * S * 3;
-  const double K = p[1];
+  const double K = __builtin_isfinite(p[1]) ? p[1] : 0.f;
   double n = 0.0, s1 = 0.0, s2 = 0.0;
   for (int64_t s = threadIdx.x & (kWave - 1); s < S; s += kWave) {
     const double nb = p[3 * s], d = static_cast<double>(p[3 * s + 1]) - K;

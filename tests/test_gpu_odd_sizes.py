@@ -188,6 +188,28 @@ def test_batchnorm_train_any_plane(n, c, hw, rocm_device):
             close(a, b, 1e-5, 1e-5, f"[{n}, {c}, {hw}] shift {shift} {name}")
 
 
+@pytest.mark.parametrize("n", [1, 3])
+def test_batchnorm_train_infinity_in_the_first_split(n, rocm_device):
+    """An infinite value gives an infinite channel mean where the merges
+    inside a workgroup keep it (it comes last in their order; in any other
+    place Chan's formula meets inf - inf), and NaN elsewhere, never a finite
+    one: the merge of the splits loses neither, also for the first split.  256
+    channels have it in one each of a workgroup's 256 threads, in the first
+    plane."""
+    import hip_oracles
+    c, hw = 256, 50001
+    x = torch.randn(n, c, 1, hw, device=rocm_device)
+    for t in range(c):  # vector 12032 + t: thread t's, the last one for t > 212
+        x[0, t, 0, 4 * (12032 + t)] = float("inf")
+    rm, rv = torch.zeros(c, device=rocm_device), torch.ones(c, device=rocm_device)
+    y, mean, invstd = hip_oracles.batchnorm_train(
+        x, torch.ones_like(rm), torch.zeros_like(rm), rm, rv, momentum=0.1, eps=1e-5, relu=False)
+    assert not bool(torch.isfinite(mean).any())
+    assert bool((mean == float("inf")).any())
+    assert bool(((rm == float("inf")) == (mean == float("inf"))).all())
+    assert bool(torch.isnan(invstd).all()) and bool(torch.isnan(rv).all())
+
+
 # One group, one value more and less; the ends of the lane counts and of the
 # short-row kernels (512, 1536); several waves and groups per row; value by
 # value (below 8).
