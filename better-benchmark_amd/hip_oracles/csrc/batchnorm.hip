@@ -116,14 +116,12 @@ __device__ __forceinline__ void split_range(int64_t N, int64_t S, int64_t s,
   n1 = (N * (s + 1)) / S;
 }
 
-// Merge the threads' triples: DPP across the wave, then the waves' triples,
-// through LDS, by the same butterflies in every wave (4 or 16 waves: two or
-// four steps), of which lane 0's order counts.  Every thread returns the
-// workgroup's total.
-template <int T = kThreads>
+// Merge the threads' triples: DPP across the wave, then the four waves'
+// triples, through LDS, by the same butterflies in every wave, of which lane
+// 0's order counts.  Every thread returns the workgroup's total.
 __device__ __forceinline__ Welford block_welford(Welford acc) {
-  constexpr int kWaves = T / kWave;
-  static_assert(kWaves == 4 || kWaves == 16, "the waves' triples fill quads or rows");
+  constexpr int kWaves = kThreads / kWave;
+  static_assert(kWaves == 4, "the waves' triples fill quads");
   acc = wave_welford(acc);
   __shared__ Welford part[kWaves];
   const int wave = threadIdx.x >> 6;
@@ -132,12 +130,38 @@ __device__ __forceinline__ Welford block_welford(Welford acc) {
   Welford w = part[threadIdx.x & (kWaves - 1)];
   w = welford_merge(w, welford_dpp<kDppQuadXor1>(w));
   w = welford_merge(w, welford_dpp<kDppQuadXor2>(w));
-  if constexpr (kWaves == 16) {
-    w = welford_merge(w, welford_dpp<kDppRowRor4>(w));
-    w = welford_merge(w, welford_dpp<kDppRowRor8>(w));
-  }
   return welford_lane(w, 0);
 }
+
+// Triples (n_s, mean_s, M2_s) merged in fp64 about a shift K, one of the means
+// (shift_of it: 0 where it is not finite, for mean_s - K of an infinite one
+// would be NaN): with d_s = mean_s - K, S1 = sum n_s d_s and S2 = sum M2_s +
+// n_s d_s^2, mean = K + S1 / N and M2 = S2 - S1^2 / N.  Each lane add()s its
+// triples in order; total() adds the lanes by wave_sum (a fixed order; all 64
+// lanes active, every lane gets the result).
+struct ChannelStats {
+  double mean, m2, count;
+};
+
+__device__ __forceinline__ double shift_of(float mean) {
+  return __builtin_isfinite(mean) ? static_cast<double>(mean) : 0.0;
+}
+
+struct ShiftedSums {
+  double K, n, s1, s2;
+  __device__ __forceinline__ void add(float nb, float mean, float m2) {
+    const double d = static_cast<double>(mean) - K;
+    n += nb;
+    s1 = __builtin_fma(static_cast<double>(nb), d, s1);
+    s2 += __builtin_fma(nb * d, d, static_cast<double>(m2));
+  }
+  __device__ __forceinline__ ChannelStats total() const {
+    const double N = wave_sum(n), a = wave_sum(s1), b = wave_sum(s2);
+    const double dm = a / N;
+    // max (NaN from the data kept): rounding can leave a tiny negative.
+    return ChannelStats{K + dm, __builtin_elementwise_maximum(b - a * dm, 0.0), N};
+  }
+};
 
 // Planes of HW >= 4 values, any alignment, as F = ceil(HW / 4) vectors each:
 // vector j of a plane starts at value min(4 j, HW - 4), so the last one of a
@@ -228,32 +252,14 @@ __global__ __launch_bounds__(kThreads) void bn_partial_stats(
   }
 }
 
-// Merge the S partial triples of channel c in fp64 about the first one's
-// mean K (0 where that is not finite: mean_s - K of an infinite one would be
-// NaN): with d_s = mean_s - K, S1 = sum n_s d_s and S2 = sum M2_s + n_s
-// d_s^2, mean = K + S1 / N and M2 = S2 - S1^2 / N.  One wave: lane l adds
-// splits l, l + 64, ... in order, then wave_sum (a fixed order).  All 64
-// lanes active; every lane returns the result.
-__device__ void channel_stats(const float* __restrict__ ws, int64_t c,
-                              int64_t S, double& mean, double& m2,
-                              double& count) {
+// The S partial triples of channel c merged about the first one's mean, lane
+// l adding splits l, l + 64, ... .
+__device__ ChannelStats channel_stats(const float* __restrict__ ws, int64_t c, int64_t S) {
   const float* p = ws + c * S * 3;
-  const double K = __builtin_isfinite(p[1]) ? p[1] : 0.f;
-  double n = 0.0, s1 = 0.0, s2 = 0.0;
-  for (int64_t s = threadIdx.x & (kWave - 1); s < S; s += kWave) {
-    const double nb = p[3 * s], d = static_cast<double>(p[3 * s + 1]) - K;
-    n += nb;
-    s1 = __builtin_fma(nb, d, s1);
-    s2 += __builtin_fma(nb * d, d, static_cast<double>(p[3 * s + 2]));
-  }
-  n = wave_sum(n);
-  s1 = wave_sum(s1);
-  s2 = wave_sum(s2);
-  const double dm = s1 / n;
-  mean = K + dm;
-  // max (NaN from the data kept): rounding can leave a tiny negative.
-  m2 = __builtin_elementwise_maximum(s2 - s1 * dm, 0.0);
-  count = n;
+  ShiftedSums sums{shift_of(p[1]), 0.0, 0.0, 0.0};
+  for (int64_t s = threadIdx.x & (kWave - 1); s < S; s += kWave)
+    sums.add(p[3 * s], p[3 * s + 1], p[3 * s + 2]);
+  return sums.total();
 }
 
 // mean / invstd from the merged (mean, M2, count) of channel c -> the
@@ -347,10 +353,9 @@ __global__ __launch_bounds__(kThreads) void bn_normalize(
   const int64_t s = bid - c * S;
   __shared__ float coef[2];
   if (threadIdx.x < kWave) {
-    double mean, m2, count;
-    channel_stats(ws, c, S, mean, m2, count);
+    const ChannelStats t = channel_stats(ws, c, S);
     if (threadIdx.x == 0)
-      channel_coefs(mean, m2, count, c, gamma, beta, running_mean, running_var, save_mean,
+      channel_coefs(t.mean, t.m2, t.count, c, gamma, beta, running_mean, running_var, save_mean,
                     save_invstd, momentum, eps, s == 0, coef);
   }
   __syncthreads();
@@ -455,11 +460,32 @@ __global__ __launch_bounds__(T) void bn_channel_small(
   } else {
     absorb<U>(acc, v, ok);
   }
-  const Welford t = block_welford<T>(acc);
   __shared__ float coef[2];
+  ChannelStats t;
+  if constexpr (T == kThreads) {
+    const Welford w = block_welford(acc);
+    t = ChannelStats{static_cast<double>(w.mean), static_cast<double>(w.m2),
+                     static_cast<double>(w.n)};
+  } else {
+    // The 16 waves' triples in fp64 by the first wave, as the split-K path
+    // merges its splits (fp32 merges left the mean up to an ulp and a half
+    // off, and the running statistics with it).
+    constexpr int kWaves = T / kWave;
+    __shared__ Welford part[kWaves];
+    acc = wave_welford(acc);
+    if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x < kWave) {
+      ShiftedSums sums{shift_of(part[0].mean), 0.0, 0.0, 0.0};
+      if (threadIdx.x < kWaves) {
+        const Welford w = part[threadIdx.x];
+        sums.add(w.n, w.mean, w.m2);
+      }
+      t = sums.total();
+    }
+  }
   if (threadIdx.x == 0)
-    channel_coefs_of(static_cast<double>(t.mean), static_cast<double>(t.m2),
-                     static_cast<double>(t.n), c, pg, pb, prm, prv, running_mean, running_var,
+    channel_coefs_of(t.mean, t.m2, t.count, c, pg, pb, prm, prv, running_mean, running_var,
                      save_mean, save_invstd, momentum, eps, true, coef);
   __syncthreads();
   const float alpha = coef[0], shift = coef[1];

@@ -188,6 +188,36 @@ def test_batchnorm_train_any_plane(n, c, hw, rocm_device):
             close(a, b, 1e-5, 1e-5, f"[{n}, {c}, {hw}] shift {shift} {name}")
 
 
+@pytest.mark.parametrize("hw", [28672, 28671], ids=["whole", "ragged"])
+def test_batchnorm_train_large_channels_merge_in_fp64(hw, rocm_device):
+    """The 1024-thread register kernel: each of its 16 waves (wave w holds the
+    float4s i with i % 1024 // 64 == w) sees one 18-bit value only, so its sum,
+    its mean and its merge over the lanes are exact and the waves' fp64 merge
+    is the one that rounds: every statistic is the fp64 one rounded to fp32."""
+    import hip_oracles
+    import numpy as np
+    c = 64
+    g = torch.Generator().manual_seed(7)
+    per_wave = (torch.randint(1 << 17, 1 << 18, (c, 16), generator=g).double()
+                * 2.0 ** torch.randint(-20, -8, (c, 16), generator=g).double()
+                * (torch.randint(0, 2, (c, 16), generator=g) * 2 - 1))
+    wave = torch.arange(hw) // 4 % 1024 // 64
+    x = per_wave[:, wave].float().view(1, c, 1, hw)
+    assert torch.equal(x.double().view(c, hw), per_wave[:, wave])
+    rm, rv = torch.zeros(c, device=rocm_device), torch.zeros(c, device=rocm_device)
+    ones = torch.ones(c, device=rocm_device)
+    _, mean, invstd = hip_oracles.batchnorm_train(x.to(rocm_device), ones, rm.clone(), rm, rv,
+                                                  momentum=0.5, eps=1e-5, relu=False)
+    x64 = x.double().view(c, hw).numpy()
+    mean64, var64 = x64.mean(1), x64.var(1)
+    assert np.array_equal(mean.cpu().numpy(), mean64.astype(np.float32))
+    assert np.array_equal(rm.cpu().numpy(), (0.5 * mean64).astype(np.float32))
+    assert np.array_equal(rv.cpu().numpy(), (0.5 * var64 * hw / (hw - 1)).astype(np.float32))
+    # var and var + eps rounded to fp32, then one square root and one division
+    want = 1 / np.sqrt(var64.astype(np.float32) + np.float32(1e-5))
+    assert np.abs(invstd.cpu().numpy() / want - 1).max() < 2.0 ** -22
+
+
 @pytest.mark.parametrize("n", [1, 3])
 def test_batchnorm_train_infinity_in_the_first_split(n, rocm_device):
     """An infinite value gives an infinite channel mean where the merges
