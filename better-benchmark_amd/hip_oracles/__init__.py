@@ -299,15 +299,40 @@ def scaled_masked_softmax(x: torch.Tensor, mask: torch.Tensor, scale: float) -> 
     return out
 
 
-# bf16 zeros [K] per (device, K): the mask row of softmax_lastdim.
-_zero_rows: dict = {}
+# One row of bf16 zeros per device, the mask of softmax_lastdim: every row held
+# in registers fits its 32768 values, a longer K replaces it by one of the next
+# power of two.  Rows that were replaced are kept (calls in flight and captured
+# graphs read them; all together they are shorter than the last).
+_zero_rows: dict = {}  # device index -> the row in use
+_old_zero_rows: list = []
+_zero_row_lock = threading.Lock()
+
+
+def _zero_row(dev: torch.device, k: int) -> torch.Tensor:
+    row = _zero_rows.get(dev.index)
+    if row is not None and row.numel() >= k:
+        return row
+    with _zero_row_lock:
+        row = _zero_rows.get(dev.index)
+        if row is None or row.numel() < k:
+            _require(not torch.cuda.is_current_stream_capturing(),
+                     "softmax: the first call on a device, and the first for a longer row than "
+                     "any before (from 32768 on), must run outside graph capture")
+            new = torch.zeros(max(32768, 1 << (k - 1).bit_length()), dtype=torch.bfloat16,
+                              device=dev)
+            # Other streams and threads use it from here on.
+            torch.cuda.current_stream(dev).synchronize()
+            if row is not None:
+                _old_zero_rows.append(row)
+            row = _zero_rows[dev.index] = new
+    return row
 
 
 def softmax_lastdim(x: torch.Tensor) -> torch.Tensor:
     """softmax(x, -1) of a contiguous bf16 tensor (fp32 max, exp, sum and
     division, bf16 out): hipo_scaled_masked_softmax_bf16 over [rows, 1, K]
     with scale 1 and one zero mask row (s = fma(x, 1, 0) = x exactly).  The
-    zero row is allocated on a device's first call with that K, which
+    zero row is made, and waited for, in a device's first call, which
     therefore must not be inside a graph capture."""
     lib = _lib or load_library()
     dev = _require_rocm(x)
@@ -317,14 +342,8 @@ def softmax_lastdim(x: torch.Tensor) -> torch.Tensor:
     out = torch.empty_like(x)
     if x.numel() == 0:
         return out
-    key = (dev.index, k)
-    zero = _zero_rows.get(key)
-    if zero is None:
-        _require(not torch.cuda.is_current_stream_capturing(),
-                 "softmax: the first call for this K must run outside graph capture")
-        zero = _zero_rows[key] = torch.zeros(k, dtype=torch.bfloat16, device=dev)
-    _call(lib.hipo_scaled_masked_softmax_bf16, "softmax_lastdim", dev, _ptr(x), _ptr(zero),
-          _ptr(out), x.numel() // k, 1, k, k, 1.0)
+    _call(lib.hipo_scaled_masked_softmax_bf16, "softmax_lastdim", dev, _ptr(x),
+          _ptr(_zero_row(dev, k)), _ptr(out), x.numel() // k, 1, k, k, 1.0)
     return out
 
 

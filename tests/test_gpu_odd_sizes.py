@@ -104,6 +104,40 @@ def test_softmax_odd_rows_special_values(k, rocm_device):
         close(got[r], want[r], 2 ** -7, 1e-6, f"row {r}")
 
 
+def test_softmax_zero_row_is_one_and_ready_for_every_stream(rocm_device, monkeypatch):
+    """softmax_lastdim's mask row: one per device whatever row lengths come,
+    filled before any other stream can use it (the first call waits for the
+    stream that fills it, here behind other work), longer ones on demand."""
+    import hip_oracles
+    monkeypatch.setattr(hip_oracles, "_zero_rows", {})
+    monkeypatch.setattr(hip_oracles, "_old_zero_rows", [])
+    x = torch.randn(64, 500).to(torch.bfloat16).to(rocm_device)
+    want = torch.softmax(x.double(), -1).to(torch.bfloat16).float().cpu()
+    a = torch.randn(4096, 4096, device=rocm_device)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream(rocm_device)
+    with torch.cuda.stream(side):
+        for _ in range(8):
+            a = a @ a
+            a = a / a.abs().max()
+        event = torch.cuda.Event()
+        event.record()
+        first = hip_oracles.softmax_lastdim(x)
+    assert event.query(), "the zero row was published before it was filled"
+    close(hip_oracles.softmax_lastdim(x), want, 2 ** -7, 1e-6, "another stream")
+    torch.cuda.synchronize()
+    close(first, want, 2 ** -7, 1e-6, "the filling stream")
+    for k in (1, 7, 197, 32768):
+        hip_oracles.softmax_lastdim(torch.zeros(2, k, dtype=torch.bfloat16, device=rocm_device))
+    assert [r.numel() for r in hip_oracles._zero_rows.values()] == [32768]
+    assert not hip_oracles._old_zero_rows
+    x = torch.randn(2, 33000).to(torch.bfloat16)
+    close(hip_oracles.softmax_lastdim(x.to(rocm_device)),
+          torch.softmax(x.double(), -1).to(torch.bfloat16).float(), 2 ** -7, 1e-6, "33000")
+    assert [r.numel() for r in hip_oracles._zero_rows.values()] == [65536]
+    assert [r.numel() for r in hip_oracles._old_zero_rows] == [32768]
+
+
 # (channels, positions): one block each way, one value more, odd planes, more
 # block columns than a tile's 8 and fewer rows, thin output rows, fewer values
 # than a block (the one-element kernel).  n fills the tile kernel's minimum.
