@@ -211,7 +211,9 @@ __global__ __launch_bounds__(256) void spatial_mean_finish(
   out[i] = static_cast<uint16_t>(pack_bf16x2(sum / static_cast<float>(P), 0.f) & 0xffffu);
 }
 
-// C < 8: one thread per (n, c), strided loads.
+// One thread per (n, c), strided loads: C < 8, ragged images too small to fill
+// workgroups (spatial_thread_per_output), and whole rows of more than 8192
+// channels, which spatial_plan does not take.
 __global__ __launch_bounds__(256) void spatial_mean_nhwc_scalar(
     const uint16_t* __restrict__ x, uint16_t* __restrict__ out, int64_t N,
     int64_t P, int64_t C) {
@@ -328,6 +330,23 @@ SpatialPlan ragged_plan(int64_t n, int64_t p, int64_t c) {
   return plan;
 }
 
+// Whether a thread per (n, c) is faster than the ragged plan: a workgroup
+// costs its dispatch however few threads a narrow image gives it.  Estimates
+// in us of both, from graph replays over C 9..1001, planes of 1 to 196
+// positions and 64 to 32768 images; of those 288 points three come out over
+// 4 % slower than the better of the two (none above 1.3 times).  Measured,
+// ragged plan / thread per output: [32768, 9, 1, 1] 13.6 / 2.9, [32768, 12, 3,
+// 3] 21.3 / 4.5, [512, 100, 4, 4] 4.8 / 3.9, [32768, 12, 7, 7] 27.5 / 17.9;
+// [4096, 100, 4, 4] 6.9 / 7.9, [4096, 20, 7, 7] 6.7 / 15.8.
+bool spatial_thread_per_output(const SpatialPlan& plan, int64_t n, int64_t p, int64_t c) {
+  const double outs = static_cast<double>(n) * static_cast<double>(c);
+  const double positions = static_cast<double>(p);
+  const double blocks = static_cast<double>(n) * plan.cblocks;
+  const double threads_us = outs * (1.5e-6 + 0.6e-6 * positions) + 0.08 * positions;
+  const double blocks_us = p <= 4 ? 0.6 + 0.4e-3 * blocks : 1.9 + 0.6e-3 * blocks;
+  return threads_us < blocks_us;
+}
+
 // The small-image kernel's loads per lane (ceil(P / 8)), or 0 where it
 // does not apply: C a multiple of 64, P <= 224, and at least 512 waves (two
 // per CU) of (image, 64-channel block).
@@ -392,7 +411,7 @@ extern "C" int hipo_spatial_mean_nhwc_bf16(const uint16_t* x, uint16_t* out, int
   }
   const bool whole = c % 8 == 0 && aligned16(x) && aligned16(out);
   const SpatialPlan plan = whole ? spatial_plan(n, hw, c) : ragged_plan(n, hw, c);
-  if (plan.threads > 0) {
+  if (plan.threads > 0 && (whole || !spatial_thread_per_output(plan, n, hw, c))) {
     const size_t need = plan.slices > 1 ? static_cast<size_t>(n * plan.slices * c) * 4 : 0;
     HIPO_REQUIRE(workspace_bytes >= need && (need == 0 || workspace != nullptr),
                  "spatial_mean: workspace of %zu bytes, need %zu", workspace_bytes, need);

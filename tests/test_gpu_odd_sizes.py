@@ -328,7 +328,9 @@ def test_norms_any_row_length(cols, rocm_device):
 # (n, c, hw): one group, one channel more and less, channel counts over several
 # blocks of groups, one position, fewer positions than rows per instruction.
 SPATIAL = [(2, 7, 9), (2, 8, 9), (3, 9, 1), (3, 15, 49), (4, 29, 3190), (2, 61, 700), (130, 1001, 49),
-           (6, 1759, 196), (1, 514, 50), (2, 8193, 4), (300, 33, 100)]
+           (6, 1759, 196), (1, 514, 50), (2, 8193, 4), (300, 33, 100),
+           # ragged plan and thread per output, on both sides of the line
+           (2100, 500, 1), (3000, 9, 4), (1500, 250, 9), (600, 250, 9), (2, 8200, 7)]
 
 
 @pytest.mark.parametrize("n,c,hw", SPATIAL)
