@@ -119,16 +119,18 @@ __global__ __launch_bounds__(256) void row_mean_f32_scalar(
 
 // bf16 rows, fp32 accumulation, optional ReLU (NaN kept):
 //   out[r] = bf16(sum_j act(x[r, j]) / cols)   (one rounding, nearest even).
-// Short rows (cols <= 512, contiguous, 16-byte aligned x): each wave takes 8
+// Short rows (cols <= 512, contiguous): each wave takes 8
 // consecutive rows -- 16 * cols bytes, a whole number of 16-byte vectors
 // whatever cols is, so the input is read as one flat stream of non-temporal
 // vector loads (the SqueezeNet rows are 169 elements, 338 bytes, not
-// vector-aligned one by one).  The wave stages its 8 rows in LDS; then 8
+// vector-aligned one by one), element-aligned ones (ALIGNED false) where x is
+// off 16 bytes.  The wave stages its 8 rows in LDS; then 8
 // lanes per row sum every 8th element in order and combine in a fixed
-// DPP butterfly.  Longer rows: one wave per row.
+// DPP butterfly.
 constexpr int kBf16RowsPerWave = 8;
 constexpr int kBf16ShortCols = 512;
 constexpr int kBf16Waves = 4;
+constexpr int64_t kBf16ShortRows = 24000;  // from here on also off alignment
 
 template <bool RELU>
 __device__ __forceinline__ float act_relu(float v) {
@@ -139,7 +141,7 @@ __device__ __forceinline__ uint16_t round_to_bf16(float v) {
   return static_cast<uint16_t>(pack_bf16x2(v, 0.0f) & 0xffffu);
 }
 
-template <bool RELU, int VPL>
+template <bool RELU, int VPL, bool ALIGNED>
 __global__ __launch_bounds__(kBf16Waves * kWave) void row_mean_bf16_short(
     const uint16_t* __restrict__ x, uint16_t* __restrict__ out, int64_t rows, int cols) {
   __shared__ __align__(16) uint16_t stage[kBf16Waves][kBf16RowsPerWave * kBf16ShortCols];
@@ -161,7 +163,11 @@ __global__ __launch_bounds__(kBf16Waves * kWave) void row_mean_bf16_short(
 #pragma unroll
       for (int k = 0; k < VPL; ++k) {
         const int i = lane + k * kWave;
-        v[k] = __builtin_nontemporal_load(xv + (i < whole ? i : whole - 1));
+        if constexpr (ALIGNED) {
+          v[k] = __builtin_nontemporal_load(xv + (i < whole ? i : whole - 1));
+        } else {
+          v[k] = ragged_load_stream(x + row0 * cols + (i < whole ? i : whole - 1) * 8);
+        }
       }
 #pragma unroll
       for (int k = 0; k < VPL; ++k) {
@@ -185,12 +191,40 @@ __global__ __launch_bounds__(kBf16Waves * kWave) void row_mean_bf16_short(
   if (k == 0 && r < nrows) out[row0 + r] = round_to_bf16(s / static_cast<float>(cols));
 }
 
-// Longer rows, and short ones off 16-byte alignment, cols >= 8: W waves per
-// row as in row_mean_f32_vec4, U 16-byte loads per lane in flight; RAGGED: any
-// length and alignment, the row's last group moved back to end with it
-// (RaggedGroup), element-aligned cached loads.  Against one wave per row with
-// one load in flight, graph replays: [2000, 16001] 74.5 -> 12.0 us, [20, 16000]
-// 7.0 -> 3.0, [16000, 777] 10.7 -> 6.3, [8000, 4096] 11.7 -> 11.8.
+// A wave per row, one load per lane in flight: many whole rows that would leave
+// much of the kernel below's loads past their ends (VEC: 16-byte loads), and
+// short ones off 16-byte alignment (single values); see the entry point.
+template <bool RELU, bool VEC>
+__global__ __launch_bounds__(kBf16Waves * kWave) void row_mean_bf16_wave(
+    const uint16_t* __restrict__ x, uint16_t* __restrict__ out, int64_t rows, int64_t cols) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * kBf16Waves + (threadIdx.x >> 6);
+  if (row >= rows) return;  // wave-uniform; no barrier follows
+  const uint16_t* xr = x + row * cols;
+  float acc = 0.0f;
+  if constexpr (VEC) {
+    const u32x4_t* p = reinterpret_cast<const u32x4_t*>(xr);
+    for (int64_t i = lane; i < cols / kRowGroup; i += kWave) {
+      const u32x4_t v = __builtin_nontemporal_load(p + i);
+      float t = 0.0f;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        t += act_relu<RELU>(bf16lo(v[d])) + act_relu<RELU>(bf16hi(v[d]));
+      acc += t;
+    }
+  } else {
+    for (int64_t i = lane; i < cols; i += kWave) acc += act_relu<RELU>(bf16_to_f32(xr[i]));
+  }
+  const float s = wave_sum(acc);
+  if (lane == 0) out[row] = round_to_bf16(s / static_cast<float>(cols));
+}
+
+// Longer rows: W waves per row as in row_mean_f32_vec4, U 16-byte loads per
+// lane in flight; RAGGED: any length >= 8 and alignment, the row's last group
+// moved back to end with it (RaggedGroup), element-aligned cached loads.
+// Against one wave per row with one load in flight, graph replays: [2000, 16001]
+// 74.5 -> 12.0 us, [20, 16000] 7.0 -> 3.0, [16000, 777] 10.7 -> 6.3, [8000, 4096]
+// 11.7 -> 11.8.
 template <bool RELU, int U, bool RAGGED>
 __global__ __launch_bounds__(kMaxThreads) void row_mean_bf16_rows(
     const uint16_t* __restrict__ x, uint16_t* __restrict__ out, int64_t rows, int64_t cols,
@@ -318,46 +352,70 @@ extern "C" int hipo_row_mean_bf16(const uint16_t* x, uint16_t* out, int64_t rows
   HIPO_REQUIRE(cols > 0, "row_mean_bf16: mean over zero elements");
   HIPO_REQUIRE(x != nullptr && out != nullptr, "row_mean_bf16: null pointer");
   const bool act = relu != 0;
-  if (cols <= kBf16ShortCols && aligned16(x)) {
-    const int64_t groups = (rows + kBf16RowsPerWave - 1) / kBf16RowsPerWave;
-    const int64_t blocks = (groups + kBf16Waves - 1) / kBf16Waves;
+  const bool aligned = aligned16(x);
+  const bool ragged = cols % 8 != 0 || !aligned;
+  const auto blocks_of = [&](int64_t rows_per_block) {
+    return (rows + rows_per_block - 1) / rows_per_block;
+  };
+  // Rows of up to 512 values off 16-byte alignment, us, a wave per row by single
+  // values / the short-row kernel / the rows kernel with one load: [10000, 100]
+  // 3.3 / 3.9 / 4.2, [100000, 100] 15.6 / 10.3 / 20.0, [100000, 256] 23.8 / 16.2
+  // / 20.3, [10000, 400] 6.5 / 7.9 / 4.8, [100000, 400] 35.1 / 23.7 / 20.2; the
+  // short-row kernel passes the first at about 24000 rows.
+  const bool off_short = !aligned && cols >= kRowGroup && cols <= 256;
+  // Whole longer rows: the rows kernel holds `held` values a row, in one sweep
+  // of 2 loads a lane or several of 4.
+  const int waves = static_cast<int>(
+      std::min<int64_t>(kMaxWaves, (cols + 2 * kRowSweep - 1) / (2 * kRowSweep)));
+  const bool two = cols <= int64_t{waves} * 2 * kRowSweep;
+  const int64_t sweep = int64_t{waves} * (two ? 2 : 4) * kRowSweep;
+  const int64_t held = (cols + sweep - 1) / sweep * sweep;
+  // With many rows a wave per row is faster where the row fills under 85 % of
+  // that (60 % where one wave holds it or in several sweeps), us, wave / rows
+  // kernel: [50000, 520] 13.8 / 14.9, [50000, 776] 16.9 / 15.5, [50000, 1032]
+  // 22.0 / 27.1, [16000, 1536] 9.5 / 10.9, [16000, 1736] 11.5 / 11.0, [8000,
+  // 2056] 7.8 / 9.4, [8000, 4104] 12.7 / 13.8, [8000, 4096] 12.1 / 12.0, [4096,
+  // 8200] 15.0 / 16.6, [4096, 12000] 21.2 / 19.6; fewer rows, [1024, 2056] 4.5 /
+  // 3.8, [3000, 1032] 3.8 / 4.4, [3000, 3080] 6.6 / 6.0.
+  const bool wave_rows = !ragged && rows >= (waves <= 2 ? 2560 : 4096) &&
+                         cols * 20 < held * (waves > 1 && two ? 17 : 12);
+  if (cols <= kBf16ShortCols && (aligned || (off_short && rows >= kBf16ShortRows))) {
+    const int64_t blocks = blocks_of(kBf16Waves * kBf16RowsPerWave);
     HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
-    const dim3 grid(static_cast<unsigned>(blocks)), block(kBf16Waves * kWave);
-    const int c = static_cast<int>(cols);
     // cols vectors of 16 bytes per wave: ceil(cols / 64) per lane.
-#define HIPO_RMB(V_)                                                                    \
-  (act ? row_mean_bf16_short<true, V_><<<grid, block, 0, stream>>>(x, out, rows, c)     \
-       : row_mean_bf16_short<false, V_><<<grid, block, 0, stream>>>(x, out, rows, c))
-    if (cols <= 2 * kWave) {
-      HIPO_RMB(2);
-    } else if (cols <= 4 * kWave) {
-      HIPO_RMB(4);
-    } else {
-      HIPO_RMB(8);
-    }
+#define HIPO_RMB(V_)                                                                          \
+  (act ? (aligned ? row_mean_bf16_short<true, V_, true> : row_mean_bf16_short<true, V_, false>) \
+       : (aligned ? row_mean_bf16_short<false, V_, true> : row_mean_bf16_short<false, V_, false>))
+    auto kernel = cols <= 2 * kWave ? HIPO_RMB(2) : cols <= 4 * kWave ? HIPO_RMB(4) : HIPO_RMB(8);
 #undef HIPO_RMB
+    kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kBf16Waves * kWave), 0, stream>>>(
+        x, out, rows, static_cast<int>(cols));
+  } else if (cols < kRowGroup) {
+    const int64_t blocks = blocks_of(256);
+    HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
+    auto kernel = act ? row_mean_bf16_scalar<true> : row_mean_bf16_scalar<false>;
+    kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(x, out, rows, cols);
+  } else if (off_short || wave_rows) {
+    const int64_t blocks = blocks_of(kBf16Waves);
+    HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
+#define HIPO_RMB(VEC_) (act ? row_mean_bf16_wave<true, VEC_> : row_mean_bf16_wave<false, VEC_>)
+    auto kernel = wave_rows ? HIPO_RMB(true) : HIPO_RMB(false);
+#undef HIPO_RMB
+    kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kBf16Waves * kWave), 0, stream>>>(
+        x, out, rows, cols);
   } else {
-    if (cols >= kRowGroup) {
-      const int waves = static_cast<int>(
-          std::min<int64_t>(kMaxWaves, (cols + 2 * kRowSweep - 1) / (2 * kRowSweep)));
-      const int rpb = kMaxWaves / waves;
-      const int64_t blocks = (rows + rpb - 1) / rpb;
-      HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
-      const bool ragged = cols % 8 != 0 || !aligned16(x);
-      const bool two = cols <= int64_t{waves} * 2 * kRowSweep;  // one sweep of 2 loads
-#define HIPO_RMB(ACT_)                                                                \
-  (two ? (ragged ? row_mean_bf16_rows<ACT_, 2, true> : row_mean_bf16_rows<ACT_, 2, false>) \
-       : (ragged ? row_mean_bf16_rows<ACT_, 4, true> : row_mean_bf16_rows<ACT_, 4, false>))
-      auto kernel = act ? HIPO_RMB(true) : HIPO_RMB(false);
+    const bool one = cols <= kRowSweep;
+    const int rpb = (one ? kBf16Waves : kMaxWaves) / waves;
+    const int64_t blocks = blocks_of(rpb);
+    HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
+#define HIPO_RMB(ACT_)                                                                     \
+  (one   ? row_mean_bf16_rows<ACT_, 1, true>                                               \
+   : two ? (ragged ? row_mean_bf16_rows<ACT_, 2, true> : row_mean_bf16_rows<ACT_, 2, false>) \
+         : (ragged ? row_mean_bf16_rows<ACT_, 4, true> : row_mean_bf16_rows<ACT_, 4, false>))
+    auto kernel = act ? HIPO_RMB(true) : HIPO_RMB(false);
 #undef HIPO_RMB
-      kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(waves * rpb * kWave), 0, stream>>>(
-          x, out, rows, cols, waves, rpb);
-    } else {
-      const int64_t blocks = (rows + 255) / 256;
-      HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
-      auto kernel = act ? row_mean_bf16_scalar<true> : row_mean_bf16_scalar<false>;
-      kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(x, out, rows, cols);
-    }
+    kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(waves * rpb * kWave), 0, stream>>>(
+        x, out, rows, cols, waves, rpb);
   }
   return check_launch("row_mean_bf16");
 }

@@ -477,3 +477,25 @@ def test_row_mean_any_row_length(cols, rocm_device):
             torch.cuda.synchronize()
             out.check(f"bf16 {cols}")
             close(out.t, ref.row_mean_bf16(xb, relu=bool(relu)), 2 ** -7, 1e-5, f"bf16 {cols}")
+
+
+# (rows, cols, elements off alignment): both sides of the lines where short
+# rows off alignment leave the wave per row for the short-row kernel (24000
+# rows, up to 256 values), and whole longer ones the several waves per row for
+# one (2560 and 4096 rows); partial last workgroups.
+@pytest.mark.parametrize("rows,cols,shift", [
+    (23999, 256, 1), (24000, 256, 1), (24013, 9, 3), (24001, 257, 1), (70, 400, 1), (9, 512, 5),
+    (2559, 520, 0), (2560, 520, 0), (2563, 1032, 0), (4095, 2056, 0), (4097, 2056, 0),
+    (4099, 4104, 0), (4097, 8200, 0), (2561, 1024, 0)])
+def test_row_mean_bf16_many_rows(rows, cols, shift, rocm_device):
+    """One rounding of an fp32 mean: one ulp, 2^-7, and 1e-5 near zero."""
+    import oracle as ref
+    torch.manual_seed(rows + cols)
+    x = torch.randn(rows, cols).to(torch.bfloat16)
+    xd = place(x, rocm_device, shift)
+    for relu in (0, 1):
+        out = Guarded((rows,), torch.bfloat16, rocm_device)
+        ok(lib().hipo_row_mean_bf16(xd.data_ptr(), out.t.data_ptr(), rows, cols, relu, None))
+        torch.cuda.synchronize()
+        out.check(f"[{rows}, {cols}]")
+        close(out.t, ref.row_mean_bf16(x, relu=bool(relu)), 2 ** -7, 1e-5, f"[{rows}, {cols}]")
