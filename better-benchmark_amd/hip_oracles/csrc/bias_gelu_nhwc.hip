@@ -23,7 +23,8 @@
 // multiples of 8, [128, 512, 28, 28] 49.8 -> 38.7, [128, 256, 28, 28] 27.6 ->
 // 17.8, [128, 16, 112, 112] 48 -> 20 ([128, 256, 56, 56] 70 either way).  What is left at 14 x 14
 // (floor 5.8 us) is arithmetic: about 23 issue slots per value.
-// Launches of at most 2^19 elements take the one-element-per-thread kernel.
+// Launches of at most 2^19 elements, and images of few values, take the
+// one-element-per-thread kernel.
 // HBM-bound: algorithmic bytes per element = 2 (read) + 2 (write).
 #include "block_tiles.h"
 #include "gelu_bf16.h"
@@ -90,6 +91,20 @@ __global__ __launch_bounds__(256) void bias_gelu_nchw_to_nhwc_scalar(
   }
 }
 
+// Whether the tiles beat a thread per element.  A wave maps 64 values a lane
+// one after the other, however few of its lanes own a block and however much
+// the last blocks overlap: estimates in us of both, from graph replays over 8
+// to 1000 channels, planes of 8 to 196 positions and 0.56 to 9 million elements
+// (of those 600 points the worst comes out 18 % slower than the better of the
+// two).  Measured, tiles / thread per element: [60000, 9, 3, 3] 91 / 18, [64,
+// 1000, 3, 3] 8.2 / 4.2, [3000, 64, 2, 5] 10.6 / 8.8, [2187, 16, 4, 4] 10.6 / 4.2,
+// [9375, 64, 3, 5] 25 / 30, [128, 512, 7, 7] 8.7 / 16.3.  Images of whole blocks
+// keep the tiles from kTileMinElems on unless their waves alone cost more.
+bool tiles_pay(const BlockTiles& t, int64_t elements, bool whole) {
+  const double tiles_us = (whole ? 0.0 : 3.6) + 1.7e-3 * t.waves;
+  return tiles_us < 3.05e-6 * static_cast<double>(elements);
+}
+
 }  // namespace
 }  // namespace hipo
 
@@ -111,7 +126,9 @@ extern "C" int hipo_bias_gelu_nchw_to_nhwc_bf16(const uint16_t* x,
   // [2, 256, 56, 56], where the tiles win).
   BlockTiles t;
   TileAccess access;
-  if (n * c * hw > kTileMinElems && block_tiles(x, out, n, c, hw, 2, t, access)) {
+  const bool whole = c % 8 == 0 && hw % 8 == 0 && aligned16(x) && aligned16(out);
+  if (n * c * hw > kTileMinElems && block_tiles(x, out, n, c, hw, 2, t, access) &&
+      tiles_pay(t, n * c * hw, whole)) {
     auto kernel = access == TileAccess::kCached
                       ? bias_gelu_nchw_to_nhwc_blocks<TileAccess::kCached>
                   : access == TileAccess::kStreamOut

@@ -140,7 +140,9 @@ def test_softmax_zero_row_is_one_and_ready_for_every_stream(rocm_device, monkeyp
 
 # (channels, positions): one block each way, one value more, odd planes, more
 # block columns than a tile's 8 and fewer rows, thin output rows, fewer values
-# than a block (the one-element kernel).  n fills the tile kernel's minimum.
+# than a block (the one-element kernel).  One image, and 2^19 and 2^21 elements:
+# past the tile kernel's minimum, and with enough ragged images for it to pay
+# (from 65 x 49 on; smaller images go one element per thread at every count).
 BIAS_GELU_CP = [(8, 8), (9, 8), (8, 9), (65, 49), (64, 196), (100, 25), (16, 1001), (230, 77),
                 (513, 17), (7, 500), (300, 7)]
 
@@ -150,7 +152,7 @@ def test_bias_gelu_any_plane(c, hw, rocm_device):
     """Both sides hold the correctly rounded bf16: equal bit for bit."""
     import oracle as ref
     torch.manual_seed(c * 1000 + hw)
-    for n in (1, (1 << 19) // (c * hw) + 2):
+    for n in (1, (1 << 19) // (c * hw) + 2, (1 << 21) // (c * hw) + 2):
         x = torch.randn(n, c, 1, hw).to(torch.bfloat16) * 3
         bias = torch.randn(c).to(torch.bfloat16)
         want = ref.bias_gelu_nchw_to_nhwc(x, bias).permute(0, 2, 3, 1)

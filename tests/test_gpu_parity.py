@@ -402,10 +402,9 @@ def test_bias_gelu_edges(rocm_device):
     assert_close(out[..., :4], want[..., :4], PROB_TOL, "gelu large |t|")
     assert out[0, 0, 0, 4].item() == float("inf") and math.isnan(out[0, 0, 0, 5].float().item())
     assert_close(out[..., 6:], want[..., 6:], PROB_TOL, "gelu +-0.5")
-    # shapes off the vector path (C % 8, HW % 8), small launches (the scalar
-    # kernel), partial channel groups and position tiles of the tile kernel;
-    # (65537, 8, 1, 8): more images than a grid's z dimension holds, so the
-    # tile kernel takes its 1-D numbering instead of the 3-D grid
+    # small launches (the scalar kernel), partial channel groups and position
+    # tiles of the tile kernel; (65537, 8, 1, 8): more images of one block each
+    # than a grid's z dimension holds (the scalar kernel)
     for shape in [(2, 5, 3, 3), (1, 264, 2, 4), (3, 16, 1, 8), (64, 264, 2, 32),
                   (1024, 16, 1, 40), (65537, 8, 1, 8)]:
         g = torch.Generator().manual_seed(sum(shape))
