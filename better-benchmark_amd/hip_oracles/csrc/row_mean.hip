@@ -293,8 +293,11 @@ extern "C" int hipo_row_mean_f32(const float* x, float* out, int64_t rows,
   // Rows off the vector path: one wave per row with 4-byte loads is as fast
   // where the rows alone fill the chip, and faster for short ones ([65536, 17]
   // 9.2 us against 11.2, [4000, 4097] 11.2 against 12.2); few long rows take
-  // several waves each ([24, 8707] 7.2 -> 3.1 us).
-  const bool ragged = !vec && cols >= kRaggedMinCols && rows < kRaggedMaxRows;
+  // several waves each ([24, 8707] 7.2 -> 3.1 us, [1536, 1537] 4.3 -> 4.1, [1920,
+  // 12001] 21.4 -> 16.4, but [2047, 1025] 3.6 -> 4.0, [1300, 1025] 3.4 -> 3.6).
+  const bool ragged = !vec && rows < kRaggedMaxRows &&
+                      cols >= (rows < kRaggedMaxRows / 2 ? kRaggedMinCols
+                                                         : kRaggedMinCols * 3 / 2);
   if (cols >= 4 && (vec || ragged)) {
     // About 2 KiB per wave: W = ceil(nvec / 128) waves per row (at most 8),
     // U = float4 per lane per sweep.

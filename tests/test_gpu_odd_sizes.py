@@ -501,3 +501,20 @@ def test_row_mean_bf16_many_rows(rows, cols, shift, rocm_device):
         torch.cuda.synchronize()
         out.check(f"[{rows}, {cols}]")
         close(out.t, ref.row_mean_bf16(x, relu=bool(relu)), 2 ** -7, 1e-5, f"[{rows}, {cols}]")
+
+
+# fp32 rows off the vector path: both sides of the lines between one wave and
+# several waves per row.
+@pytest.mark.parametrize("rows,cols", [(1023, 1025), (1024, 1025), (1024, 1535), (1025, 1537),
+                                       (2047, 1537), (2048, 1537), (1000, 1023)])
+def test_row_mean_f32_ragged_lines(rows, cols, rocm_device):
+    """fp32 sums in another order: 1e-5."""
+    import oracle as ref
+    torch.manual_seed(rows + cols)
+    x = torch.randn(rows, cols)
+    xd = place(x, rocm_device, 1)
+    out = Guarded((rows,), torch.float32, rocm_device)
+    ok(lib().hipo_row_mean_f32(xd.data_ptr(), out.t.data_ptr(), rows, cols, cols, None))
+    torch.cuda.synchronize()
+    out.check(f"[{rows}, {cols}]")
+    close(out.t, ref.row_mean(x), 1e-5, 1e-5, f"[{rows}, {cols}]")
