@@ -353,8 +353,9 @@ __global__ __launch_bounds__(256) void bn_nhwc_apply_pad_scalar(
 }
 
 // ---------------------------------------------------------------------------
-// NCHW, planes below 8 values of fewer than 8 channels (and grids past the
-// index range): a workgroup of kNchwImages waves covers a block of
+// NCHW, planes below 8 values of fewer than 8 channels, or few enough
+// (tiny_ragged_planes), and grids past the index range: a workgroup of
+// kNchwImages waves covers a block of
 // 64 channels (lane = channel) of kNchwImages consecutive images (wave =
 // image); each lane reads its channel's HW values from memory.
 // ---------------------------------------------------------------------------
@@ -467,8 +468,9 @@ __global__ __launch_bounds__(kNchwImages * kWave) void bn_nchw_small_hw(
 }
 
 // ---------------------------------------------------------------------------
-// NCHW with small planes (C >= 8, HW <= kPlanesMaxHw): a wave covers 8 consecutive channels of the kNchwImages images
-// of one slice -- per image, 8 consecutive H x W planes: 16 * HW bytes, a
+// NCHW with small planes (C >= 8, HW <= kPlanesMaxHw, but for
+// tiny_ragged_planes): a wave covers 8 consecutive channels of the kNchwImages
+// images of one slice -- per image, 8 consecutive H x W planes: 16 * HW bytes, a
 // whole number of 16-byte vectors whatever HW is.  The wave issues all its
 // non-temporal 16-byte loads at once, stages the planes in LDS, and reduces
 // each plane over 8 lanes (lane 8r + k takes elements k, k + 8, ... of plane
@@ -1100,6 +1102,18 @@ NhwcPlan nhwc_plan(int64_t M, int64_t C, bool vec_ok) {
 
 int64_t nchw_slices(int64_t n) { return (n + kNchwImages - 1) / kNchwImages; }
 
+// Planes of a few values, C not a multiple of 8 or x off 16-byte alignment, for
+// which a lane per channel is faster than a wave per 8 channels, whose few
+// hundred bytes do not pay for it; with many images the latter's merge of the
+// slices wins.  Graph replays in us, wave per 8 channels / lane per channel: [4,
+// 1071, 1, 1] 6.3 / 5.4, [58, 2113, 1, 1] 9.0 / 6.7, [129, 2113, 2, 2] 14.4 / 11.9,
+// [204, 1071, 1, 2] 12.8 / 12.3; [256, 2113, 1, 1] 25.4 / 29.6, [204, 17, 1, 1]
+// 7.1 / 9.1, [129, 1071, 2, 2] 10.1 / 10.2, [204, 4001, 2, 2] 32.9 / 34.5.
+bool tiny_ragged_planes(int64_t n, int64_t c, int64_t hw) {
+  if (hw <= 3) return n <= 48 || (n < 256 && c >= 1024);
+  return hw <= 6 && c >= 2048 && n >= 32 && n < 160;
+}
+
 }  // namespace
 }  // namespace hipo
 
@@ -1246,13 +1260,13 @@ extern "C" int hipo_batchnorm_nchw_act_mean_bf16(
   const NchwMerge none{};
   const NchwMerge mg{part, slices, running_mean, running_var, save_mean, save_rstd,
                      momentum, eps, var_scale};
-  if (c >= kPlaneChannels && hw <= kPlanesMaxHw) {
+  const bool whole = c % kPlaneChannels == 0 && aligned16(x);
+  if (c >= kPlaneChannels && hw <= kPlanesMaxHw && (whole || !tiny_ragged_planes(n, c, hw))) {
     const int64_t cb = (c + kPlaneWaves * kPlaneChannels - 1) / (kPlaneWaves * kPlaneChannels);
     const dim3 grid(static_cast<unsigned>(cb), static_cast<unsigned>(slices));
     const dim3 block(kPlaneWaves * kWave);
     const int h = static_cast<int>(hw);
     const DivMagic by_hw = div_magic(static_cast<uint32_t>(hw));
-    const bool whole = c % kPlaneChannels == 0 && aligned16(x);
 #define HIPO_PLANES(B_)                                                                      \
   do {                                                                                       \
     auto stats = whole ? bn_nchw_planes<0, B_, false> : bn_nchw_planes<0, B_, true>;          \
