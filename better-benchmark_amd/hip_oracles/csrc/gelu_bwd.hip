@@ -354,15 +354,17 @@ BwdPlan bwd_plan(int64_t rows, int64_t cols) {
 }
 
 // Rows per block as launched: the plan's, which sizes the workspace, rounded
-// up to whole passes of the 16 waves, a multiple of 32 rows (fewer row blocks,
+// up to whole passes of the 16 waves, 32, 64 or 96 rows (fewer row blocks,
 // so the workspace holds them).  A last pass that only some rows fill reads
 // and looks up as much as a full one.  Graph replays, the plan's rows -> here:
 // [25216, 3072] 73 -> 96, 91.6 -> 88.5 us; [8192, 6144] 48 -> 64, 65.2 -> 59.5;
 // [28000, 2880] 82 -> 96, 98.0 -> 93.2; [16384, 4608] 72 -> 96, 87.1 -> 86.4.
-// Powers of two instead: 86.9 at the first, but 91.3 at the last.
+// Powers of two instead: 86.9 at the first, but 91.3 at the last.  Not to 128
+// rows, whose fewer blocks end more unevenly: [25216, 4096] 98 -> 128, 115 ->
+// 120; [20000, 5120] 97 -> 128, 113 -> 117; [12800, 8192] 100 -> 128, 113 -> 119.
 int64_t bwd_launch_rows(const BwdPlan& p) {
-  if (p.threads != 1024 || p.rows_per_block > 128) return p.rows_per_block;
   constexpr int64_t kPass = 16 * kRows;
+  if (p.threads != 1024 || p.rows_per_block > 3 * kPass) return p.rows_per_block;
   return (p.rows_per_block + kPass - 1) / kPass * kPass;
 }
 
