@@ -310,8 +310,9 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_apply_pad(
   }
 }
 
-// C < 8, or too many rows for the kernels above: one thread per (slice,
-// channel), and per output value (also in place with C not a multiple of 8).
+// C < 8, few ragged rows, or too many rows for the kernels above: one thread per
+// (slice, channel), and per output value (also in place with C not a multiple
+// of 8).
 __global__ __launch_bounds__(256) void bn_nhwc_partial_scalar(
     const uint16_t* __restrict__ x, float2* __restrict__ part, int64_t M, int64_t C, int64_t L) {
   const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1074,6 +1075,12 @@ constexpr int64_t kNhwcMinSlice = 64;
 constexpr int64_t kNhwcMaxSlices = 512;
 constexpr int64_t kNhwcFewSlices = 192;
 
+// Fewer rows of C not a multiple of 8 (or off alignment) go one thread per
+// channel: a workgroup's tree over its row partials takes longer than so few
+// rows one after the other, [5, 237, 1, 1] 10.5 us against 7.7, [4, 425, 2, 2]
+// 10.7 against 9.5, [1, 429, 5, 5] 10.8 against 10.2.
+constexpr int64_t kNhwcMinRagged = 40;
+
 struct NhwcPlan {
   int threads = 0;  // of the epilogue
   int stat_threads = 0;
@@ -1144,7 +1151,7 @@ extern "C" int hipo_batchnorm_nhwc_act_pad_bf16(
   const int64_t rows_out = n * Ho * Wo;
   const bool small_rows = rows_out < (int64_t{1} << 31) && M < (int64_t{1} << 31);
   const bool whole = c % 8 == 0 && aligned16(x) && aligned16(out);
-  const NhwcPlan plan = nhwc_plan(M, c, small_rows);
+  const NhwcPlan plan = nhwc_plan(M, c, small_rows && (whole || M >= kNhwcMinRagged));
   const size_t need = static_cast<size_t>(plan.slices * c) * sizeof(float2);
   HIPO_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
                "%s: workspace of %zu bytes (16-byte aligned), need %zu", what, workspace_bytes,
