@@ -396,12 +396,16 @@ constexpr int64_t kLargeMinChannels = 32;
 // a multiple of 4, where over a third of those vectors' values would be
 // read twice, go value by value.  Workgroups in XCD order: neighbouring
 // channels share the cache lines at their planes' ends.  [128, 2048, 7, 7]
-// 39.0 us value by value -> 19.0 (5.4 TB/s).
+// 39.0 us value by value -> 19.0 (5.4 TB/s).  Whole planes of 4 KiB and more,
+// which share few, in launch order: [1, 300, 16000] 10.8 us against 11.5, [1,
+// 600, 10708] 11.5 against 12.0, [4, 600, 2676] 11.5 against 11.9; but [64, 512,
+// 196] 11.6 against 11.4.
 struct SmallGeom {
   int total;      // vectors, or values, per channel
   int per_plane;  // HW / 4 (kWhole) or HW (kValues)
   DivMagic by_plane;
   PlaneGeom ragged;  // kRagged
+  bool xcd;          // workgroups in XCD order
 };
 
 enum class SmallKind { kValues, kWhole, kRagged };
@@ -416,7 +420,7 @@ __global__ __launch_bounds__(T) void bn_channel_small(
   constexpr bool kVec = KIND != SmallKind::kValues;
   constexpr bool kRagged = KIND == SmallKind::kRagged;
   using Elem = std::conditional_t<kRagged, f32x4_t, std::conditional_t<kVec, float4, float>>;
-  const int64_t c = xcd_order(blockIdx.x, gridDim.x);
+  const int64_t c = g.xcd ? xcd_order(blockIdx.x, gridDim.x) : blockIdx.x;
   float pg = 0.f, pb = 0.f, prm = 0.f, prv = 0.f;
   if (threadIdx.x == 0) {
     pg = gamma[c];
@@ -540,6 +544,7 @@ int small_launch(const float* x, const float* gamma, const float* beta, float* r
   g.per_plane = static_cast<int>(whole ? hw / 4 : hw);
   g.by_plane = div_magic(static_cast<uint32_t>(g.per_plane));
   g.ragged = plane_geom(hw);
+  g.xcd = !whole || hw < 1024;
   g.total = static_cast<int>(n) * (ragged ? g.ragged.F : g.per_plane);
 #define HIPO_BN_SMALL(K, ...)                                                        \
   launch_small<SmallKind::K, __VA_ARGS__>(x, gamma, beta, running_mean, running_var, y, \
