@@ -118,6 +118,14 @@ __device__ __forceinline__ void bn_act_x8(float (&y)[8]) {
   }
 }
 
+// A sum of squares about a shift less its correction: rounding can leave a
+// tiny negative.  max(v, 0) that keeps NaN, the M2 of a channel with a NaN or an
+// infinite value (a zero there would give it a finite rstd and finite outputs).
+template <typename T>
+__device__ __forceinline__ T not_negative(T v) {
+  return __builtin_elementwise_maximum(v, T(0));
+}
+
 // Chan's pairwise merge of (count, mean, M2) partials: (n, mean, m2) <-
 // (n, mean, m2) + (nb, meanb, m2b).
 template <typename T>
@@ -242,7 +250,7 @@ __global__ __launch_bounds__(kMaxThreads) void bn_nhwc_partial(
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float d = s1[e] / n;
-    dst[e] = make_float2(shift[e] + d, fmaxf(s2[e] - s1[e] * d, 0.f));
+    dst[e] = make_float2(shift[e] + d, not_negative(s2[e] - s1[e] * d));
   }
 }
 
@@ -329,7 +337,7 @@ __global__ __launch_bounds__(256) void bn_nhwc_partial_scalar(
   }
   const float n = static_cast<float>(p1 - p0);
   const float d = s1 / n;
-  part[s * C + c] = make_float2(shift + d, fmaxf(s2 - s1 * d, 0.f));
+  part[s * C + c] = make_float2(shift + d, not_negative(s2 - s1 * d));
 }
 
 __global__ __launch_bounds__(256) void bn_nhwc_apply_pad_scalar(
@@ -448,7 +456,7 @@ __global__ __launch_bounds__(kNchwImages * kWave) void bn_nchw_small_hw(
     }
     const double dm = s1 / n;
     const float mc = static_cast<float>(K + dm);
-    const float var_f = static_cast<float>(std::max(0.0, s2 - s1 * dm) / n);
+    const float var_f = static_cast<float>(not_negative(s2 - s1 * dm) / n);
     const float rc = 1.0f / __builtin_sqrtf(__fadd_rn(var_f, mg.eps));
     if (blockIdx.y == 0 && w == 0 && c < C) {
       mg.save_mean[c] = mc;
@@ -582,7 +590,7 @@ __global__ __launch_bounds__(kPlaneWaves * kWave) void bn_nchw_planes(
       s2 = sum8(s2);
       const double dm = s1 / n;
       mc = static_cast<float>(K + dm);
-      const float var_f = static_cast<float>(std::max(0.0, s2 - s1 * dm) / n);
+      const float var_f = static_cast<float>(not_negative(s2 - s1 * dm) / n);
       rc = 1.0f / __builtin_sqrtf(__fadd_rn(var_f, mg.eps));
       if (s == 0 && k == 0 && own) {
         mg.save_mean[c] = mc;
@@ -715,7 +723,7 @@ __global__ __launch_bounds__(kWideWaves * kWave) void bn_nchw_wide(
     s2 = wave_sum(s2);
     const double dm = s1 / n;
     mc = static_cast<float>(K + dm);
-    const float var_f = static_cast<float>(std::max(0.0, s2 - s1 * dm) / n);
+    const float var_f = static_cast<float>(not_negative(s2 - s1 * dm) / n);
     rc = 1.0f / __builtin_sqrtf(__fadd_rn(var_f, mg.eps));
     g = gamma[c];
     b = beta[c];
@@ -944,7 +952,7 @@ __global__ __launch_bounds__(kChanThreads) void bn_nchw_channels(
   const double mean = static_cast<double>(shift) + dmean;
   const float mf = static_cast<float>(mean);
   const double m2 = t2 - t1 * dmean;
-  const float var_f = static_cast<float>(std::max(0.0, m2) / cnt);
+  const float var_f = static_cast<float>(not_negative(m2) / cnt);
   const float rc = 1.0f / __builtin_sqrtf(__fadd_rn(var_f, eps));
   if (part == 0 && lane == 0) {
     save_mean[c] = mf;
@@ -1041,7 +1049,7 @@ __global__ __launch_bounds__(kFinalThreads) void bn_finalize(
   s2 = red[2][t];
   const double dm = s1 / n;
   const float mean_f = static_cast<float>(K + dm);
-  const float var_f = static_cast<float>(std::max(0.0, s2 - s1 * dm) / n);
+  const float var_f = static_cast<float>(not_negative(s2 - s1 * dm) / n);
   save_mean[c] = mean_f;
   save_rstd[c] = 1.0f / __builtin_sqrtf(__fadd_rn(var_f, eps));
   const float keep = 1.0f - momentum;
