@@ -187,6 +187,27 @@ def test_transpose_any_matrix(r, c, dtype, rocm_device):
         assert torch.equal(out.t.cpu(), x.transpose(1, 2).contiguous()), f"[{r}, {c}]"
 
 
+# Every cache policy of the register-block transposes: rows of whole cache lines
+# both ways up to 32 MB read and written and beyond 160 MB (non-temporal; in
+# plain workgroup order where four tiles cover the output rows, XCD order
+# otherwise), between the two (non-temporal stores), and rows that are not whole
+# lines beyond 160 MB (cached).
+@pytest.mark.parametrize("batch,r,c,dtype", [
+    (2, 512, 384, torch.bfloat16), (2, 256, 192, torch.float32), (40, 512, 512, torch.bfloat16),
+    (161, 256, 1024, torch.bfloat16), (161, 128, 1024, torch.float32),
+    (81, 1024, 512, torch.bfloat16), (161, 520, 500, torch.bfloat16)])
+def test_transpose_cache_policies(batch, r, c, dtype, rocm_device):
+    g = torch.Generator(device=rocm_device).manual_seed(r + c)
+    bits = torch.int16 if dtype == torch.bfloat16 else torch.int32
+    x = torch.randint(-2 ** 15, 2 ** 15, (batch, r, c), generator=g, device=rocm_device).to(bits)
+    out = Guarded((batch, c, r), bits, rocm_device)
+    ok(lib().hipo_transpose_last2(x.data_ptr(), out.t.data_ptr(), batch, r, c, x.element_size(),
+                                  None))
+    torch.cuda.synchronize()
+    out.check(f"[{batch}, {r}, {c}]")
+    assert torch.equal(out.t, x.transpose(1, 2)), f"[{batch}, {r}, {c}]"
+
+
 # (n, c, hw): planes of whole float4s and not, value by value (below 9), one
 # vector a thread and many, the 1024-thread kernel from 16385 values on (both
 # kinds, its largest), split-K past it, with one plane and with many.

@@ -1146,11 +1146,11 @@ def test_batchnorm_nchw_act_mean(n, c, h, w, act, rocm_device):
     assert_close(out, wy.mean((2, 3)), BF16_TOL, "spatial mean")
 
 
-def test_batchnorm_nchw_misaligned_x_takes_the_general_kernel(rocm_device):
-    """x 2 bytes off a 16-byte boundary: neither the register-held channels
-    kernel (8-byte words) nor the planes kernel (16-byte vectors) applies,
-    and the lane-per-channel kernel gives the same statistics and means as
-    the aligned call at the same shape (which takes the channels kernel)."""
+def test_batchnorm_nchw_misaligned_x_takes_the_ragged_planes(rocm_device):
+    """x 2 bytes off a 16-byte boundary: the register-held channels kernel
+    (8-byte words) does not apply, and the planes kernel with element-aligned
+    loads gives the same statistics and means as the aligned call at the same
+    shape (which takes the channels kernel)."""
     import hip_oracles
     n, c, h, w = 64, 32, 7, 7
     x, (gm, bt, rm, rv) = _bn_bf16_inputs(n, c, h, w, 77, False)
@@ -1321,35 +1321,44 @@ def test_batchnorm_closed_forms_and_edges(rocm_device):
     assert (y[:, :3] < 0).any(), "relu=False keeps negatives"
 
 
-# (N, C, HW, what the shape exercises): channels of more than 16384 values
-# take the single-pass kernel (or the split-K path where it does not
-# apply), smaller ones the register-held one-launch kernel.
+# (N, C, HW, whether the single-pass kernel takes it, what the shape
+# exercises): channels of up to 16384 values, and larger ones of up to 28672
+# (whole float4 planes, at least 32 channels) or 12 vectors a thread of 1024
+# (other planes), are held in registers by one workgroup each; larger ones take
+# the single-pass kernel, or split-K where that does not apply.
 BN_PLAN_SHAPES = [
-    (16, 300, 3136, "exact slabs, 1 slab/channel, 2 rounds (C > CUs)"),
-    (32, 8, 3136, "exact slabs, 2 slabs/channel, 1 round"),
-    (7, 5, 2800, "masked V=16"),
-    (30, 100, 4000, "masked V=24, 3 slabs/channel, 2 rounds"),
-    (2, 600, 8200, "3 rounds (odd)"),
-    (2, 1000, 8200, "4 rounds (even)"),
-    (8, 9, 2060, "HW % 4 == 0 but F not a power of two"),
-    (40, 3, 4001, "more than 64 rounds, HW % 4 != 0: split-K path"),
-    (2, 6, 64, "small channels, 1 float4 per thread"),
-    (5, 7, 1600, "small channels, 8 float4 per thread"),
-    (4, 3, 4096, "small channels at the limit, 16 float4 per thread"),
-    (3, 20000, 16, "small channels, 20000 workgroups"),
-    (4, 9, 60, "small channels, F not a power of two"),
-    (3, 7, 49, "small channels, HW % 4 != 0: single values"),
-    (1, 5, 16383, "small channels at the limit, HW % 4 != 0: 64 values per thread"),
-    (7, 4, 2, "small channels, HW % 4 != 0, 4 values per thread"),
+    (16, 300, 3136, True, "exact slabs, 1 slab/channel, 2 rounds (C > CUs)"),
+    (32, 8, 3136, True, "exact slabs, 2 slabs/channel, 1 round"),
+    (7, 5, 2800, True, "masked V=16"),
+    (30, 100, 4000, True, "masked V=24, 3 slabs/channel, 2 rounds"),
+    (2, 600, 14500, True, "masked slabs, 3 rounds (odd)"),
+    (2, 1000, 14500, True, "masked slabs, 4 rounds (even)"),
+    (8, 9, 2060, True, "HW % 4 == 0 but F not a power of two"),
+    (40, 3, 4001, False, "more than 64 rounds, HW % 4 != 0: split-K path"),
+    (2, 600, 8200, False, "larger channels in registers, 5 float4 per thread"),
+    (2, 1000, 8200, False, "larger channels in registers, 1000 workgroups"),
+    (2, 6, 64, False, "small channels, 1 float4 per thread"),
+    (5, 7, 1600, False, "small channels, 8 float4 per thread"),
+    (4, 3, 4096, False, "small channels at the limit, 16 float4 per thread"),
+    (3, 20000, 16, False, "small channels, 20000 workgroups"),
+    (4, 9, 60, False, "small channels, F not a power of two"),
+    (3, 7, 49, False, "small channels, HW % 4 != 0: last vector moved back"),
+    (1, 5, 16383, False, "small channels at the limit, HW % 4 != 0: 16 vectors per thread"),
+    (7, 4, 2, False, "small channels, value by value, 1 per thread"),
+    (100, 3, 7, False, "small channels, value by value, 4 per thread"),
+    (500, 3, 5, False, "small channels, value by value, 16 per thread"),
+    (2300, 2, 7, False, "small channels, value by value, 64 per thread"),
+    (5000, 2, 3, False, "small channels, value by value, planes below a vector"),
 ]
 
 
-@pytest.mark.parametrize("n,c,hw,what", BN_PLAN_SHAPES, ids=[s[3] for s in BN_PLAN_SHAPES])
-def test_batchnorm_plans_vs_oracle(n, c, hw, what, rocm_device):
+@pytest.mark.parametrize("n,c,hw,single_pass,what", BN_PLAN_SHAPES,
+                         ids=[s[4] for s in BN_PLAN_SHAPES])
+def test_batchnorm_plans_vs_oracle(n, c, hw, single_pass, what, rocm_device):
     """Every instantiation of the single-pass kernel, the split-K fallback
-    and the small-channel kernel against the CPU oracle, twice in a row on
+    and the register-held kernels against the CPU oracle, twice in a row on
     the shared workspace (the second single-pass call runs under the next
-    launch epoch)."""
+    launch epoch, which the workspace counts)."""
     import hip_oracles
     import oracle as ref
     print(f"[bn plan] {n}x{c}x{hw}: {what}", flush=True)
@@ -1360,12 +1369,16 @@ def test_batchnorm_plans_vs_oracle(n, c, hw, what, rocm_device):
     rm, rv = 0.1 * torch.randn(c, generator=g), 1 + 0.1 * torch.rand(c, generator=g)
     want = ref.batchnorm_train(x, gamma, beta, rm, rv, momentum=0.1, eps=1e-5, relu=True)
     xd = x.to(rocm_device)
+    epochs = []
     for call in range(2):
         rm_d, rv_d = rm.to(rocm_device), rv.to(rocm_device)
         y, sm, si = hip_oracles.batchnorm_train(xd, gamma.to(rocm_device), beta.to(rocm_device),
                                                 rm_d, rv_d, momentum=0.1, eps=1e-5, relu=True)
+        ws = hip_oracles._bn_workspaces[rocm_device.index]
+        epochs.append(int(ws[4:8].view(torch.int32).item()))
         for name, a, w in zip(("y", "mean", "invstd", "rm", "rv"), (y, sm, si, rm_d, rv_d), want):
             assert_close(a, w, F32_TOL, f"bn {n}x{c}x{hw} call {call} {name}")
+    assert epochs[1] - epochs[0] == int(single_pass), "the route the shape is listed for"
     assert hip_oracles.batchnorm_error_flag(rocm_device) == 0
 
 

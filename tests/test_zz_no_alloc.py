@@ -4,9 +4,9 @@ hipo_batchnorm_train_fwd_f32_noalloc keeps its workspace in a file-scope
 device array instead of a caller allocation.  Called through the C ABI, it
 must give bit-identical outputs (y, save_mean, save_invstd and the updated
 running statistics) to hipo_batchnorm_train_fwd_f32 with a zeroed caller
-workspace on the same inputs: the same kernels run in both.  Two calls in a
-row, the second on a smaller shape (the array keeps the first call's state),
-plus a shape beyond the array's size, which must be rejected.
+workspace on the same inputs: the same kernels run in both.  Calls in a row
+on smaller shapes (the array keeps the earlier calls' state), plus a shape
+beyond the array's size, which must be rejected.
 """
 import ctypes
 
@@ -15,10 +15,15 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
+# (shape, whether the single-pass kernel, with its exchange state in the
+# workspace, takes it)
 SHAPES = [
-    (128, 256, 56, 56),  # the BASELINE config: the single-pass kernel
-    (16, 24, 7, 7),      # smaller, HW % 4 != 0: one workgroup per channel
-    (32, 64, 28, 28),    # smaller again, single pass with another slab plan
+    ((128, 256, 56, 56), True),  # the largest: the single-pass kernel
+    ((16, 24, 7, 7), False),     # smaller, HW % 4 != 0: one workgroup per channel
+    ((64, 64, 28, 28), True),    # smaller, single pass with another slab plan
+    ((32, 64, 28, 28), False),   # one 1024-thread workgroup per channel
+    ((30, 20, 41, 41), False),   # two split-K launches
+    ((64, 64, 28, 28), True),    # single pass again, on what the others left
 ]
 
 
@@ -33,7 +38,7 @@ def _inputs(shape, seed):
     return x, gamma, beta, rm, rv
 
 
-def _run(lib, dev, shape, seed, noalloc):
+def _run(lib, dev, shape, seed, noalloc, single_pass=None):
     n, c, h, w = shape
     x, gamma, beta, rm, rv = (t.to(dev) for t in _inputs(shape, seed))
     y = torch.empty_like(x)
@@ -50,6 +55,8 @@ def _run(lib, dev, shape, seed, noalloc):
                                               ws.data_ptr(), need, stream)
     assert rc == 0, lib.hipo_last_error().decode()
     torch.cuda.synchronize(dev)
+    if single_pass is not None:  # its launch epoch, bytes 4..7 of the zeroed workspace
+        assert int(ws[4:8].view(torch.int32).item()) == int(single_pass), shape
     return [t.cpu() for t in (y, save_mean, save_invstd, rm, rv)]
 
 
@@ -57,9 +64,9 @@ def test_noalloc_matches_workspace_entry_point(rocm_device):
     import hip_oracles
     lib = hip_oracles.load_library()
     names = ("y", "save_mean", "save_invstd", "running_mean", "running_var")
-    for k, shape in enumerate(SHAPES):
+    for k, (shape, single_pass) in enumerate(SHAPES):
         print(f"noalloc vs workspace: shape {shape}", flush=True)
-        want = _run(lib, rocm_device, shape, 100 + k, noalloc=False)
+        want = _run(lib, rocm_device, shape, 100 + k, noalloc=False, single_pass=single_pass)
         got = _run(lib, rocm_device, shape, 100 + k, noalloc=True)
         for name, a, b in zip(names, got, want):
             assert torch.isfinite(a).all(), f"{shape} {name}: non-finite values"
@@ -90,7 +97,7 @@ def test_noalloc_forced_timeout_is_reported(rocm_device, monkeypatch):
     without injection matches the workspace entry point again."""
     import hip_oracles
     lib = hip_oracles.load_library()
-    shape = SHAPES[0]  # the single-pass kernel with its cross-workgroup exchange
+    shape = SHAPES[0][0]  # the single-pass kernel with its cross-workgroup exchange
     _run(lib, rocm_device, shape, 5, noalloc=True)  # the array is set up
     hip_oracles.device_faults()  # start clean
     monkeypatch.setenv("HIPO_TEST_FORCE_BN_TIMEOUT", "1")
