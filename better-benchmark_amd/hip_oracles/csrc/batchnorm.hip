@@ -405,7 +405,7 @@ struct SmallGeom {
   int per_plane;  // HW / 4 (kWhole) or HW (kValues)
   DivMagic by_plane;
   PlaneGeom ragged;  // kRagged
-  bool xcd;          // workgroups in XCD order
+  bool xcd;          // kWhole: workgroups in XCD order (the others always)
 };
 
 enum class SmallKind { kValues, kWhole, kRagged };
@@ -420,7 +420,8 @@ __global__ __launch_bounds__(T) void bn_channel_small(
   constexpr bool kVec = KIND != SmallKind::kValues;
   constexpr bool kRagged = KIND == SmallKind::kRagged;
   using Elem = std::conditional_t<kRagged, f32x4_t, std::conditional_t<kVec, float4, float>>;
-  const int64_t c = g.xcd ? xcd_order(blockIdx.x, gridDim.x) : blockIdx.x;
+  const bool xcd = KIND != SmallKind::kWhole || g.xcd;
+  const int64_t c = xcd ? xcd_order(blockIdx.x, gridDim.x) : blockIdx.x;
   float pg = 0.f, pb = 0.f, prm = 0.f, prv = 0.f;
   if (threadIdx.x == 0) {
     pg = gamma[c];
@@ -544,7 +545,7 @@ int small_launch(const float* x, const float* gamma, const float* beta, float* r
   g.per_plane = static_cast<int>(whole ? hw / 4 : hw);
   g.by_plane = div_magic(static_cast<uint32_t>(g.per_plane));
   g.ragged = plane_geom(hw);
-  g.xcd = !whole || hw < 1024;
+  g.xcd = hw < 1024;
   g.total = static_cast<int>(n) * (ragged ? g.ragged.F : g.per_plane);
 #define HIPO_BN_SMALL(K, ...)                                                        \
   launch_small<SmallKind::K, __VA_ARGS__>(x, gamma, beta, running_mean, running_var, y, \
