@@ -213,7 +213,9 @@ def test_transpose_cache_policies(batch, r, c, dtype, rocm_device):
 # kinds, its largest), split-K past it, with one plane and with many.
 BN_TRAIN = [(3, 5, 7), (3, 5, 9), (4, 5, 12), (26, 9, 49), (334, 3, 49), (335, 3, 49), (128, 40, 196),
             (146, 33, 196), (147, 33, 196), (1820, 2, 9), (2000, 3, 13), (17, 6, 1295), (5, 3, 9999),
-            (1, 4, 50001), (60, 2, 1023), (9000, 2, 3), (700, 2, 70)]
+            (1, 4, 50001), (60, 2, 1023), (9000, 2, 3), (700, 2, 70),
+            # 9 vectors a thread: split-K for few channels of long planes only
+            (16, 3, 2209), (16, 32, 2209), (900, 2, 41)]
 
 
 @pytest.mark.parametrize("n,c,hw", BN_TRAIN)
