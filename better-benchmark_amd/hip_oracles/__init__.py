@@ -429,8 +429,8 @@ def rmsnorm_ex(x, gamma, eps: float, *, residual=None, scale: float = 1.0, mode:
 
 def scaled_bias_softmax(x, bias, scale: float, heads: int):
     """softmax(x * scale + bias, -1) for bf16 x [B, Q, K] and a bias
-    [B / heads, Q, K] (any layout with unit inner stride and 8-aligned row and
-    batch strides) shared by `heads` consecutive batch entries."""
+    [B / heads, Q, K] (any layout with unit inner stride) shared by `heads`
+    consecutive batch entries."""
     lib = _lib or load_library()
     dev = _require_rocm(x, bias)
     _require(x.dtype == torch.bfloat16 and bias.dtype == torch.bfloat16,

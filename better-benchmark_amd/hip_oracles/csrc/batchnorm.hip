@@ -379,19 +379,19 @@ constexpr int64_t kSmallChannel = 16384;
 // Larger ones take the same kernel with 1024 threads: whole float4 planes up
 // to 7 a thread (28672 values; two workgroups per CU) and at least 32
 // channels, ragged ones, whose alternative reads x twice, up to 8 vectors a
-// thread, and up to 12 in planes below 1024 values or 32 channels and more.  Graph replays in us, single-pass kernel / here, inputs reused [not
-// reused]: [128, 1024, 14, 14] 56.7 / 39.3 [57.3 / 47.7], [128, 256, 14, 14]
+// thread, and up to 12 in planes below 1024 values or 32 channels and more.
+// Graph replays in us, single-pass kernel / here, inputs reused [not reused]: [128, 1024, 14, 14] 56.7 / 39.3 [57.3 / 47.7], [128, 256, 14, 14]
 // 15.6 / 11.9 [16.5 / 14.8], [128, 64, 14, 14] 9.2 / 7.1 [9.6 / 8.6], but
 // [64, 512, 28, 28], 50176 values, 37.7 / 40.5 [37.8 / 52.0] and [6, 960, 72,
 // 70], 30240, 52.4 / 47.8 [52.8 / 57.8].  Split-K before / split-K now / here:
 // [512, 512, 7, 7] 95 / 34.5 / 23.0, [17, 488, 35, 37] 41.2 / 32.5 / 19.4, [21,
 // 782, 46, 43] 119 / 81 / 58, [12, 1280, 46, 45] 105 / 78 / 53; with 16 vectors
-// a thread (and spills) [5, 32, 101, 99] 22.7 / 9.7 / 12.3.  Ragged planes of few
-// channels, split-K / here: up to 8 vectors a thread here is faster down to one
-// channel ([2, 1, 99, 101] 8.9 / 6.7, [400, 4, 7, 7] 11.6 / 7.0); beyond, only for
-// planes that are short ([900, 1, 7, 7] 11.5 / 9.7, but [16, 1, 47, 47] 7.5 / 9.1,
-// [16, 16, 47, 47] 7.9 / 9.6, [3, 4, 127, 127] 10.1 / 10.2; from 32 channels on they
-// are even).
+// a thread (and spills) [5, 32, 101, 99] 22.7 / 9.7 / 12.3.  Ragged planes of
+// few channels, split-K / here: up to 8 vectors a thread here is faster down to
+// one channel ([2, 1, 99, 101] 8.9 / 6.7, [400, 4, 7, 7] 11.6 / 7.0); beyond, only
+// for planes that are short ([900, 1, 7, 7] 11.5 / 9.7, but [16, 1, 47, 47] 7.5 /
+// 9.1, [16, 16, 47, 47] 7.9 / 9.6, [3, 4, 127, 127] 10.1 / 10.2; from 32 channels
+// on they are even).
 constexpr int64_t kLargeChannel = 65536;
 constexpr int kLargeThreads = 1024;
 constexpr int64_t kLargeMinChannels = 32;

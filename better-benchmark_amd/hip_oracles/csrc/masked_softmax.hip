@@ -474,7 +474,8 @@ template <int U, int WT, bool RAGGED>
 void launch_vec(dim3 grid, const RowPlan& plan, hipStream_t stream, const uint16_t* x,
                 const uint16_t* mask, uint16_t* out, int64_t rows, int64_t Q, int64_t K,
                 int64_t ms, int64_t mbs, int64_t heads, float scale) {
-  // Used for rows < 2^31 only, where q and heads are below 2^31 too.
+  // The multipliers stand for rows < 2^31, where q and heads are below 2^31
+  // too; the kernel divides from there on.
   const bool small = rows < (int64_t{1} << 31);
   const DivMagic qd = small ? div_magic(static_cast<uint32_t>(Q)) : DivMagic{};
   const DivMagic hd = small ? div_magic(static_cast<uint32_t>(heads)) : DivMagic{};

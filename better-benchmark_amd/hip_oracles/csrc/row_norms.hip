@@ -356,7 +356,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_scalar(
   const float rstd =
       1.0f / __builtin_sqrtf(wave_sum(sq) / static_cast<float>(cols) + eps);
   for (int64_t j = lane; j < cols; j += kWave) {
-      float v = (H_OVER ? bf16_to_f32(h[base + j]) : hval(j)) * rstd;
+    float v = (H_OVER ? bf16_to_f32(h[base + j]) : hval(j)) * rstd;
     if (mode == 0) {
       v = v * bf16_to_f32(gamma[j]);
       if (scale != 1.0f) v *= scale;
