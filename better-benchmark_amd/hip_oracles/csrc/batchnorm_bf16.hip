@@ -1061,11 +1061,16 @@ __global__ __launch_bounds__(kFinalThreads) void bn_finalize(
 // Channels-last plan: threads per workgroup (0: scalar kernels), rows per
 // slice and slice count.  A workgroup has R rows of G = ceil(C / 8) groups
 // per instruction, R a power of two, up to 512 threads in the statistics pass
-// and 256 in the epilogue (the last wave may be partial).  Slices are of a multiple of 512 rows, at most about 512 of them;
-// where that gives under 192, they are halved, down to 64 rows: a launch of a
-// dozen workgroups, one per 512 rows, took twice as long.  The slicing depends on the shape alone, and so
-// does the workspace size; its traffic (8 B per channel per slice) stays
-// under 3 % of x.
+// and 256 in the epilogue (the last wave may be partial).  Slices are of a
+// multiple of 512 rows, at most about 512 of them; where that gives under 128,
+// they are halved, down to 64 rows: a launch of a dozen workgroups, one per 512
+// rows, took twice as long.  Under 96 / 128 / 192 / 288, us: C 48, 20300 rows 12.3
+// / 12.4 / 13.7 / -, C 40, 42200 rows 13.4 / 13.4 / 14.1 / -, C 64, 68992 rows - /
+// 16.4 / 17.7 / 21.3, C 512, 94080 rows - / 54.6 / 56.5 / 56.6, C 1024, 28000 and
+// 55000 rows 36.8 / 35.5 / 35.8 and 61.8 / 59.0 / 59.1.  The slicing depends on
+// the shape alone, and so does the workspace size; its traffic, 8 B per channel
+// and slice written and read, is 6 % of x each way for 64-row slices (fewer than
+// 16384 rows) and under 1 % for 512.
 // Graph replays of the whole call in us, before (at least 512-row slices, a
 // slice stride between a workgroup's results) -> now: [128, 240, 28, 28] 33.0
 // -> 31.6, [128, 96, 112, 112] 159.0 -> 156.7, [29, 896, 14, 14] 32.5 -> 16.3,
@@ -1081,7 +1086,7 @@ constexpr int kNhwcApplyThreads = 256;
 constexpr int64_t kNhwcSliceStep = 512;
 constexpr int64_t kNhwcMinSlice = 64;
 constexpr int64_t kNhwcMaxSlices = 512;
-constexpr int64_t kNhwcFewSlices = 192;
+constexpr int64_t kNhwcFewSlices = 128;
 
 // Fewer rows of C not a multiple of 8 (or off alignment) go one thread per
 // channel: a workgroup's tree over its row partials takes longer than so few

@@ -383,7 +383,9 @@ def test_spatial_mean_any_channels(n, c, hw, rocm_device):
 BN_NHWC = [(2, 7, 3, 3, 1), (2, 8, 3, 3, 0), (3, 9, 5, 4, 1), (2, 28, 20, 21, 1), (4, 103, 9, 9, 0),
            (2, 664, 6, 5, 1), (3, 2049, 3, 2, 1), (40, 33, 31, 30, 0), (1, 8200, 2, 2, 0),
            # 39 and 40 rows: one thread per channel, and workgroups
-           (3, 237, 13, 1, 1), (4, 237, 5, 2, 1), (4, 9, 2, 5, 0)]
+           (3, 237, 13, 1, 1), (4, 237, 5, 2, 1), (4, 9, 2, 5, 0),
+           # 127 128-row slices, halved, and 128 of them, a partial last one
+           (1, 40, 127, 128, 0), (1, 40, 128, 128, 1), (1, 9, 131, 127, 0)]
 
 
 @pytest.mark.parametrize("n,c,h,w,pad", BN_NHWC)
