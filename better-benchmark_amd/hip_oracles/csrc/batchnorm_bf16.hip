@@ -1036,7 +1036,11 @@ __global__ __launch_bounds__(kFinalThreads) void bn_finalize(
   red[1][t] = s1;
   red[2][t] = s2;
   __syncthreads();
-  for (int half = kFinalLanes / 2; half > 0; half /= 2) {
+  // Lanes past the slices hold zeros: the tree starts at the others ([2, 179, 2,
+  // 1], one slice, 8.9 -> 6.7 us a call).
+  int half = kFinalLanes / 2;
+  while (half > 0 && half >= slices) half /= 2;
+  for (; half > 0; half /= 2) {
     if (j < half) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) red[q][t] += red[q][t + half * kFinalCols];
