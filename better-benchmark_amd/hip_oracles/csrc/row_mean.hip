@@ -373,15 +373,23 @@ extern "C" int hipo_row_mean_bf16(const uint16_t* x, uint16_t* out, int64_t rows
   const bool two = cols <= int64_t{waves} * 2 * kRowSweep;
   const int64_t sweep = int64_t{waves} * (two ? 2 : 4) * kRowSweep;
   const int64_t held = (cols + sweep - 1) / sweep * sweep;
-  // With many rows a wave per row is faster where the row fills under 85 % of
-  // that (60 % where one wave holds it or in several sweeps), us, wave / rows
-  // kernel: [50000, 520] 13.8 / 14.9, [50000, 776] 16.9 / 15.5, [50000, 1032]
-  // 22.0 / 27.1, [16000, 1536] 9.5 / 10.9, [16000, 1736] 11.5 / 11.0, [8000,
-  // 2056] 7.8 / 9.4, [8000, 4104] 12.7 / 13.8, [8000, 4096] 12.1 / 12.0, [4096,
-  // 8200] 15.0 / 16.6, [4096, 12000] 21.2 / 19.6; fewer rows, [1024, 2056] 4.5 /
-  // 3.8, [3000, 1032] 3.8 / 4.4, [3000, 3080] 6.6 / 6.0.
-  const bool wave_rows = !ragged && rows >= (waves <= 2 ? 2560 : 4096) &&
-                         cols * 20 < held * (waves > 1 && two ? 17 : 12);
+  const int64_t fill = cols * 100 / held;
+  // A wave per row is faster where many rows fill little of that, and where
+  // one or two waves a row come to more workgroups than CUs.  The rows kernel's
+  // time over the wave's, graph replays, 700 points of 520 to 12296 values and 1
+  // to 60000 rows.  One wave: 520 values, 2048 rows 1.02, 2300 1.17, 60000 1.08;
+  // 776, 3600 rows 1.16, 16000 1.07, 32000 0.95; 1024, 2300 rows 1.14, 24000
+  // 0.99.  Two: 1032 values 1.02 to 1.37 from 1400 rows on; 1224, 1400 rows 1.02,
+  // 1600 1.13; 1448, 1500 rows 0.93, 2800 1.12; 1736, 3400 rows 1.00, 5000 1.12.
+  // Three: 2056 values, 2600 rows 1.01, 3200 1.06; 2312, 2800 rows 0.97, 4000
+  // 1.07.  More: 4104 values, 3400 rows 0.95, 5000 1.10; 8200, 4096 rows 1.17;
+  // 10248, 5000 rows 1.07, 12296, 4096 rows 0.93.
+  const int64_t wave_from = waves == 1   ? 2049
+                            : waves == 2 ? (fill < 54 ? 1 : fill < 76 ? 1537 : 4096)
+                            : waves <= 4 ? (fill < 70 ? 2816 : 3584)
+                                         : 4096;
+  const bool little = waves == 1 ? fill < 60 || rows <= 16384 : fill < (two ? 85 : 60);
+  const bool wave_rows = !ragged && little && rows >= wave_from;
   if (cols <= kBf16ShortCols && (aligned || (off_short && rows >= kBf16ShortRows))) {
     const int64_t blocks = blocks_of(kBf16Waves * kBf16RowsPerWave);
     HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
@@ -407,8 +415,15 @@ extern "C" int hipo_row_mean_bf16(const uint16_t* x, uint16_t* out, int64_t rows
     kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kBf16Waves * kWave), 0, stream>>>(
         x, out, rows, cols);
   } else {
+    // Workgroups of 4 waves where 2 to 4 of them make a row (8 / 4 waves, us:
+    // [1500, 1448] 3.18 / 2.93, [1280, 1640] 3.05 / 2.73, [9000, 3592] 11.3 / 10.7,
+    // [16000, 2312] 14.6 / 13.2), 8 for rows of one wave and two loads (even) and
+    // for many ragged rows of 3 and 4 waves (2880 to 4095 values, 1500 rows 0.98,
+    // 5000 to 16000 rows 1.05 times the 8 waves' time).
     const bool one = cols <= kRowSweep;
-    const int rpb = (one ? kBf16Waves : kMaxWaves) / waves;
+    const bool small_groups =
+        one || waves == 2 || (waves > 2 && waves <= kBf16Waves && (!ragged || rows <= 2048));
+    const int rpb = (small_groups ? kBf16Waves : kMaxWaves) / waves;
     const int64_t blocks = blocks_of(rpb);
     HIPO_REQUIRE(blocks <= 0x7fffffff, "row_mean_bf16: too many rows");
 #define HIPO_RMB(ACT_)                                                                     \

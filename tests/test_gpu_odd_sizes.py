@@ -524,12 +524,16 @@ def test_row_mean_any_row_length(cols, rocm_device):
 
 # (rows, cols, elements off alignment): both sides of the lines where short
 # rows off alignment leave the wave per row for the short-row kernel (24000
-# rows, up to 256 values), and whole longer ones the several waves per row for
-# one (2560 and 4096 rows); partial last workgroups.
+# rows, up to 256 values), and whole longer ones the rows kernel for one wave
+# each, by waves a row and how full they are; partial last workgroups.
 @pytest.mark.parametrize("rows,cols,shift", [
     (23999, 256, 1), (24000, 256, 1), (24013, 9, 3), (24001, 257, 1), (70, 400, 1), (9, 512, 5),
     (2559, 520, 0), (2560, 520, 0), (2563, 1032, 0), (4095, 2056, 0), (4097, 2056, 0),
-    (4099, 4104, 0), (4097, 8200, 0), (2561, 1024, 0)])
+    (4099, 4104, 0), (4097, 8200, 0), (2561, 1024, 0),
+    (2048, 520, 0), (2049, 1000, 0), (16384, 1000, 0), (16385, 1000, 0), (16385, 520, 0),
+    (3, 1096, 0), (3, 1112, 0), (1536, 1448, 0), (1537, 1448, 0), (4095, 1736, 0), (4096, 1736, 0),
+    (2815, 2056, 0), (2816, 2056, 0), (3583, 3080, 0), (3584, 3080, 0), (4099, 3592, 0),
+    (2048, 3001, 0), (2049, 3001, 0), (2047, 4095, 3), (2053, 4095, 0), (999, 1500, 1)])
 def test_row_mean_bf16_many_rows(rows, cols, shift, rocm_device):
     """One rounding of an fp32 mean: one ulp, 2^-7, and 1e-5 near zero."""
     import oracle as ref
