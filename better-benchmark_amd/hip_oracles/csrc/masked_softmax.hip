@@ -30,14 +30,15 @@
 //   otherwise (or a per-batch mask the grouping cannot share): the
 //     row_layout.h plan, W waves per row, 2 KiB per wave.
 // Rows that are not whole 16-byte groups, or not 16-byte aligned, take the
-// first and the last of these with element-aligned groups (row_layout.h,
+// first and the last of these (a few rows of at most 64 values a wave each,
+// value by value) with element-aligned groups (row_layout.h,
 // RaggedGroup) instead of a one-value-per-lane kernel that read each row
-// three times: graph replays, [1536, 197, 197] 209 -> 56 us (4.2 TB/s),
-// [96, 577, 577] 75 -> 34, [512, 50, 77] causal 11.2 -> 4.7, [8, 1500, 1501]
+// three times: graph replays, [1536, 197, 197] 207 -> 51.8 us (4.6 TB/s),
+// [96, 577, 577] 70 -> 34, [512, 50, 77] causal 10.8 -> 4.6, [8, 1500, 1501]
 // with a bias 55 -> 20.  What bounds them is the arithmetic of the lanes a
 // row leaves idle (25 groups on 32 lanes at K = 197) more than the
-// misalignment: K = 193 takes 53 us and K = 192, aligned, 50.5, while 256,
-// no lane idle, moves the same bytes in 43.
+// misalignment: K = 193 takes 51.0 us and K = 192, aligned, 47.9, while 256,
+// no lane idle, moves 1.3 times the bytes of 197 in 51.9.
 // HBM-bound: algorithmic bytes per element = 2 (read) + 2 (write), plus the
 // mask once.
 #include "row_layout.h"
@@ -509,7 +510,13 @@ int softmax_impl(const uint16_t* x, const uint16_t* mask, uint16_t* out, int64_t
   const bool vec = held && k % 8 == 0 && mask_row_stride % 8 == 0 &&
                    mask_batch_stride % 8 == 0 && aligned16(x) && aligned16(mask) &&
                    aligned16(out);
-  const int lanes = short_row_lanes(k);
+  // A few short rows off the vector path take the one-value-per-lane kernel: a
+  // wave each, K <= 64, ends sooner than lanes of 8 values in few waves.  Graph
+  // replays in us, short rows / value by value: 800 rows of 17 values 2.59 / 2.36,
+  // of 33 2.54 / 2.36, 2000 rows of 63 2.7 / 2.5; 3000 rows of 17 2.6 / 2.7, 1000
+  // of 65 2.60 / 2.86, 80 of 12 2.1 / 2.2.
+  const bool few_short = !vec && k <= 64 && rows <= 2048 && (k > 16 || rows > 256);
+  const int lanes = few_short ? 0 : short_row_lanes(k);
   if (held && lanes > 0 && rows < (int64_t{1} << 31)) {
     const int64_t rows_per_block = int64_t{kShortV} * (kWave / lanes) * (kShortThreads / kWave);
     const dim3 grid(static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block));
@@ -540,7 +547,7 @@ int softmax_impl(const uint16_t* x, const uint16_t* mask, uint16_t* out, int64_t
       launch_shared_mask<2048>(sp, stream, x, mask, out, batch, q, mask_row_stride,
                                mask_batch_stride, scale);
     }
-  } else if (held) {
+  } else if (held && !few_short) {
     const int64_t blocks = (rows + plan.rows_per_block - 1) / plan.rows_per_block;
     HIPO_REQUIRE(blocks <= 0x7fffffff, "%s: too many rows", what);
     const dim3 grid(static_cast<unsigned>(blocks));

@@ -86,6 +86,28 @@ def test_softmax_any_row_length(k, rocm_device):
         close(out.t, ref.scaled_bias_softmax(x, bias, 0.5, heads), 2 ** -7, 1e-6, f"bias K={k}")
 
 
+# Both sides of the lines where few short rows off the vector path go value by
+# value (2048 rows, and 256 of up to 16 values), and every lane count past them.
+@pytest.mark.parametrize("b,q,k,shift", [
+    (1, 256, 9, 0), (1, 257, 9, 0), (4, 512, 12, 0), (3, 683, 12, 0), (2, 1024, 17, 0),
+    (2049, 1, 17, 0), (683, 3, 33, 0), (683, 3, 50, 0), (4, 512, 64, 1), (683, 3, 64, 1),
+    (3, 700, 8, 1), (3, 700, 16, 1), (8, 16, 65, 0)])
+def test_softmax_few_short_rows(b, q, k, shift, rocm_device):
+    import oracle as ref
+    torch.manual_seed(b + q + k)
+    x = torch.randn(b, q, k).to(torch.bfloat16)
+    x[0, 0, k - 1] = float("inf")
+    mask = torch.randn(q, k).to(torch.bfloat16)
+    mask[q // 2, : k - 1] = float("-inf")
+    xd, md = place(x, rocm_device, shift), place(mask, rocm_device, shift)
+    out = Guarded((b, q, k), torch.bfloat16, rocm_device, shift)
+    ok(lib().hipo_scaled_masked_softmax_bf16(xd.data_ptr(), md.data_ptr(), out.t.data_ptr(), b, q,
+                                             k, k, 0.125, None))
+    torch.cuda.synchronize()
+    out.check(f"[{b}, {q}, {k}]")
+    close(out.t, ref.scaled_masked_softmax(x, mask, 0.125), 2 ** -7, 1e-6, f"[{b}, {q}, {k}]")
+
+
 @pytest.mark.parametrize("k", [9, 197, 577, 1025])
 def test_softmax_odd_rows_special_values(k, rocm_device):
     """A row that is -inf throughout is NaN; NaN and +inf scores make their
