@@ -127,7 +127,8 @@ __device__ __forceinline__ T not_negative(T v) {
 }
 
 // Chan's pairwise merge of (count, mean, M2) partials: (n, mean, m2) <-
-// (n, mean, m2) + (nb, meanb, m2b).
+// (n, mean, m2) + (nb, meanb, m2b).  The counts come between the two factors d: 0
+// for an empty partial even where the square of meanb overflows.
 template <typename T>
 __device__ __forceinline__ void chan_merge(T& n, T& mean, T& m2, T nb, T meanb, T m2b) {
   if (nb == T(0)) return;
@@ -135,7 +136,7 @@ __device__ __forceinline__ void chan_merge(T& n, T& mean, T& m2, T nb, T meanb, 
   const T d = meanb - mean;
   const T f = nb / nn;
   mean = mean + d * f;
-  m2 = m2 + m2b + d * d * n * f;
+  m2 = m2 + m2b + d * (n * f) * d;
   n = nn;
 }
 

@@ -12,7 +12,10 @@ struct Welford {
   float m2;
 };
 
-// Chan et al. pairwise merge of two triples over disjoint sets.
+// Chan et al. pairwise merge of two triples over disjoint sets.  The counts come
+// between the two factors d: an empty triple then adds 0 to M2 even where the
+// square of the other's mean overflows (d * d * 0 would make the variance of
+// finite values NaN).
 __device__ __forceinline__ Welford welford_merge(Welford a, Welford b) {
   const float n = a.n + b.n;
   if (n == 0.f) return a;
@@ -21,7 +24,7 @@ __device__ __forceinline__ Welford welford_merge(Welford a, Welford b) {
   Welford r;
   r.n = n;
   r.mean = __builtin_fmaf(d, wb, a.mean);
-  r.m2 = a.m2 + b.m2 + d * d * a.n * wb;
+  r.m2 = a.m2 + b.m2 + d * (a.n * wb) * d;
   return r;
 }
 

@@ -101,6 +101,52 @@ def test_batchnorm_nchw_mean(n, c, h, w, rocm_device):
                    yw.float().reshape(n, c).T, 2 ** -6, 1e-2, f"[{n}, {c}, {h}, {w}]")
 
 
+# Finite values whose squares overflow: the variance is infinite, rstd 0, and the
+# outputs are act(beta).  Every route as above but the kernels that sum about one
+# of the channel's values, and shapes whose huge value is the only one of a
+# thread's first merge.
+@pytest.mark.parametrize("n,c,hw", [(3, 5, 7), (26, 9, 49), (400, 9, 49), (4, 8, 196), (21, 5, 961),
+                                    (128, 40, 196), (3, 40, 8836), (1100, 5, 49), (2, 5, 9999),
+                                    (7, 5, 8649)])
+@pytest.mark.parametrize("where", [0, 1, 4097, -1])
+def test_batchnorm_train_overflowing_squares(n, c, hw, where, rocm_device):
+    import hip_oracles
+    torch.manual_seed(n + c)
+    x = torch.randn(n, c, 1, hw)
+    flat = x.transpose(0, 1).reshape(c, -1)
+    at = where % flat.shape[1]
+    x[at // hw, 1, 0, at % hw] = 3e38
+    x[at // hw, 2, 0, at % hw] = -3e38
+    gm, bt, rm, rv = params(c)
+    d = [t.to(rocm_device) for t in (x, gm, bt, rm, rv)]
+    y, mean, rstd = hip_oracles.batchnorm_train(*d, momentum=0.1, eps=1e-5, relu=False)
+    for ch, v in ((1, 3e38), (2, -3e38)):
+        assert float(mean[ch]) == pytest.approx(v / (n * hw), rel=1e-5)
+        assert float(rstd[ch]) == 0 and float(d[4][ch]) == INF
+        assert bool((y[:, ch] == d[2][ch]).all())
+    assert bool(torch.isfinite(y).all())
+
+
+@pytest.mark.parametrize("n,c,h,w", [(5, 6, 10, 20), (6, 7, 25, 21), (5, 7, 40, 41), (5, 36, 85, 85),
+                                     (300, 8, 7, 7), (300, 9, 7, 7)])
+@pytest.mark.parametrize("where", [0, 1, -1])
+def test_batchnorm_nchw_mean_overflowing_squares(n, c, h, w, where, rocm_device):
+    import hip_oracles
+    torch.manual_seed(n + c)
+    x = torch.randn(n, c, h, w).to(torch.bfloat16)
+    at = where % (n * h * w)
+    x[at // (h * w), 1].view(-1)[at % (h * w)] = 3e38
+    gm, bt, rm, rv = params(c)
+    d = [t.to(rocm_device) for t in (x, gm, bt, rm, rv)]
+    mean, rstd, out = hip_oracles.batchnorm_nchw_act_mean(*d, momentum=0.1, eps=1e-5, var_scale=1.0,
+                                                          act="relu")
+    big = float(torch.tensor(3e38).to(torch.bfloat16))
+    assert float(mean.view(-1)[1]) == pytest.approx(big / (n * h * w), rel=1e-5)
+    assert float(rstd.view(-1)[1]) == 0 and float(d[4][1]) == INF
+    want = torch.relu(bt[1]).to(torch.bfloat16).float()
+    assert torch.allclose(out[:, 1].float().cpu(), want.expand(n), rtol=2 ** -7, atol=1e-6)
+
+
 # Short rows aligned and not, a wave per row, several waves per row in one sweep
 # and in several, whole and ragged; fp32: the vector kernel, its ragged form,
 # single values.
