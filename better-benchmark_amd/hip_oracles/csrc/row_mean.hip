@@ -378,8 +378,8 @@ extern "C" int hipo_row_mean_bf16(const uint16_t* x, uint16_t* out, int64_t rows
   // one or two waves a row come to more workgroups than CUs.  The rows kernel's
   // time over the wave's, graph replays, 700 points of 520 to 12296 values and 1
   // to 60000 rows.  One wave: 520 values, 2048 rows 1.02, 2300 1.17, 60000 1.08;
-  // 776, 3600 rows 1.16, 16000 1.07, 32000 0.95; 1024, 2300 rows 1.14, 24000
-  // 0.99.  Two: 1032 values 1.02 to 1.37 from 1400 rows on; 1224, 1400 rows 1.02,
+  // 704, 24000 rows 1.04 (1.08 with ReLU), 32000 1.01 (1.07), 50000 0.95; 776,
+  // 3600 rows 1.16, 16000 1.07, 32000 0.95; 1024, 2300 rows 1.14, 24000 0.99.  Two: 1032 values 1.02 to 1.37 from 1400 rows on; 1224, 1400 rows 1.02,
   // 1600 1.13; 1448, 1500 rows 0.93, 2800 1.12; 1736, 3400 rows 1.00, 5000 1.12.
   // Three: 2056 values, 2600 rows 1.01, 3200 1.06; 2312, 2800 rows 0.97, 4000
   // 1.07.  More: 4104 values, 3400 rows 0.95, 5000 1.10; 8200, 4096 rows 1.17;
@@ -388,7 +388,8 @@ extern "C" int hipo_row_mean_bf16(const uint16_t* x, uint16_t* out, int64_t rows
                             : waves == 2 ? (fill < 54 ? 1 : fill < 76 ? 1537 : 4096)
                             : waves <= 4 ? (fill < 70 ? 2816 : 3584)
                                          : 4096;
-  const bool little = waves == 1 ? fill < 60 || rows <= 16384 : fill < (two ? 85 : 60);
+  const bool little = waves == 1 ? fill < 60 || rows <= (fill < 70 ? 32768 : 16384)
+                                 : fill < (two ? 85 : 60);
   const bool wave_rows = !ragged && little && rows >= wave_from;
   if (cols <= kBf16ShortCols && (aligned || (off_short && rows >= kBf16ShortRows))) {
     const int64_t blocks = blocks_of(kBf16Waves * kBf16RowsPerWave);

@@ -563,6 +563,7 @@ def test_row_mean_bf16_many_rows(rows, cols, shift, rocm_device):
     x = torch.randn(rows, cols).to(torch.bfloat16)
     xd = place(x, rocm_device, shift)
     for relu in (0, 1):
+    (32768, 704, 0), (32769, 704, 0),
         out = Guarded((rows,), torch.bfloat16, rocm_device)
         ok(lib().hipo_row_mean_bf16(xd.data_ptr(), out.t.data_ptr(), rows, cols, relu, None))
         torch.cuda.synchronize()
