@@ -179,6 +179,20 @@ __global__ __launch_bounds__(kTrThreads) void transpose_tiles(const T* __restric
   }
 }
 
+// Output rows that are not whole halves of a cache line: the tiles' runs end inside
+// one, and non-temporal stores send both parts to memory, so that the pieces had
+// better meet in the L2 (rows of whole quarters only beyond 32 MB read and
+// written).  Graph replays in us, non-temporal stores / cached: [218, 500, 128]
+// fp32 27.4 / 18.0, [1093, 100, 128] fp32 45 / 18.7, [43, 4968, 64] bf16 15.3 /
+// 10.9, [44, 4964, 64] fp32 28.1 / 18.2; 4000-byte rows of 31 MB 7.5 / 7.9, of 112
+// MB 24.4 / 18.9; 8000-byte rows (whole halves) of 31 and 61 MB 5.5 / 7.5, 11.6 /
+// 12.2.  The bias + GELU tiles cover their short rows whole and keep
+// non-temporal stores ([128, 232, 14, 14] 6.5 / 7.7).
+bool halves_meet_in_l2(int64_t mats, int64_t R, int64_t C, int64_t size) {
+  const int64_t out_row = R * size;
+  return out_row % 64 != 0 && (out_row % 32 != 0 || 2 * mats * C * out_row > kTileSmallBytes);
+}
+
 template <typename T>
 int launch_transpose(const void* xp, void* yp, int64_t batch, int64_t R, int64_t C,
                      hipStream_t stream) {
@@ -227,6 +241,8 @@ int launch_transpose(const void* xp, void* yp, int64_t batch, int64_t R, int64_t
       transpose_whole<T, kTrMaxVecPerThread><<<grid, block, lds_bytes, stream>>>(x, y, g);
     }
   } else if (block_tiles(x, y, batch, R, C, static_cast<int>(sizeof(T)), t, access)) {
+    if (access == TileAccess::kStreamOut && halves_meet_in_l2(batch, R, C, sizeof(T)))
+      access = TileAccess::kCached;
     auto kernel = access == TileAccess::kCached      ? transpose_blocks<T, TileAccess::kCached>
                   : access == TileAccess::kStreamOut ? transpose_blocks<T, TileAccess::kStreamOut>
                                                      : transpose_blocks<T, TileAccess::kStream>;

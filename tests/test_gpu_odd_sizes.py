@@ -217,7 +217,10 @@ def test_transpose_any_matrix(r, c, dtype, rocm_device):
 @pytest.mark.parametrize("batch,r,c,dtype", [
     (2, 512, 384, torch.bfloat16), (2, 256, 192, torch.float32), (40, 512, 512, torch.bfloat16),
     (161, 256, 1024, torch.bfloat16), (161, 128, 1024, torch.float32),
-    (81, 1024, 512, torch.bfloat16), (161, 520, 500, torch.bfloat16)])
+    (81, 1024, 512, torch.bfloat16), (161, 520, 500, torch.bfloat16),
+    # output rows of whole 16, 32 and 64 bytes, the second below and beyond 32 MB
+    (3, 500, 72, torch.float32), (62, 1000, 64, torch.float32), (63, 1000, 64, torch.float32),
+    (70, 2000, 66, torch.float32), (5, 4968, 64, torch.bfloat16)])
 def test_transpose_cache_policies(batch, r, c, dtype, rocm_device):
     g = torch.Generator(device=rocm_device).manual_seed(r + c)
     bits = torch.int16 if dtype == torch.bfloat16 else torch.int32
