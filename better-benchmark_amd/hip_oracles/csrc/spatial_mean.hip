@@ -295,9 +295,21 @@ SpatialPlan spatial_plan(int64_t n, int64_t p, int64_t c) {
   plan.group_block = static_cast<int>(G);
   const int64_t lcm = G / gcd64(G, kWave) * kWave;
   // Whole waves, about 512 threads, where the group count allows them, else
-  // as many rows as fit 512 threads (the last wave is partial).
+  // as many rows as fit 512 threads (the last wave is partial), but no more than
+  // give a thread kUnroll positions (two times that for wide rows, and one row
+  // up to 12 positions; 48 positions from 768 images on, three workgroups a CU):
+  // adding the rows' partials takes longer than a few loads more.  Graph replays in
+  // us, one row / as many as fit / here: [128, 168, 2, 2] 2.4 / 2.9 / 2.5, [800, 296,
+  // 3, 4] 3.4 / 5.5 / 3.2, [800, 296, 7, 7] 10.9 / 6.3 / 6.3, [800, 1000, 2, 2] 3.1 /
+  // 5.6 / 3.1, [128, 1240, 4, 4] 4.4 / 4.1 / 3.9, [800, 1240, 4, 4] 6.7 / 8.3 / 6.7,
+  // [800, 1000, 6, 6] 10.7 / 12.4 / 10.7.
+  constexpr int64_t kWide = 96;
+  const int64_t few = G <= kWide ? (p + kUnroll - 1) / kUnroll
+                      : n >= 768 ? (p + 12 * kUnroll - 1) / (12 * kUnroll)
+                      : p <= 12  ? 1
+                                 : (p + 2 * kUnroll - 1) / (2 * kUnroll);
   int64_t T = lcm <= kMaxThreads ? lcm * std::max<int64_t>(1, 512 / lcm)
-                                 : G * std::max<int64_t>(1, 512 / G);
+                                 : G * std::max<int64_t>(1, std::min(512 / G, few));
   const int64_t rows = T / G;
   if (rows > p) T = G * std::max<int64_t>(1, p);  // no more rows than positions
   plan.threads = static_cast<int>(std::min<int64_t>(T, kMaxThreads));

@@ -380,7 +380,14 @@ def test_norms_any_row_length(cols, rocm_device):
 SPATIAL = [(2, 7, 9), (2, 8, 9), (3, 9, 1), (3, 15, 49), (4, 29, 3190), (2, 61, 700), (130, 1001, 49),
            (6, 1759, 196), (1, 514, 50), (2, 8193, 4), (300, 33, 100),
            # ragged plan and thread per output, on both sides of the line
-           (2100, 500, 1), (3000, 9, 4), (1500, 250, 9), (600, 250, 9), (2, 8200, 7)]
+           (2100, 500, 1), (3000, 9, 4), (1500, 250, 9), (600, 250, 9), (2, 8200, 7),
+           # whole groups: as many rows as give a thread its loads, one row, two.
+           # Powers of two positions: the sum times 1 / P is exact and rounds
+           # once, as in the oracle; other counts round twice, and among as many
+           # outputs some lie an ulp off, 2^-7 of a value just above a power of 2
+           # ([3, 1000, 13]: 2^-9 at 0.27).
+           (3, 168, 4), (3, 168, 8), (5, 232, 64), (3, 1000, 8), (3, 1000, 16), (767, 1240, 16),
+           (768, 1240, 16), (769, 1000, 64)]
 
 
 @pytest.mark.parametrize("n,c,hw", SPATIAL)
@@ -556,6 +563,7 @@ def test_row_mean_any_row_length(cols, rocm_device):
     (2559, 520, 0), (2560, 520, 0), (2563, 1032, 0), (4095, 2056, 0), (4097, 2056, 0),
     (4099, 4104, 0), (4097, 8200, 0), (2561, 1024, 0),
     (2048, 520, 0), (2049, 1000, 0), (16384, 1000, 0), (16385, 1000, 0), (16385, 520, 0),
+    (32768, 704, 0), (32769, 704, 0),
     (3, 1096, 0), (3, 1112, 0), (1536, 1448, 0), (1537, 1448, 0), (4095, 1736, 0), (4096, 1736, 0),
     (2815, 2056, 0), (2816, 2056, 0), (3583, 3080, 0), (3584, 3080, 0), (4099, 3592, 0),
     (2048, 3001, 0), (2049, 3001, 0), (2047, 4095, 3), (2053, 4095, 0), (999, 1500, 1)])
@@ -566,7 +574,6 @@ def test_row_mean_bf16_many_rows(rows, cols, shift, rocm_device):
     x = torch.randn(rows, cols).to(torch.bfloat16)
     xd = place(x, rocm_device, shift)
     for relu in (0, 1):
-    (32768, 704, 0), (32769, 704, 0),
         out = Guarded((rows,), torch.bfloat16, rocm_device)
         ok(lib().hipo_row_mean_bf16(xd.data_ptr(), out.t.data_ptr(), rows, cols, relu, None))
         torch.cuda.synchronize()
