@@ -93,16 +93,23 @@ __global__ __launch_bounds__(256) void bias_gelu_nchw_to_nhwc_scalar(
 
 // Whether the tiles beat a thread per element.  A wave maps 64 values a lane
 // one after the other, however few of its lanes own a block and however much
-// the last blocks overlap: estimates in us of both, from graph replays over 8
-// to 1000 channels, planes of 8 to 196 positions and 0.56 to 9 million elements
-// (of those 600 points the worst comes out 18 % slower than the better of the
-// two).  Measured, tiles / thread per element: [60000, 9, 3, 3] 91 / 18, [64,
-// 1000, 3, 3] 8.2 / 4.2, [3000, 64, 2, 5] 10.6 / 8.8, [2187, 16, 4, 4] 10.6 / 4.2,
-// [9375, 64, 3, 5] 25 / 30, [128, 512, 7, 7] 8.7 / 16.3.  Images of whole blocks
-// keep the tiles from kTileMinElems on unless their waves alone cost more.
-bool tiles_pay(const BlockTiles& t, int64_t elements, bool whole) {
-  const double tiles_us = (whole ? 0.0 : 3.6) + 1.7e-3 * t.waves;
-  return tiles_us < 3.05e-6 * static_cast<double>(elements);
+// the last blocks overlap; a thread per element reads a cache line for each of
+// its wave's channels, which longer planes of many channels do not find in the
+// L1 again for their next positions.  Estimates in us of both, fitted to graph
+// replays over 9 to 1500 channels, planes of 9 to 1369 positions and 0.55 to 8
+// million elements: of 1499 points 18 come out over 5 % slower than the better of
+// the two, the worst 18 %.  Measured, tiles / thread per element: [60000, 9, 3, 3]
+// 91 / 18, [64, 1000, 3, 3] 8.2 / 4.2, [3000, 64, 2, 5] 10.6 / 8.8, [2187, 16, 4, 4]
+// 10.6 / 4.2, [9375, 64, 3, 5] 25 / 30, [834, 40, 6, 6] 5.0 / 5.8, [128, 512, 7, 7]
+// 8.7 / 16.3, [19, 640, 12, 9] 5.1 / 9.4, [2, 982, 19, 21] 4.6 / 5.6.  Images of whole
+// blocks keep the tiles from kTileMinElems on unless their waves alone cost more.
+bool tiles_pay(const BlockTiles& t, int64_t elements, int64_t c, int64_t hw, bool whole) {
+  const auto ramp = [](int64_t v, double from, double to) {
+    return std::min(1.0, std::max(0.0, (static_cast<double>(v) - from) / (to - from)));
+  };
+  const double element_us = 3.05e-6 * (1.0 + 0.6 * ramp(hw, 20, 60) * ramp(c, 60, 260));
+  const double tiles_us = whole ? 1.7e-3 * t.waves : 2.8 + 1.3e-3 * t.waves;
+  return tiles_us < element_us * static_cast<double>(elements);
 }
 
 }  // namespace
@@ -128,7 +135,7 @@ extern "C" int hipo_bias_gelu_nchw_to_nhwc_bf16(const uint16_t* x,
   TileAccess access;
   const bool whole = c % 8 == 0 && hw % 8 == 0 && aligned16(x) && aligned16(out);
   if (n * c * hw > kTileMinElems && block_tiles(x, out, n, c, hw, 2, t, access) &&
-      tiles_pay(t, n * c * hw, whole)) {
+      tiles_pay(t, n * c * hw, c, hw, whole)) {
     auto kernel = access == TileAccess::kCached
                       ? bias_gelu_nchw_to_nhwc_blocks<TileAccess::kCached>
                   : access == TileAccess::kStreamOut
