@@ -27,9 +27,11 @@ namespace hipo {
 namespace {
 
 constexpr int kUnroll = 4;
-// Row partials are added one by one up to here, by a tree beyond: by a tree from 17
-// on, [30, 208, 8, 8] took 5.0 us and one by one 4.6, [128, 232, 14, 14] 7.4 and 6.7.
-constexpr int kSerialRows = 32;
+// Up to how many row partials G groups of threads add one by one, by a tree beyond.
+// 32 rows, us, tree / one by one: [30, 208, 8, 8], 26 groups, 5.0 / 4.6, [5, 96, 62,
+// 12], 12 groups, 6.4 / 6.6, [77, 149, 16, 18], 5 groups, 5.3 / 5.8; 17 rows, [128,
+// 232, 14, 14], 7.4 / 6.7.
+__device__ __forceinline__ int serial_rows(int G) { return G >= 16 ? 32 : 16; }
 constexpr int kMaxThreads = 1024;
 
 // RAGGED (ragged_plan): any C >= 8, any alignment.  The last group of a row
@@ -87,7 +89,7 @@ __global__ __launch_bounds__(kMaxThreads) void spatial_mean_nhwc_partial(
       }
     }
   }
-  if (R > kSerialRows) {
+  if (R > serial_rows(G)) {
     // Rows r and r + half, half halving: a fixed order for any R.
     int top = 1;
     while (top < R) top *= 2;
