@@ -1067,12 +1067,16 @@ __global__ __launch_bounds__(kFinalThreads) void bn_finalize(
 // slice and slice count.  A workgroup has R rows of G = ceil(C / 8) groups
 // per instruction, R a power of two, up to 512 threads in the statistics pass
 // and 256 in the epilogue (the last wave may be partial).  Slices are of a
-// multiple of 512 rows, at most about 512 of them; where that gives under 128,
-// they are halved, down to 64 rows: a launch of a dozen workgroups, one per 512
-// rows, took twice as long.  Under 96 / 128 / 192 / 288, us: C 48, 20300 rows 12.3
-// / 12.4 / 13.7 / -, C 40, 42200 rows 13.4 / 13.4 / 14.1 / -, C 64, 68992 rows - /
-// 16.4 / 17.7 / 21.3, C 512, 94080 rows - / 54.6 / 56.5 / 56.6, C 1024, 28000 and
-// 55000 rows 36.8 / 35.5 / 35.8 and 61.8 / 59.0 / 59.1.  The slicing depends on
+// multiple of 512 rows, at most about 512 of them; where that gives under 128
+// (192 for wide rows whose workgroups are less than two thirds full, and for the
+// scalar kernels), they are halved, down to 64 rows: a launch of a dozen
+// workgroups, one per 512 rows, took twice as long.  Under 96 / 128 / 192 / 288, us:
+// C 48 (384 threads), 20300 rows 12.3 / 12.4 / 13.7 / -, C 40, 42200 rows 13.4 /
+// 13.4 / 14.1 / -, C 64, 68992 rows - / 16.4 / 17.7 / 21.3, C 512, 94080 rows - /
+// 54.6 / 56.5 / 56.6, C 1024, 28000 and 55000 rows 36.8 / 35.5 / 35.8 and 61.8 / 59.0 /
+// 59.1; C 546 (276 threads), 32928 rows - / 29.3 / 26.8 / -, C 5, 37536 rows - / 29.2 /
+// 18.5 / -; over 253 points 128 takes 0.91 to 1.03 times 192's time where it is
+// taken and 0.97 to 1.13 where it is not.  The slicing depends on
 // the shape alone, and so does the workspace size; its traffic, 8 B per channel
 // and slice written and read, is 6 % of x each way for 64-row slices (fewer than
 // 16384 rows) and under 1 % for 512.
@@ -1091,7 +1095,9 @@ constexpr int kNhwcApplyThreads = 256;
 constexpr int64_t kNhwcSliceStep = 512;
 constexpr int64_t kNhwcMinSlice = 64;
 constexpr int64_t kNhwcMaxSlices = 512;
-constexpr int64_t kNhwcFewSlices = 128;
+constexpr int64_t kNhwcFewSlices = 192;
+constexpr int64_t kNhwcFewSlicesFull = 128;
+constexpr int64_t kNhwcFullThreads = 336;
 
 // Fewer rows of C not a multiple of 8 (or off alignment) go one thread per
 // channel: a workgroup's tree over its row partials takes longer than so few
@@ -1110,16 +1116,18 @@ NhwcPlan nhwc_plan(int64_t M, int64_t C, bool vec_ok) {
   NhwcPlan plan;
   if (M <= 0 || C <= 0) return plan;
   const int64_t G = (C + 7) / 8;
-  if (vec_ok && C >= 8 && G <= kMaxThreads) {
+  int64_t few = kNhwcFewSlices;
+  if (C >= 8 && G <= kMaxThreads) {
     int64_t R = 1;
     while (G * R * 2 <= kNhwcApplyThreads) R *= 2;
-    plan.threads = static_cast<int>(G * R);
+    if (vec_ok) plan.threads = static_cast<int>(G * R);
     while (G * R * 2 <= kNhwcStatThreads) R *= 2;
-    plan.stat_threads = static_cast<int>(G * R);
+    if (vec_ok) plan.stat_threads = static_cast<int>(G * R);
+    if (G < 16 || G * R >= kNhwcFullThreads) few = kNhwcFewSlicesFull;
   }
   const int64_t want = (M + kNhwcMaxSlices - 1) / kNhwcMaxSlices;
   int64_t len = (want + kNhwcSliceStep - 1) / kNhwcSliceStep * kNhwcSliceStep;
-  while (len > kNhwcMinSlice && M / len < kNhwcFewSlices) len /= 2;
+  while (len > kNhwcMinSlice && M / len < few) len /= 2;
   plan.slice_len = len;
   plan.slices = (M + len - 1) / len;
   return plan;
