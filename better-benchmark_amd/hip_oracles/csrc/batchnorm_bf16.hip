@@ -1039,14 +1039,18 @@ __global__ __launch_bounds__(kFinalThreads) void bn_finalize(
   __syncthreads();
   // Lanes past the slices hold zeros: the tree starts at the others ([2, 179, 2,
   // 1], one slice, 8.9 -> 6.7 us a call).
-  int half = kFinalLanes / 2;
-  while (half > 0 && half >= slices) half /= 2;
-  for (; half > 0; half /= 2) {
+  auto add_half = [&](int half) {
     if (j < half) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) red[q][t] += red[q][t + half * kFinalCols];
     }
     __syncthreads();
+  };
+  if (slices > kFinalLanes / 2) {
+    for (int half = kFinalLanes / 2; half > 0; half /= 2) add_half(half);
+  } else {
+    for (int half = kFinalLanes / 4; half > 0; half /= 2)
+      if (half < slices) add_half(half);
   }
   if (!owner) return;
   n = red[0][t];
