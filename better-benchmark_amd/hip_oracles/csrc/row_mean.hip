@@ -379,11 +379,12 @@ extern "C" int hipo_row_mean_bf16(const uint16_t* x, uint16_t* out, int64_t rows
   // time over the wave's, graph replays, 700 points of 520 to 12296 values and 1
   // to 60000 rows.  One wave: 520 values, 2048 rows 1.02, 2300 1.17, 60000 1.08;
   // 704, 24000 rows 1.04 (1.08 with ReLU), 32000 1.01 (1.07), 50000 0.95; 776,
-  // 3600 rows 1.16, 16000 1.07, 32000 0.95; 1024, 2300 rows 1.14, 24000 0.99.  Two: 1032 values 1.02 to 1.37 from 1400 rows on; 1224, 1400 rows 1.02,
-  // 1600 1.13; 1448, 1500 rows 0.93, 2800 1.12; 1736, 3400 rows 1.00, 5000 1.12.
-  // Three: 2056 values, 2600 rows 1.01, 3200 1.06; 2312, 2800 rows 0.97, 4000
-  // 1.07.  More: 4104 values, 3400 rows 0.95, 5000 1.10; 8200, 4096 rows 1.17;
-  // 10248, 5000 rows 1.07, 12296, 4096 rows 0.93.
+  // 3600 rows 1.16, 16000 1.07, 32000 0.95; 1024, 2300 rows 1.14, 24000 0.99.
+  // Two: 1032 values 1.02 to 1.37 from 1400 rows on; 1224, 1400 rows 1.02, 1600
+  // 1.13; 1448, 1500 rows 0.93, 2800 1.12; 1736, 3400 rows 1.00, 5000 1.12. Three:
+  // 2056 values, 2600 rows 1.01, 3200 1.06; 2312, 2800 rows 0.97, 4000 1.07.
+  // More: 4104 values, 3400 rows 0.95, 5000 1.10; 8200, 4096 rows 1.17; 10248,
+  // 5000 rows 1.07, 12296, 4096 rows 0.93.
   const int64_t wave_from = waves == 1   ? 2049
                             : waves == 2 ? (fill < 54 ? 1 : fill < 76 ? 1537 : 4096)
                             : waves <= 4 ? (fill < 70 ? 2816 : 3584)
